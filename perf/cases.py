@@ -3,7 +3,7 @@ of rows, widths, shapes and activation types (``QLinear.init`` and ``layer(x)``)
 tensor (``convert_params``), and a Llama-shaped model around them (decode step and prefill).
 
 A case is a dict of plain values; ``prepare`` makes what a program holds before the call, ``run`` is one pass through
-the public entry points, ``work`` what the pass cannot do without, ``tolerance`` how far another correct
+the public entry points, ``work`` what the pass cannot do without, ``exact`` the results in 64 bits, ``tolerance`` how far another correct
 implementation's results may be off.
 """
 import os
@@ -208,3 +208,85 @@ def tolerance(case):
     # eight layers of fp16 roundings between the linears: 8.5e-4 and 6e-3 measured against the same model with
     # PyTorch operations there
     return {"rel": 4e-3, "max": 3e-2}
+
+
+def _exact_linear(x, q, zero, scale, gs):
+    """``x @ ((q - zero) * scale)`` in 64 bits: q (K, N), zero and scale (K / gs, N)."""
+    w = q.to(torch.float64)
+    if scale is not None:
+        w = ((w.reshape(-1, gs, q.shape[1]) - zero.to(torch.float64)[:, None]) * scale.to(torch.float64)[:, None]).reshape(q.shape)
+    return x @ w
+
+
+def _packed_fields(t):
+    """The sixteen values of a byte pair's four-bit fields, in the order of the elements: (rows, bytes) -> (rows, 2 * bytes).
+    In a word the even elements fill the low half, the odd ones the high half."""
+    b = t.view(torch.uint8).reshape(t.shape[0], -1, 4)
+    nibbles = torch.stack((b & 15, b >> 4), dim=-1).reshape(t.shape[0], -1, 2, 4)
+    return nibbles.transpose(2, 3).reshape(t.shape[0], -1)
+
+
+def _exact_model(case, seed):
+    """Logits and caches of the model cases in 64 bits: the same random packed tensors, plain matrix products, no fp16 between the steps."""
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    batch, hd, f64 = case["batch"], HIDDEN // HEADS, torch.float64
+    weights = torch.Generator(device="cuda").manual_seed(seed)
+    embed = (torch.randn(VOCAB, HIDDEN, device="cuda", generator=weights) * 0.5).to(torch.float16)
+
+    def linear(K, N):
+        w = torch.randint(-128, 128, (N, K // 2), dtype=torch.int8, device="cuda", generator=weights)
+        z = torch.randint(-128, 128, (N, K // 256), dtype=torch.int8, device="cuda", generator=weights).view(torch.uint8)
+        s = ((torch.rand(N, K // 128, device="cuda", generator=weights) + 0.5) * (0.5 / (16 * 0.41 * K ** 0.5))).to(torch.float16)
+        zero = torch.stack((z & 15, z >> 4), dim=-1).reshape(N, K // 128)
+        return lambda x: _exact_linear(x, _packed_fields(w).T, zero.T, s.T, 128)
+
+    layers = [[linear(HIDDEN, 3 * HIDDEN), linear(HIDDEN, HIDDEN), linear(HIDDEN, 2 * MLP), linear(MLP, HIDDEN)] for _ in range(MODEL_LAYERS)]
+    head = linear(HIDDEN, VOCAB)
+    k_cache = torch.zeros(MODEL_LAYERS, batch, HEADS, MAX_LEN, hd, dtype=f64, device="cuda")
+    v_cache = torch.zeros_like(k_cache)
+    if case["kind"] == "prefill":
+        tokens = torch.randint(0, VOCAB, (batch, case["tokens"]), device="cuda", generator=gen)
+        pos = torch.arange(case["tokens"], device="cuda")
+    else:
+        for cache in (k_cache, v_cache):
+            for layer in cache:
+                layer[:, :, :case["pos"]] = torch.randn(batch, HEADS, case["pos"], hd, device="cuda", generator=gen).to(torch.float16)
+        tokens = torch.randint(0, VOCAB, (batch, 1), device="cuda", generator=gen)
+        pos = torch.full((1,), case["pos"], dtype=torch.int64, device="cuda")
+    T = tokens.shape[1]
+    angle = pos.to(f64)[:, None] / 10000.0 ** (torch.arange(0, hd, 2, device="cuda", dtype=f64) / hd)[None]
+    cos, sin = angle.cos(), angle.sin()
+    hidden = (torch.arange(MAX_LEN, device="cuda")[None] > pos[:, None])[None, None]
+
+    def norm(x):
+        return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + 1e-5)
+
+    def rope(x):
+        a, b = x[..., 0::2], x[..., 1::2]
+        return torch.stack((a * cos - b * sin, a * sin + b * cos), dim=-1).flatten(-2)
+
+    x = embed[tokens].to(f64).reshape(batch * T, HIDDEN)
+    for li, (qkv, o, gate_up, down) in enumerate(layers):
+        q, k, v = qkv(norm(x)).reshape(batch, T, 3, HEADS, hd).permute(2, 0, 3, 1, 4)
+        k_cache[li][:, :, pos], v_cache[li][:, :, pos] = rope(k), v
+        scores = (rope(q) @ k_cache[li].transpose(-1, -2).contiguous()) * hd ** -0.5
+        att = scores.masked_fill(hidden, float("-inf")).softmax(-1) @ v_cache[li]
+        x = x + o(att.transpose(1, 2).reshape(batch * T, HIDDEN))
+        gate, up = gate_up(norm(x)).split(MLP, dim=1)
+        x = x + down(gate / (1 + torch.exp(-gate)) * up)
+    return {"logits": head(norm(x.reshape(batch, T, HIDDEN)[:, -1])), "k": k_cache, "v": v_cache}
+
+
+def exact(case, seed):
+    """What ``run`` returns for these inputs, in 64 bits and without this repository's kernels."""
+    if case["kind"] in ("decode", "prefill"):
+        return _exact_model(case, seed)
+    if case["kind"] == "convert":
+        return None                                              # packed bytes: compared bit for bit
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    weight, scale, zero = _gptq_tensors(case, gen)
+    x = torch.randn(case["M"], case["K"], device="cuda", generator=gen).to(torch.bfloat16 if case["dtype"] == "bf16" else torch.float16)
+    top = 2 ** case["nbits"] - 1
+    if scale is not None:                                        # GPTQ stores the zero-point less one; the packed form clamps the sum
+        zero = torch.full_like(scale, (top + 1) // 2) if zero is None else (zero + 1).clamp(max=top)
+    return _exact_linear(x.to(torch.float64), weight, zero, scale, case["gs"])
