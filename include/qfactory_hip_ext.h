@@ -1,0 +1,26 @@
+/*
+ * Entry points of libqfactory_hip.so that the package's own host code calls beside those of qfactory_hip.h; the same
+ * conventions (device pointers, a hipStream_t, calls only enqueue; 0 success, 1 invalid arguments, 2 launch failed).
+ */
+#ifndef QFACTORY_HIP_EXT_H
+#define QFACTORY_HIP_EXT_H
+
+#include <stddef.h>
+#include <stdint.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/*
+ * qf_pack_weight and qf_pack_zero with the range check of the fields in the same pass: *bad (device memory, may be
+ * null) is set to a nonzero value if any value lies outside [0, 2^nbits) and left alone otherwise; the caller clears
+ * it first.
+ */
+int qf_pack_weight_checked(const int32_t* weight, int8_t* out, int64_t K, int64_t N, int nbits, uint32_t* bad, void* stream);
+int qf_pack_zero_checked(const int32_t* zero, int8_t* out, int64_t G, int64_t N, int nbits, uint32_t* bad, void* stream);
+
+#ifdef __cplusplus
+}
+#endif
+#endif

@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include "qfactory_hip.h"
+#include "qfactory_hip_ext.h"
 
 namespace {
 
@@ -25,69 +26,130 @@ int launched(const char* fn) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Weight repack.  One thread builds one 32-bit output word of one output row.  Threads of a
-// block are arranged 32 (rows n) x 8 (words): the reads of weight[k][n] are contiguous over n
-// (128 B per k), the 4-byte writes of a row are contiguous over the 8 words.
+// Weight repack, bound by memory: four bytes are read per field.  A block takes 64 columns n and 32 main-plane words
+// of K (16 threads x 4 columns side by side, 16 units of K): a thread reads 16 bytes of every k of its unit -- 256
+// contiguous bytes per k and 16 threads, all of a unit's loads in flight -- builds four columns' words in registers,
+// and the words change their orientation through LDS, so that a row of the output is written 128 bytes at a time
+// (a 4-byte word per thread straight to its row left 32-byte pieces: 22016 x 4096 at 4 bits 102 us = 4.0 TB/s; this
+// form 76 us = 5.4 TB/s).  Both planes of the 3-bit layout come out of one read of the fields.
 // Position j of a word holds element (j < P/2 ? 2j : 2(j - P/2) + 1) of its P = 32/b elements
 // (identity for 8-bit): evens in the low half-word, odds in the high half-word.  The 1-bit plane
 // of the 3-bit layout has its own order (hi_plane_pos): every high bit sits where one shift of
 // the word drops it directly above the element's field in the 2-bit plane.
+// Fields outside [0, 2^b) are counted by the same read: any bit above the field (a negative number has them all) is
+// collected per thread, and a wave that saw one sets `bad`.
 // ---------------------------------------------------------------------------------------------
 __host__ __device__ constexpr int hi_plane_pos(int e) {
     const int r = e / 16, ep = e % 16, i = ep / 2, h = ep % 2, p = i % 4, upper = i / 4;
     return ((p % 2 == 0) ? 2 * p + 2 : 2 * p - 2) + 8 * upper + r + 16 * h;
 }
+// bit position of element e inside its word of a plane of B-bit fields
+template <int B>
+__host__ __device__ constexpr int field_bit(int e) {
+    return B == 8 ? 8 * e : B == 1 ? hi_plane_pos(e) : B * (e / 2 + (e % 2) * (16 / B));
+}
 
-template <int B>   // field width of the plane being written: 1, 2, 4 or 8
-__device__ __forceinline__ uint32_t build_word(const int32_t* __restrict__ weight, int64_t N, int64_t n,
-                                               int64_t k0, int shift, uint32_t mask) {
-    constexpr int P = 32 / B;
-    uint32_t word = 0;
+template <int NBITS>
+struct PackCfg {
+    static constexpr int B = NBITS == 3 ? 2 : NBITS;           // field width of the main plane
+    static constexpr int P = 32 / B;                           // elements per main-plane word
+    static constexpr int UNIT = NBITS == 3 ? 32 : (P < 8 ? 8 : P);      // elements of K per thread and pass
+    static constexpr int UW = UNIT / P;                        // main-plane words per unit
+    static constexpr int WORDS = 32;                           // main-plane words of a block
+    static constexpr int PASSES = WORDS / UW / 16;
+    static constexpr int KB = WORDS * P;                       // elements of K of a block
+    static constexpr int HI = NBITS == 3 ? WORDS / 2 : 0;      // 1-bit-plane words of a block
+    static constexpr int PITCH = WORDS + HI + 1;               // odd: the transposed accesses spread over the banks
+};
+
+// VEC: N a multiple of four and 16-byte aligned rows, four columns per load; otherwise single words
+template <int NBITS, bool VEC>
+__global__ __launch_bounds__(256) void pack_weight_kernel(const int32_t* __restrict__ weight, uint32_t* __restrict__ out,
+                                                          int64_t K, int64_t N, uint32_t* __restrict__ bad) {
+    using C = PackCfg<NBITS>;
+    __shared__ uint32_t tile[64][C::PITCH];
+    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
+    const int64_t n0 = (int64_t)blockIdx.x * 64, n = n0 + 4 * tx;
+    const int64_t k_blk = (int64_t)blockIdx.y * C::KB;
+    constexpr uint32_t MASK = (1u << NBITS) - 1u;
+    uint32_t seen = 0;
 #pragma unroll
-    for (int j = 0; j < P; j++) {
-        // hi_plane_pos is its own inverse: bit j holds element hi_plane_pos(j)
-        const int src = (B == 8) ? j : (B == 1) ? hi_plane_pos(j) : (j < P / 2 ? 2 * j : 2 * (j - P / 2) + 1);
-        const uint32_t v = ((uint32_t)weight[(k0 + src) * N + n] >> shift) & mask;
-        word |= v << (j * B);
+    for (int pass = 0; pass < C::PASSES; pass++) {
+        const int unit = pass * 16 + ty;
+        const int64_t k0 = k_blk + (int64_t)unit * C::UNIT;
+        uint32_t word[4][C::UW] = {}, high[4] = {};
+        if (k0 < K && n < N) {                                  // K is a multiple of 32, hence of the unit
+            u32x4 v[C::UNIT];
+#pragma unroll
+            for (int e = 0; e < C::UNIT; e++) {
+                const uint32_t* src = reinterpret_cast<const uint32_t*>(weight) + (k0 + e) * N + n;
+                if constexpr (VEC) {
+                    v[e] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src));
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; c++) v[e][c] = n + c < N ? src[c] : 0u;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < C::UNIT; e++)
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    seen |= v[e][c];
+                    word[c][e / C::P] |= (v[e][c] & MASK & ((1u << C::B) - 1u)) << field_bit<C::B>(e % C::P);
+                    if constexpr (NBITS == 3) high[c] |= ((v[e][c] >> 2) & 1u) << field_bit<1>(e);
+                }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+#pragma unroll
+            for (int w = 0; w < C::UW; w++) tile[4 * tx + c][unit * C::UW + w] = word[c][w];
+            if constexpr (NBITS == 3) tile[4 * tx + c][C::WORDS + unit] = high[c];
+        }
     }
-    return word;
+    if (bad != nullptr && __any((seen & ~MASK) != 0) && (threadIdx.x & 63) == 0) atomicOr(bad, 1u);
+    __syncthreads();
+    const int64_t row_words = K * NBITS / 32;
+    const int64_t w0 = (int64_t)blockIdx.y * C::WORDS;
+    for (int i = threadIdx.x; i < 64 * C::WORDS; i += 256) {
+        const int r = i / C::WORDS, w = i % C::WORDS;
+        if (n0 + r < N && w0 + w < K / C::P) out[(n0 + r) * row_words + w0 + w] = tile[r][w];
+    }
+    if constexpr (NBITS == 3) {                                 // the 1-bit plane behind the row's 2-bit plane
+        const int64_t h0 = (int64_t)blockIdx.y * C::HI;
+        for (int i = threadIdx.x; i < 64 * C::HI; i += 256) {
+            const int r = i / C::HI, w = i % C::HI;
+            if (n0 + r < N && h0 + w < K / 32) out[(n0 + r) * row_words + K / 16 + h0 + w] = tile[r][C::WORDS + w];
+        }
+    }
 }
 
-template <int B>
-__global__ __launch_bounds__(256) void pack_plane_kernel(const int32_t* __restrict__ weight, uint32_t* __restrict__ out,
-                                                         int64_t K, int64_t N, int64_t row_words, int64_t word_offset,
-                                                         int shift, uint32_t mask) {
-    constexpr int P = 32 / B;
-    const int64_t n = (int64_t)blockIdx.x * 32 + (threadIdx.x & 31);
-    const int64_t wi = (int64_t)blockIdx.y * 8 + (threadIdx.x >> 5);
-    if (n >= N || wi >= K / P) return;
-    out[n * row_words + word_offset + wi] = build_word<B>(weight, N, n, wi * P, shift, mask);
-}
-
-template <int B>
-void launch_plane(const int32_t* weight, int8_t* out, int64_t K, int64_t N, int64_t row_words, int64_t word_offset,
-                  int shift, uint32_t mask, hipStream_t stream) {
-    constexpr int P = 32 / B;
-    dim3 grid((unsigned)((N + 31) / 32), (unsigned)((K / P + 7) / 8));
-    hipLaunchKernelGGL(pack_plane_kernel<B>, grid, dim3(256), 0, stream, weight, (uint32_t*)out, K, N, row_words,
-                       word_offset, shift, mask);
+template <int NBITS>
+void launch_pack(const int32_t* weight, int8_t* out, int64_t K, int64_t N, uint32_t* bad, hipStream_t stream) {
+    const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((K + PackCfg<NBITS>::KB - 1) / PackCfg<NBITS>::KB));
+    const bool vec = N % 4 == 0 && (uintptr_t)weight % 16 == 0;
+    hipLaunchKernelGGL((vec ? pack_weight_kernel<NBITS, true> : pack_weight_kernel<NBITS, false>), grid, dim3(256), 0, stream,
+                       weight, (uint32_t*)out, K, N, bad);
 }
 
 __global__ __launch_bounds__(256) void pack_zero_kernel(const int32_t* __restrict__ zero, uint8_t* __restrict__ out,
-                                                        int64_t G, int64_t N, int nbits, int fb) {
+                                                        int64_t G, int64_t N, int nbits, int fb,
+                                                        uint32_t* __restrict__ bad) {
     const int p8 = 8 / fb;
     const int64_t row_bytes = G / p8;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;      // over N * row_bytes, n fastest
     if (idx >= N * row_bytes) return;
     const int64_t n = idx % N, byte = idx / N;
     const int32_t maxv = (1 << nbits) - 1;
-    uint32_t v = 0;
+    uint32_t v = 0, seen = 0;
     for (int i = 0; i < p8; i++) {
-        int32_t z = zero[(byte * p8 + i) * N + n] + 1;
+        int32_t z = zero[(byte * p8 + i) * N + n];
+        seen |= (uint32_t)z;
+        z = z == 0x7fffffff ? z : z + 1;
         z = z > maxv ? maxv : z;
         v |= (uint32_t)z << (i * fb);
     }
     out[n * row_bytes + byte] = (uint8_t)v;
+    if (bad != nullptr && (seen & ~(uint32_t)maxv) != 0) atomicOr(bad, 1u);
 }
 
 __global__ __launch_bounds__(256) void transpose_u16_kernel(const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
@@ -179,26 +241,27 @@ extern "C" int qf_bf16_to_f16(const uint16_t* src, uint16_t* dst, int64_t n, voi
     return launched("qf_bf16_to_f16");
 }
 
-extern "C" int qf_pack_weight(const int32_t* weight, int8_t* out, int64_t K, int64_t N, int nbits, void* stream_) {
+extern "C" int qf_pack_weight_checked(const int32_t* weight, int8_t* out, int64_t K, int64_t N, int nbits, uint32_t* bad,
+                                      void* stream_) {
     hipStream_t stream = (hipStream_t)stream_;
     if (!weight || !out) return fail("qf_pack_weight", "null pointer");
     if (K <= 0 || N <= 0 || K % 32 != 0) return fail("qf_pack_weight", "K must be a positive multiple of 32, N positive");
-    const uint32_t mask = (1u << nbits) - 1u;
-    const int64_t row_words = K * nbits / 32;
     switch (nbits) {
-        case 8: launch_plane<8>(weight, out, K, N, row_words, 0, 0, mask, stream); break;
-        case 4: launch_plane<4>(weight, out, K, N, row_words, 0, 0, mask, stream); break;
-        case 2: launch_plane<2>(weight, out, K, N, row_words, 0, 0, mask, stream); break;
-        case 3:   // low two bits in the 2-bit layout, then the high bit as a 1-bit plane
-            launch_plane<2>(weight, out, K, N, row_words, 0, 0, 3u, stream);
-            launch_plane<1>(weight, out, K, N, row_words, K / 16, 2, 1u, stream);
-            break;
+        case 8: launch_pack<8>(weight, out, K, N, bad, stream); break;
+        case 4: launch_pack<4>(weight, out, K, N, bad, stream); break;
+        case 3: launch_pack<3>(weight, out, K, N, bad, stream); break;
+        case 2: launch_pack<2>(weight, out, K, N, bad, stream); break;
         default: return fail("qf_pack_weight", "nbits must be 2, 3, 4 or 8");
     }
     return launched("qf_pack_weight");
 }
 
-extern "C" int qf_pack_zero(const int32_t* zero, int8_t* out, int64_t G, int64_t N, int nbits, void* stream_) {
+extern "C" int qf_pack_weight(const int32_t* weight, int8_t* out, int64_t K, int64_t N, int nbits, void* stream_) {
+    return qf_pack_weight_checked(weight, out, K, N, nbits, nullptr, stream_);
+}
+
+extern "C" int qf_pack_zero_checked(const int32_t* zero, int8_t* out, int64_t G, int64_t N, int nbits, uint32_t* bad,
+                                    void* stream_) {
     hipStream_t stream = (hipStream_t)stream_;
     if (!zero || !out) return fail("qf_pack_zero", "null pointer");
     if (nbits != 2 && nbits != 3 && nbits != 4 && nbits != 8) return fail("qf_pack_zero", "nbits must be 2, 3, 4 or 8");
@@ -206,8 +269,12 @@ extern "C" int qf_pack_zero(const int32_t* zero, int8_t* out, int64_t G, int64_t
     if (G <= 0 || N <= 0 || G % (8 / fb) != 0) return fail("qf_pack_zero", "G must fill whole bytes of zero-points");
     const int64_t total = N * (G / (8 / fb));
     hipLaunchKernelGGL(pack_zero_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, zero, (uint8_t*)out, G,
-                       N, nbits, fb);
+                       N, nbits, fb, bad);
     return launched("qf_pack_zero");
+}
+
+extern "C" int qf_pack_zero(const int32_t* zero, int8_t* out, int64_t G, int64_t N, int nbits, void* stream_) {
+    return qf_pack_zero_checked(zero, out, G, N, nbits, nullptr, stream_);
 }
 
 extern "C" int qf_transpose_scale(const uint16_t* scale, uint16_t* out, int64_t G, int64_t N, void* stream_) {

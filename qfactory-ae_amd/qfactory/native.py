@@ -41,6 +41,12 @@ SIGNATURES = {
     "qf_greedy_next": (_INT, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _P]),
 }
 
+# the same for include/qfactory_hip_ext.h
+EXT_SIGNATURES = {
+    "qf_pack_weight_checked": (_INT, [_P, _P, _I64, _I64, _INT, _P, _P]),
+    "qf_pack_zero_checked": (_INT, [_P, _P, _I64, _I64, _INT, _P, _P]),
+}
+
 _lock = threading.Lock()
 _lib = None
 
@@ -68,7 +74,7 @@ def load():
                 raise RuntimeError(f"{LIBRARY} is missing: build it with qfactory.native.build() "
                                    "(hipcc, no GPU needed); there is no CPU substitute for the device packers")
             lib = ctypes.CDLL(LIBRARY)
-            for name, (res, args) in SIGNATURES.items():
+            for name, (res, args) in {**SIGNATURES, **EXT_SIGNATURES}.items():
                 fn = getattr(lib, name)
                 fn.restype, fn.argtypes = res, args
             _lib = lib
@@ -85,24 +91,27 @@ def _check(rc, what):
         raise RuntimeError(f"{what} failed with return code {rc}")
 
 
-def pack_weight(weight, nbits):
-    """(K, N) int32 device tensor -> (N, K*nbits/8) int8, bit-identical to convert._transform_weight_basic."""
+def pack_weight(weight, nbits, bad=None):
+    """(K, N) int32 device tensor -> (N, K*nbits/8) int8, bit-identical to convert._transform_weight_basic.  ``bad``: a
+    one-element int32 device tensor, set nonzero if a field lies outside [0, 2^nbits)."""
     import torch
     assert weight.is_cuda and weight.dtype == torch.int32 and weight.is_contiguous() and weight.dim() == 2
     K, N = weight.shape
     out = torch.empty(N, K * nbits // 8, dtype=torch.int8, device=weight.device)
-    _check(load().qf_pack_weight(weight.data_ptr(), out.data_ptr(), K, N, nbits, _stream()), "qf_pack_weight")
+    _check(load().qf_pack_weight_checked(weight.data_ptr(), out.data_ptr(), K, N, nbits, bad.data_ptr() if bad is not None else None,
+                                         _stream()), "qf_pack_weight")
     return out
 
 
-def pack_zero(zero, nbits):
-    """(G, N) int32 device tensor -> (N, G*fb/8) int8 holding min(zero + 1, 2^nbits - 1)."""
+def pack_zero(zero, nbits, bad=None):
+    """(G, N) int32 device tensor -> (N, G*fb/8) int8 holding min(zero + 1, 2^nbits - 1); ``bad`` as for ``pack_weight``."""
     import torch
     assert zero.is_cuda and zero.dtype == torch.int32 and zero.is_contiguous() and zero.dim() == 2
     G, N = zero.shape
     fb = 4 if nbits == 3 else nbits
     out = torch.empty(N, G * fb // 8, dtype=torch.int8, device=zero.device)
-    _check(load().qf_pack_zero(zero.data_ptr(), out.data_ptr(), G, N, nbits, _stream()), "qf_pack_zero")
+    _check(load().qf_pack_zero_checked(zero.data_ptr(), out.data_ptr(), G, N, nbits, bad.data_ptr() if bad is not None else None,
+                                       _stream()), "qf_pack_zero")
     return out
 
 

@@ -77,3 +77,42 @@ def test_bad_arguments_are_rejected_without_launching():
     assert lib.qf_pack_zero(buf.data_ptr(), buf.data_ptr(), 3, 1, 4, None) == 1         # G % 2
     assert lib.qf_stream_copy(buf.data_ptr(), buf.data_ptr(), 24, None) == 1            # bytes % 16
     assert lib.qf_pack_weight(None, buf.data_ptr(), 32, 1, 4, None) == 1
+
+
+@pytest.mark.parametrize("nbits", [2, 3, 4, 8])
+@pytest.mark.parametrize("K,N,offset", [(32, 64, 0), (1056, 68, 0), (544, 67, 0), (512, 132, 1), (4128, 1, 0)])
+def test_weight_packer_at_tile_edges(oracle, nbits, K, N, offset):
+    """Partial tiles of 64 columns and 32 words, single-word loads (odd N, a tensor that starts off a 16-byte boundary)."""
+    from qfactory import native
+    g = torch.Generator().manual_seed(K + N + nbits)
+    weight = torch.randint(0, 2 ** nbits, (K, N), dtype=torch.int32, generator=g)
+    store = torch.empty(K * N + offset, dtype=torch.int32, device="cuda")
+    dev = store[offset:].view(K, N)
+    dev.copy_(weight)
+    bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+    w = native.pack_weight(dev, nbits, bad)
+    assert bad.item() == 0
+    assert np.array_equal(w.cpu().numpy(), oracle.pack_weight(weight.numpy(), nbits))
+
+
+@pytest.mark.parametrize("nbits", [2, 3, 4, 8])
+@pytest.mark.parametrize("value", ["top", "negative", "lowest", "highest"])
+def test_values_out_of_range_are_refused(nbits, value):
+    """A single bad field or zero-point anywhere -- first, last, in a partial tile -- is refused as on the host."""
+    from qfactory import convert
+    K, N, GS = 544 * 4, 67, 544
+    v = {"top": 2 ** nbits, "negative": -1, "lowest": -2 ** 31, "highest": 2 ** 31 - 1}[value]
+    weight, scale, zero = (t.cuda() for t in _tensors(nbits, K, N, nbits, GS))
+    args = {"K": K, "N": N, "NBITS": nbits, "GS": GS}
+    convert.convert_params(args, (weight, scale, zero))
+    for k, n in ((0, 0), (K - 1, N - 1), (700, 64)):
+        bad = weight.clone()
+        bad[k, n] = v
+        with pytest.raises(AssertionError):
+            convert.convert_params(args, (bad, scale, zero))
+        with pytest.raises(AssertionError):
+            convert.convert_params({"K": K, "N": N, "NBITS": nbits}, (bad,))
+    bad = zero.clone()
+    bad[-1, -1] = v
+    with pytest.raises(AssertionError):
+        convert.convert_params(args, (weight, scale, bad))
