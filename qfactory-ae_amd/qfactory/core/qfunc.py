@@ -161,7 +161,8 @@ class QMatmulQFunc(QFunc):
         if regime == "skinny":
             return tiling.skinny_tiling(p["M"], p["N"], p["K"], nbits, gs)
         if regime == "gemm":
-            return tiling.gemm_tiling(p["M"], p["N"], p["K"], nbits, gs)
+            return (tiling.gemm_wide_tiling(p["M"], p["N"], p["K"], nbits, gs)
+                    or tiling.gemm_tiling(p["M"], p["N"], p["K"], nbits, gs))
         return tiling.mfma_tiling(p["M"], p["N"], p["K"], nbits, gs)
 
     def arg_name_type(self):
@@ -207,6 +208,9 @@ class QMatmulQFunc(QFunc):
             cands = tiling.skinny_candidates(p["M"], p["N"], p["K"], p["NBITS"], p["GS"])
         elif self.regime == "gemm":
             cands = tiling.gemm_candidates(p["M"], p["N"], p["K"], p["NBITS"], p["GS"])
+            default = self.default_tiling("gemm")
+            if default not in cands:
+                cands = [default] + cands
         else:
             cands = tiling.mfma_candidates(p["M"], p["N"], p["K"], p["NBITS"], p["GS"])
         return [self.clone(tiling_configs=c) for c in cands]
@@ -230,7 +234,8 @@ class QMatmulQFunc(QFunc):
             # the matrix-core kernels expose their dequantisation's vector-instruction issue and have
             # registers to spare: the one-instruction mask-and-merge decode pays there (2 - 7 %
             # measured); it does not in the 4-bit GEMV kernel, where it costs a resident wave
-            defines.setdefault("QF_FUSED_AND_OR", 1)
+            # (the pipelined GEMM kernel places every vector instruction itself: it needs the form the scheduler can see)
+            defines.setdefault("QF_FUSED_AND_OR", 2 if "WM" in t else 1)
         if self.regime == "gemv" and p["NBITS"] in (2, 3) and t["VB"] == 8 and t["MT"] == 1 \
                 and self.decode_strategy == "deferred" and not self.smem_quant \
                 and tiling.gemv_chunks_per_lane(p["K"], p["NBITS"], t) == 1:
@@ -272,7 +277,7 @@ class QMatmulQFunc(QFunc):
             # rows (two slabs) 125 -> 80 MB and 65.2 -> 62.8 us -- and loses where there are many, because the blocks of
             # an XCD then share no activation slab: 12288 x 4096 at 8192 rows 806 -> 3260 MB, 753 -> 791 us.
             slabs = -(-p["M"] // t["BM"])
-            if 2 <= slabs <= 8 and -(-p["N"] // (32 * t["NT32"] * t["WN"])) >= 8:
+            if 2 <= slabs <= 8 and -(-p["N"] // (32 * (t["NT"] if "WM" in t else t["NT32"]) * t["WN"])) >= 8:
                 defines.setdefault("QF_GEMM_XCD_MAP", 1)
         assert t.get("KS", 1) == 1 or (self.input_prologue == "none" and self.output_epilogue != "silu_mul"), \
             "a block that sees part of K can neither normalise a row nor pair gate with up: build the object with ksplit=False"
@@ -309,6 +314,10 @@ class QMatmulQFunc(QFunc):
             code += '#include "qf_skinny.hip.h"\n'
             cfg = tiling.skinny_cfg_string(p, t, not self.l2cache_b)
             call = "qf::skinny_launch<Cfg>"
+        elif self.regime == "gemm" and "WM" in t:
+            code += '#include "qf_gemm.hip.h"\n#include "qf_gemm_wide.hip.h"\n'
+            cfg = tiling.gemm_wide_cfg_string(p, t)
+            call = "qf::gemm_wide_launch<Cfg>"
         elif self.regime == "gemm":
             code += '#include "qf_gemm.hip.h"\n'
             cfg = tiling.gemm_cfg_string(p, t, not self.l2cache_b)

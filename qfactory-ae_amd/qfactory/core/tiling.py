@@ -827,6 +827,83 @@ def gemm_candidates(M, N, K, nbits, group_size):
     return out
 
 
+# Tilings of the pipelined kernel (qf::GemmWideCfg, include/qf_gemm_wide.hip.h): (WM, WN, MT, NT, KI, WK) -> us per round
+# of blocks and 64 elements of K.  The figures are medians of a sweep of eighteen tilings over 22016 x 4096, 12288 x 4096,
+# 4096 x 4096, 4096 x 11008, 10240 x 8192, 8192 x 28672 and 57344 x 8192 at 33 ... 2048 rows (W4 g128, cold weights): with the
+# round model of gemm_wide_tiling they pick the fastest of the sweep on all but three of its cells (2 - 7 % off there).
+GEMM_WIDE_COST = {
+    (1, 4, 8, 2, 1, 1): 1.547,     # 256 x 256
+    (2, 2, 4, 3, 1, 1): 1.289,     # 256 x 192
+    (1, 4, 6, 2, 1, 1): 1.212,     # 192 x 256
+    (1, 4, 4, 2, 1, 1): 0.952,     # 128 x 256
+    (1, 4, 4, 1, 2, 1): 0.572,     # 128 x 128
+    (1, 3, 4, 1, 2, 1): 0.505,     # 128 x 96
+    (1, 4, 3, 1, 2, 1): 0.462,     # 96 x 128
+    (1, 4, 2, 1, 2, 2): 0.341,     # 64 x 128
+    (1, 3, 2, 1, 2, 2): 0.307,     # 64 x 96
+    (1, 2, 2, 1, 2, 2): 0.217,     # 64 x 64
+    (1, 2, 1, 1, 2, 4): 0.148,     # 32 x 64
+    (1, 1, 1, 1, 2, 4): 0.100,     # 32 x 32
+}
+GEMM_WIDE_MIN_M = 33
+
+
+def gemm_wide_lds_bytes(cfg, nbits):
+    """The larger of the groups' tiles and windows and of what the end of the kernel needs (GemmWideCfg::LDS_BYTES)."""
+    wm, wn, mt, nt, ki, wk = (cfg[k] for k in ("WM", "WN", "MT", "NT", "KI", "WK"))
+    bm, bn = 32 * mt * wm, 32 * nt * wn
+    windows = 2 if 1024 // nbits // 64 // ki > 1 else 3
+    tiles = wk * (3 * ki * bm * 128 + windows * bn * 128)
+    return max(tiles, (wk - 1) * bm * bn * 4 + wm * wn * 32 * mt * (64 * nt + 16))
+
+
+def gemm_wide_valid(cfg, K, nbits, group_size):
+    """Mirror of the static checks in gemm_wide_launch (qf_gemm_wide.hip.h)."""
+    if nbits not in (2, 4, 8):
+        return False
+    supk = 1024 // nbits
+    if K % supk or (supk // 64) % cfg["KI"] or cfg["WK"] > K // supk:
+        return False
+    if -(-(K // supk) // cfg["WK"]) * (supk // 64 // cfg["KI"]) < 3:
+        return False                   # fewer than three iterations: nothing to pipeline, and too few waits for the ISA check to re-count
+    if group_size <= 0 or K % group_size or group_size % 32:
+        return False
+    if (supk % group_size) if group_size < supk else (group_size % supk):
+        return False
+    ngs = max(1, supk // group_size)
+    return ngs <= 8 and ngs * nbits <= 32 and gemm_wide_lds_bytes(cfg, nbits) <= 160 * 1024
+
+
+def gemm_wide_tiling(M, N, K, nbits, group_size):
+    """Tiling of the pipelined kernel for this problem, None where the kernel of gemm_tiling serves: up to 32 rows, 3 bits,
+    and K that is not whole 128-byte windows.  A launch costs its exact number of rounds of blocks plus 40 % of the rounding
+    up (rounds overlap), a single partial round 0.6 + 0.4 x the share of the CUs that get a block; a block row taller than
+    twice the rows is not considered."""
+    if M < GEMM_WIDE_MIN_M:
+        return None
+    best = None
+    for (wm, wn, mt, nt, ki, wk), per_step in GEMM_WIDE_COST.items():
+        bm, bn = 32 * mt * wm, 32 * nt * wn
+        if bm >= 2 * M:
+            continue
+        cfg = {"BM": bm, "WM": wm, "WN": wn, "MT": mt, "NT": nt, "KI": ki, "WK": wk, "PA": 3}
+        if ki > 1 and not gemm_wide_valid(cfg, K, nbits, group_size):
+            cfg["KI"] = 1              # 8 bits, where three windows do not fit beside the tiles, and the shortest rows
+        if not gemm_wide_valid(cfg, K, nbits, group_size):
+            continue
+        exact = (-(-N // bn) * -(-M // bm)) / NUM_CUS
+        rounds = exact + 0.4 * (-(-exact // 1) - exact) if exact > 1 else 0.6 + 0.4 * exact
+        if best is None or rounds * per_step < best[0]:
+            best = (rounds * per_step, cfg)
+    return None if best is None else best[1]
+
+
+def gemm_wide_cfg_string(problem, t):
+    b = lambda x: "true" if x else "false"
+    return (f"qf::GemmWideCfg<{problem['NBITS']}, {problem['GS']}, {b(problem['SYM'])}, {problem['N']}, {problem['K']}, "
+            f"{t['WM']}, {t['WN']}, {t['MT']}, {t['NT']}, {t['KI']}, {t['WK']}>")
+
+
 def gemm_cfg_string(problem, t, nt_b):
     b = lambda x: "true" if x else "false"
     return (f"qf::GemmCfg<{problem['NBITS']}, {problem['GS']}, {b(problem['SYM'])}, {problem['N']}, {problem['K']}, "

@@ -156,6 +156,8 @@ class GPTQLinear(torch.nn.Module):
         if regime == "mgemv":
             return self.out_features % 32 == 0
         if regime == "gemm":
+            if tiling.gemm_wide_tiling(bucket, self.out_features, self.in_features, self.n_bits, self.group_size) is not None:
+                return self.out_features % 8 == 0           # whole groups of four pairs
             t = tiling.gemm_tiling(bucket, self.out_features, self.in_features, self.n_bits, self.group_size)
             return self.out_features % (32 * t["NT32"]) == 0
         if regime != "gemv":

@@ -1,0 +1,55 @@
+"""The pipelined GEMM kernel (include/qf_gemm_wide.hip.h) at the edges of its tilings against the CPU oracle."""
+import pytest
+import torch
+
+import prebuild
+from helpers import assert_close, make_problem, reference_output
+
+pytestmark = pytest.mark.gpu
+
+NO_SEARCH = {"enable_transform": False, "enable_schedule": False, "enable_lower": False}
+
+
+def _id(c):
+    t = dict(c["tiling"])
+    return (f"M{c['M']}-N{c['N']}-K{c['K']}-b{c['NBITS']}-g{c['GS']}-{'sym' if c['sym'] else 'asym'}-"
+            + "x".join(str(t[k]) for k in ("WM", "WN", "MT", "NT", "KI", "WK")))
+
+
+def _launch(runtime, x, layer, out):
+    z = layer.z if layer.z is not None else torch.empty(1, dtype=torch.int8, device="cuda")
+    rc = runtime.run_raw(x.shape[0], (x.data_ptr(), layer.w.data_ptr(), out.data_ptr(), layer.s.data_ptr(), z.data_ptr()),
+                         torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0
+
+
+@pytest.mark.parametrize("case", prebuild.wide_cases(), ids=_id)
+def test_tilings_at_their_edges(oracle, case):
+    from qfactory import QLinear
+    from qfactory.jit import jit
+    M, N, K, nbits, GS, sym = (case[k] for k in ("M", "N", "K", "NBITS", "GS", "sym"))
+    print(f"[case] {_id(case)}", flush=True)
+    A, weight, scale, zero = make_problem(77 + N + K + M, M, N, K, nbits, GS, sym)
+    layer = QLinear.init(1, K, N, nbits, weight.cuda(), GS, scale.cuda(), None if zero is None else zero.cuda(),
+                         compile_flags=NO_SEARCH)
+    (qfunc,) = prebuild.qfuncs_of(case)
+    assert qfunc.regime == "gemm" and qfunc.tiling_configs == dict(case["tiling"])
+    runtime = jit.compile(qfunc)
+    assert runtime.description.endswith("waits=counted")
+    x = A.cuda()
+    # a row of its own behind the output: nothing may be written there
+    store = torch.full((M + 1, N), float("nan"), dtype=torch.float16, device="cuda")
+    _launch(runtime, x, layer, store[:M])
+    assert store[M].isnan().all()
+    first = store[:M].clone()
+    assert_close(oracle, first.cpu().numpy(), reference_output(oracle, A, layer.w, layer.s, layer.z, nbits, GS), _id(case))
+    _launch(runtime, x, layer, store[:M])
+    assert torch.equal(first, store[:M])
+    # an activation that starts off a 16-byte boundary, a single row, rows of one tile only
+    shifted = torch.empty(M * K + 8, dtype=torch.float16, device="cuda")[1:1 + M * K].view(M, K)
+    shifted.copy_(x)
+    for rows in (M, min(M, 32), 1):
+        store.fill_(float("nan"))
+        _launch(runtime, shifted[:rows], layer, store[:rows])
+        assert torch.equal(first[:rows], store[:rows]) and store[rows:].isnan().all()
