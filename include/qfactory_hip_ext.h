@@ -20,6 +20,14 @@ extern "C" {
 int qf_pack_weight_checked(const int32_t* weight, int8_t* out, int64_t K, int64_t N, int nbits, uint32_t* bad, void* stream);
 int qf_pack_zero_checked(const int32_t* zero, int8_t* out, int64_t G, int64_t N, int nbits, uint32_t* bad, void* stream);
 
+/*
+ * Causal attention of `tokens` positions of every sequence over its cache: q and out (batch, tokens, heads, head_dim)
+ * fp16, caches (batch, heads, max_len, head_dim) fp16, pos (tokens) int64 device values; token t sees cache rows
+ * 0 .. pos[t].  head_dim 64 or 128; q, caches and out 16-byte aligned.  Scores and sums in fp32.
+ */
+int qf_prefill_attention(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, const int64_t* pos, uint16_t* out,
+                         int64_t batch, int64_t tokens, int64_t heads, int64_t head_dim, int64_t max_len, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -140,8 +140,8 @@ class QuantLlama:
     def prefill(self, tokens, pos):
         """``forward`` with the RMSNorm as a single launch of libqfactory_hip.so (any number of rows), the residual
         adds in the o and down projections' epilogues and SiLU * up in the gate+up projection's (or launches of their
-        own where a kernel cannot), RoPE and the cache update of all positions as one launch; causal attention stays
-        a PyTorch op."""
+        own where a kernel cannot), RoPE and the cache update of all positions as one launch, causal attention over
+        the cache as another (head sizes 64 and 128; a PyTorch op otherwise)."""
         from qfactory import native
         shape = self.shape
         B, T = tokens.shape
@@ -150,9 +150,10 @@ class QuantLlama:
         hdn = torch.empty_like(x)
         own = self.linear is self._own_linear
         act = None if own else torch.empty(B * T, shape.mlp, dtype=torch.float16, device="cuda")
-        mask = (torch.arange(shape.max_len, device="cuda")[None, :] <= pos[:, None])[None, None]
         delta = None
         q_rows = torch.empty(B, T, H, hd, dtype=torch.float16, device="cuda") if own else None
+        att_rows = torch.empty_like(q_rows) if own and hd in (64, 128) else None
+        mask = None if att_rows is not None else (torch.arange(shape.max_len, device="cuda")[None, :] <= pos[:, None])[None, None]
         pos = pos.contiguous()
         for li, layer in enumerate(self.layers):
             native.add_rmsnorm(x, delta, layer["norm1"], hdn, shape.eps)
@@ -160,14 +161,17 @@ class QuantLlama:
             if own:
                 # RoPE of q and k and the cache write of k and v for all T positions: one launch
                 native.rope_kv_store_rows(qkv, pos, self.cos, self.sin, q_rows, self.k_cache[li], self.v_cache[li])
-                q = q_rows.transpose(1, 2)                      # (B, H, T, hd) view: the attention output comes back in row order
+                q = q_rows.transpose(1, 2)                      # (B, H, T, hd) view
             else:
                 qkv = qkv.reshape(B, T, 3, H, hd).permute(2, 0, 3, 1, 4)
                 q, k, v = self._rope(qkv[0], pos), self._rope(qkv[1], pos), qkv[2]
                 self.k_cache[li].index_copy_(2, pos, k)
                 self.v_cache[li].index_copy_(2, pos, v)
-            att = F.scaled_dot_product_attention(q, self.k_cache[li], self.v_cache[li], attn_mask=mask)
-            att = att.permute(0, 2, 1, 3).reshape(B * T, shape.hidden)
+            if att_rows is not None:
+                att = native.prefill_attention(q_rows, self.k_cache[li], self.v_cache[li], pos, att_rows).reshape(B * T, shape.hidden)
+            else:
+                att = F.scaled_dot_product_attention(q, self.k_cache[li], self.v_cache[li], attn_mask=mask)
+                att = att.permute(0, 2, 1, 3).reshape(B * T, shape.hidden)
             if own:
                 # the o and down projections add their result to the residual stream themselves (the norms then only
                 # read it), SiLU(gate) * up is the gate+up projection's epilogue where it can be

@@ -15,7 +15,8 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC_DIR = os.path.join(PKG_DIR, "csrc") if os.path.isdir(os.path.join(PKG_DIR, "csrc")) else os.path.join(os.path.dirname(PKG_DIR), "csrc")
 REPO_INCLUDE = (os.path.join(PKG_DIR, "abi") if os.path.isdir(os.path.join(PKG_DIR, "abi"))
                 else os.path.join(os.path.dirname(os.path.dirname(PKG_DIR)), "include"))
-SOURCES = [os.path.join(CSRC_DIR, "qfactory_hip.hip"), os.path.join(CSRC_DIR, "qfactory_decode.hip")]
+SOURCES = [os.path.join(CSRC_DIR, "qfactory_hip.hip"), os.path.join(CSRC_DIR, "qfactory_decode.hip"),
+           os.path.join(CSRC_DIR, "qfactory_prefill.hip")]
 LIBRARY = os.path.join(CSRC_DIR, "libqfactory_hip.so")
 
 HIPCC_FLAGS = ["--offload-arch=gfx950", "-std=c++20", "-shared", "-fPIC", "-O3",
@@ -45,6 +46,7 @@ SIGNATURES = {
 EXT_SIGNATURES = {
     "qf_pack_weight_checked": (_INT, [_P, _P, _I64, _I64, _INT, _P, _P]),
     "qf_pack_zero_checked": (_INT, [_P, _P, _I64, _I64, _INT, _P, _P]),
+    "qf_prefill_attention": (_INT, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P]),
 }
 
 _lock = threading.Lock()
@@ -199,6 +201,19 @@ def rope_kv_store_rows(qkv, pos, cos, sin, q_out, k_cache, v_cache):
     _check(load().qf_rope_kv_store_rows(_f16(qkv), pos.data_ptr(), cos.data_ptr(), sin.data_ptr(), _f16(q_out), _f16(k_cache),
                                         _f16(v_cache), B, T, H, hd, max_len, _stream()), "qf_rope_kv_store_rows")
     return q_out
+
+
+def prefill_attention(q, k_cache, v_cache, pos, out):
+    """q and out (B, T, H, hd), caches (B, H, max_len, hd), pos T int64 device values: causal attention, token t over the
+    cache rows 0 .. pos[t].  hd 64 or 128."""
+    import torch
+    B, H, max_len, hd = k_cache.shape
+    T = pos.numel()
+    assert q.shape == (B, T, H, hd) and out.shape == q.shape and v_cache.shape == k_cache.shape
+    assert pos.is_cuda and pos.dtype == torch.int64 and pos.is_contiguous()
+    _check(load().qf_prefill_attention(_f16(q), _f16(k_cache), _f16(v_cache), pos.data_ptr(), _f16(out), B, T, H, hd, max_len,
+                                       _stream()), "qf_prefill_attention")
+    return out
 
 
 def decode_attention(q, k_cache, v_cache, pos, out):
