@@ -335,11 +335,11 @@ def wide_cases():
         (300, 500, 1024, 4, 128, False, (1, 4, 8, 2, 1, 1)), (257, 388, 768, 4, 128, False, (2, 2, 4, 3, 1, 1)),
         (193, 264, 1024, 2, 64, True, (1, 4, 6, 2, 1, 1)), (129, 260, 1280, 8, 32, False, (1, 4, 4, 2, 1, 1)),
         (130, 130, 1024, 4, 32, False, (1, 4, 4, 1, 2, 1)), (100, 136, 896, 8, 64, True, (1, 4, 4, 1, 2, 1)),
-        (128, 97, 512, 4, 64, False, (1, 3, 4, 1, 2, 1)), (97, 128, 1536, 4, 256, True, (1, 4, 3, 1, 2, 1)),
+        (128, 97, 768, 4, 64, False, (1, 3, 4, 1, 2, 1)), (97, 128, 1536, 4, 256, True, (1, 4, 3, 1, 2, 1)),
         (65, 140, 1280, 4, 128, False, (1, 4, 2, 1, 2, 2)), (64, 104, 2816, 4, 64, False, (1, 3, 2, 1, 2, 2)),
         (50, 64, 2048, 2, 128, False, (1, 2, 2, 1, 2, 2)), (70, 132, 640, 8, 64, False, (1, 4, 2, 1, 1, 2)),
         (33, 72, 2816, 4, 128, False, (1, 2, 1, 1, 2, 4)), (40, 33, 3328, 4, 128, False, (1, 1, 1, 1, 2, 4)),
-        (34, 68, 896, 8, 64, True, (1, 2, 1, 1, 1, 4))]]
+        (34, 68, 1152, 8, 64, True, (1, 2, 1, 1, 1, 4))]]
 
 
 def search_cases():

@@ -864,8 +864,8 @@ def gemm_wide_valid(cfg, K, nbits, group_size):
     supk = 1024 // nbits
     if K % supk or (supk // 64) % cfg["KI"] or cfg["WK"] > K // supk:
         return False
-    if -(-(K // supk) // cfg["WK"]) * (supk // 64 // cfg["KI"]) < 3:
-        return False                   # fewer than three iterations: nothing to pipeline, and too few waits for the ISA check to re-count
+    if -(-(K // supk) // cfg["WK"]) * (supk // 64 // cfg["KI"]) < 5:
+        return False                   # fewer than five iterations: nothing to pipeline, and too few waits for the ISA check to re-count
     if group_size <= 0 or K % group_size or group_size % 32:
         return False
     if (supk % group_size) if group_size < supk else (group_size % supk):
@@ -887,9 +887,12 @@ def gemm_wide_tiling(M, N, K, nbits, group_size):
         if bm >= 2 * M:
             continue
         cfg = {"BM": bm, "WM": wm, "WN": wn, "MT": mt, "NT": nt, "KI": ki, "WK": wk, "PA": 3}
-        if ki > 1 and not gemm_wide_valid(cfg, K, nbits, group_size):
-            cfg["KI"] = 1              # 8 bits, where three windows do not fit beside the tiles, and the shortest rows
-        if not gemm_wide_valid(cfg, K, nbits, group_size):
+        # 8 bits (three windows do not fit beside the tiles) and short rows: one step per iteration, fewer groups
+        for ki, wk in ((ki, wk), (1, wk), (1, -(-wk // 2)), (1, 1)):
+            cfg.update(KI=ki, WK=wk)
+            if gemm_wide_valid(cfg, K, nbits, group_size):
+                break
+        else:
             continue
         exact = (-(-N // bn) * -(-M // bm)) / NUM_CUS
         rounds = exact + 0.4 * (-(-exact // 1) - exact) if exact > 1 else 0.6 + 0.4 * exact

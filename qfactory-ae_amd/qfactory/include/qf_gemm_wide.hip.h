@@ -177,6 +177,14 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
             if (part < 0 || p % C::PARTS == part) buffer_to_lds_16(w_rows, w_off[p], (uint32_t)sup * 128u, dst + min(p * WAVES + wave, C::WB - 1) * 1024);
     };
 
+    // the first windows and tiles go out before anything else is computed
+#pragma unroll
+    for (int w = 0; w < C::WS - 1; w++)
+        if (w < C::NWIN) request_w(w, window_of(w), -1);
+    request_a(0, 0, 0, 1);
+    if (C::ITERS > 1) request_a(1, 1, 0, 1);
+    __builtin_amdgcn_sched_barrier(0);
+
     // ---- scales and zero-points of the wave's rows, one window in registers and the next on its way ----
     struct Quant { uint32_t s[NT][C::SREGS]; uint32_t z[NT]; };
     uint32_t s_off[NT], z_off[NT];                             // byte offsets from the block's first row
@@ -326,48 +334,47 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
     constexpr int AHEAD = C::AHEAD, SEGS = C::SEGS, KI = C::KI, WS = C::WS, STEPS = C::STEPS;
     constexpr int LAST_BEFORE = SEGS - AHEAD - 1;              // the barrier follows this segment: the next ones read the next tile
     Quant quant[WS];
-    // iteration `it` of the group; s = it % PASS a constant, live 0: nothing to multiply (a group with one window less), b0, b1, b2 the buffers of tiles it, it + 1 and it + 2
-    auto iteration = [&](int it, auto s_tag, auto live_tag, int b0, int b1, int b2) __attribute__((always_inline)) {
-        constexpr int s = decltype(s_tag)::value;
+    // iteration `it` of the group; s = it % PASS a constant, live 0: nothing to multiply (a group with one window less), left:
+    // iterations behind this one, where that is known to be few (tiles and windows past the end are not requested, and the
+    // last iteration reads nothing ahead and meets nobody); b0, b1, b2 the buffers of tiles it, it + 1 and it + 2
+    auto iteration = [&](int it, auto s_tag, auto live_tag, auto left_tag, int b0, int b1, int b2) __attribute__((always_inline)) {
+        constexpr int s = decltype(s_tag)::value, left = decltype(left_tag)::value;
         constexpr int q = s % SUP, win = s / SUP;              // iteration of the window; window counted inside a pass
+        constexpr bool next_tile = left >= 1, request_tile = left >= 2, request_window = (left + q) / SUP >= WS - 1;
+        constexpr int requests = (request_tile ? C::UA : 0) + (request_window ? wide_window_requests<C>(q) : 0);
         const int sup = it / SUP;
         static_for<0, SEGS>([&](auto g_tag) __attribute__((always_inline)) {
             constexpr int g = decltype(g_tag)::value, step = s * KI + g / 4;
             // fragments of segment g + AHEAD
             if constexpr (g + AHEAD < SEGS) read_frags(af[(g + AHEAD) % C::SETS], b0, g + AHEAD);
-            else read_frags(af[(g + AHEAD) % C::SETS], b1, g + AHEAD - SEGS);
+            else if constexpr (next_tile) read_frags(af[(g + AHEAD) % C::SETS], b1, g + AHEAD - SEGS);
             // packed words of the next 64-element step, in front of the first segment that dequantises them
             constexpr int next = step + 1, next_win = next / STEPS % WS;
-            constexpr bool packed_here = g % 4 == 4 - AHEAD;
+            constexpr bool packed_here = g % 4 == 4 - AHEAD && (next_tile || g + 4 < SEGS);
             if constexpr (packed_here) read_packed(pk[next % 2], next_win, next % STEPS);
             // weight fragments of segment g + 1
-            if constexpr (g % 4 == 3) {
+            if constexpr (g == SEGS - 1 && !next_tile) {
+            } else if constexpr (g % 4 == 3) {
                 constexpr int qn = next % STEPS;
                 if constexpr (qn * 64 % C::GS == 0 || qn == 0) make_consts(quant[next_win], qn);
                 dequant(wf[(g + 1) % 2], pk[next % 2], 0);
             } else {
                 dequant(wf[(g + 1) % 2], pk[step % 2], g % 4 + 1);
             }
-            // past the end of K the last window and the last tile are requested again: the waits count on the number
-            if constexpr (g == 0 && q == 0) load_quant(quant[(win + WS - 1) % WS], window_of(sup + WS - 1));
-            if constexpr (g == LAST_BEFORE && wide_window_requests<C>(q) > 0) request_w((win + WS - 1) % WS, window_of(sup + WS - 1), q);
-            if constexpr (g <= LAST_BEFORE) request_a(b2, min(it + 2, C::ITERS - 1), g, LAST_BEFORE + 1);
+            if constexpr (request_window && g == 0 && q == 0) load_quant(quant[(win + WS - 1) % WS], window_of(sup + WS - 1));
+            if constexpr (request_window && g == LAST_BEFORE && wide_window_requests<C>(q) > 0) request_w((win + WS - 1) % WS, window_of(sup + WS - 1), q);
+            if constexpr (request_tile && g <= LAST_BEFORE) request_a(b2, it + 2, g, LAST_BEFORE + 1);
             if constexpr (decltype(live_tag)::value != 0) multiply(wf[g % 2], af[g % C::SETS]);
-            interleave(IntTag<MT + (packed_here ? NT * (C::NBITS == 8 ? 2 : 1) : 0)>{});
-            if constexpr (g == LAST_BEFORE) {
-                wait_loads_and_barrier<QF_GEMM_FULL_DRAIN ? 0 : C::UA + wide_window_requests<C>(q)>();
+            interleave(IntTag<(next_tile || g + AHEAD < SEGS ? MT : 0) + (packed_here ? NT * (C::NBITS == 8 ? 2 : 1) : 0)>{});
+            if constexpr (g == LAST_BEFORE && next_tile) {
+                wait_loads_and_barrier<QF_GEMM_FULL_DRAIN ? 0 : requests>();
                 __builtin_amdgcn_sched_barrier(0);
             }
         });
     };
 
 #pragma unroll
-    for (int w = 0; w < WS - 1; w++) {
-        request_w(w, window_of(w), -1);
-        load_quant(quant[w], window_of(w));
-    }
-    request_a(0, 0, 0, 1);
-    request_a(1, min(1, C::ITERS - 1), 0, 1);
+    for (int w = 0; w < WS - 1; w++) load_quant(quant[w], window_of(w));
     wait_loads_and_barrier<0>();
     read_packed(pk[0], 0, 0);
 #pragma unroll
@@ -386,28 +393,30 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
         }
     };
     pin();
-    // whole passes (the period of the buffers and register sets) and a straight-line rest, which holds the window that
-    // some groups do not have: those meet the same barriers and requests without multiplying
+    // Whole passes (the period of the buffers and register sets) and a straight-line rest of at least two iterations, which
+    // also holds the window that some groups do not have: those meet the same barriers and requests without multiplying.
     constexpr int PASS = (WS == 3 ? 6 : 2) * SUP;
-    constexpr int FULL_PASSES = C::ITERS / PASS - (C::ODD != 0 && C::ITERS % PASS == 0 ? 1 : 0);
+    constexpr int FULL_PASSES = C::ITERS / PASS - (C::ITERS >= PASS && C::ITERS % PASS < 2 ? 1 : 0);
     constexpr int REST = C::ITERS - FULL_PASSES * PASS, SHARED = C::ODD != 0 ? SUP : 0;
     int b0 = 0, b1 = 1, b2 = 2;
-    auto step = [&](int it, auto s_tag, auto live_tag) __attribute__((always_inline)) {
-        iteration(it, s_tag, live_tag, b0, b1, b2);
+    auto step = [&](int it, auto s_tag, auto live_tag, auto left_tag) __attribute__((always_inline)) {
+        iteration(it, s_tag, live_tag, left_tag, b0, b1, b2);
         const int first = b0;
         b0 = b1; b1 = b2; b2 = first;
     };
+    auto rest = [&](auto s_tag, auto live_tag) __attribute__((always_inline)) {
+        constexpr int s = decltype(s_tag)::value;
+        step(FULL_PASSES * PASS + s, IntTag<s % PASS>{}, live_tag, IntTag<REST - 1 - s>{});
+    };
 #pragma unroll 1
     for (int pass = 0; pass < FULL_PASSES; pass++)
-        static_for<0, PASS>([&](auto s_tag) { step(pass * PASS + decltype(s_tag)::value, s_tag, IntTag<1>{}); });
-    static_for<0, REST - SHARED>([&](auto s_tag) { step(FULL_PASSES * PASS + decltype(s_tag)::value, s_tag, IntTag<1>{}); });
+        static_for<0, PASS>([&](auto s_tag) { step(pass * PASS + decltype(s_tag)::value, s_tag, IntTag<1>{}, IntTag<PASS + REST>{}); });
+    static_for<0, REST - SHARED>([&](auto s_tag) { rest(s_tag, IntTag<1>{}); });
     if constexpr (SHARED > 0) {
-        if (grp < C::ODD)
-            static_for<REST - SHARED, REST>([&](auto s_tag) { step(FULL_PASSES * PASS + decltype(s_tag)::value, s_tag, IntTag<1>{}); });
-        else
-            static_for<REST - SHARED, REST>([&](auto s_tag) { step(FULL_PASSES * PASS + decltype(s_tag)::value, s_tag, IntTag<0>{}); });
+        if (grp < C::ODD) static_for<REST - SHARED, REST>([&](auto s_tag) { rest(s_tag, IntTag<1>{}); });
+        else static_for<REST - SHARED, REST>([&](auto s_tag) { rest(s_tag, IntTag<0>{}); });
     }
-    wait_loads_and_barrier<0>();                               // the repeated requests of the last iterations target LDS: drained before the wave ends
+    wait_loads_and_barrier<0>();                               // every wave has read its last tile: LDS is free
 
     pin();
 
