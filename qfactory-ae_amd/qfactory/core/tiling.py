@@ -20,9 +20,12 @@ Five kernel families (``regime_for`` picks one):
   ``WK`` waves splitting K, ``SB`` tiles per batch, ``D`` stages in flight, ``AST`` resident fragments.
 * ``gemm``  -- larger M (and what ``mgemv`` cannot hold): ``qf::GemmCfg`` (include/qf_gemm.hip.h):
   ``BM`` activation rows per block, ``NT32`` 32-row weight tiles per wave, ``WN`` waves along N,
-  ``WK`` wave groups along K, ``PA`` activation tiles in flight.
+  ``WK`` wave groups along K, ``PA`` activation tiles in flight; from 17 rows on, where it takes the problem,
+  ``qf::GemmWideCfg`` (include/qf_gemm_wide.hip.h): ``WM`` x ``WN`` waves of ``MT`` x ``NT`` 32-row tiles, ``KI`` steps
+  of 64 elements per iteration.
 * ``mfma``  -- generic fallback, ``qf::MfmaCfg`` (include/qf_mfma.hip.h).
 """
+import functools
 import json
 import os
 
@@ -829,7 +832,7 @@ def gemm_candidates(M, N, K, nbits, group_size):
 
 # Tilings of the pipelined kernel (qf::GemmWideCfg, include/qf_gemm_wide.hip.h): (WM, WN, MT, NT, KI, WK) -> us per round
 # of blocks and 64 elements of K.  The figures are medians of a sweep of eighteen tilings over 22016 x 4096, 12288 x 4096,
-# 4096 x 4096, 4096 x 11008, 10240 x 8192, 8192 x 28672 and 57344 x 8192 at 33 ... 2048 rows (W4 g128, cold weights): with the
+# 4096 x 4096, 4096 x 11008, 10240 x 8192, 8192 x 28672 and 57344 x 8192 at 32 ... 2048 rows (W4 g128, cold weights): with the
 # round model of gemm_wide_tiling they pick the fastest of the sweep on all but three of its cells (2 - 7 % off there).
 GEMM_WIDE_COST = {
     (1, 4, 8, 2, 1, 1): 1.547,     # 256 x 256
@@ -839,13 +842,15 @@ GEMM_WIDE_COST = {
     (1, 4, 4, 1, 2, 1): 0.572,     # 128 x 128
     (1, 3, 4, 1, 2, 1): 0.505,     # 128 x 96
     (1, 4, 3, 1, 2, 1): 0.462,     # 96 x 128
-    (1, 4, 2, 1, 2, 2): 0.341,     # 64 x 128
+    (1, 7, 2, 1, 2, 1): 0.620,     # 64 x 224: 57344 columns are 256 of them
+    (1, 4, 2, 1, 2, 2): 0.338,     # 64 x 128
     (1, 3, 2, 1, 2, 2): 0.307,     # 64 x 96
     (1, 2, 2, 1, 2, 2): 0.217,     # 64 x 64
+    (1, 7, 1, 1, 2, 1): 0.528,     # 32 x 224
     (1, 2, 1, 1, 2, 4): 0.148,     # 32 x 64
     (1, 1, 1, 1, 2, 4): 0.100,     # 32 x 32
 }
-GEMM_WIDE_MIN_M = 33
+GEMM_WIDE_MIN_M = 17           # the 32-row bucket: 9280 x 4608 at 2 bits 13.9 -> 11.6 us, 8192 x 28672 49.8 -> 46.3, 8192 x 8192 level
 
 
 def gemm_wide_lds_bytes(cfg, nbits):
@@ -875,10 +880,16 @@ def gemm_wide_valid(cfg, K, nbits, group_size):
 
 
 def gemm_wide_tiling(M, N, K, nbits, group_size):
-    """Tiling of the pipelined kernel for this problem, None where the kernel of gemm_tiling serves: up to 32 rows, 3 bits,
+    """Tiling of the pipelined kernel for this problem, None where the kernel of gemm_tiling serves: up to 16 rows, 3 bits,
     and K that is not whole 128-byte windows.  A launch costs its exact number of rounds of blocks plus 40 % of the rounding
     up (rounds overlap), a single partial round 0.6 + 0.4 x the share of the CUs that get a block; a block row taller than
     twice the rows is not considered."""
+    cfg = _gemm_wide_tiling(M, N, K, nbits, group_size)
+    return None if cfg is None else dict(cfg)
+
+
+@functools.lru_cache(maxsize=4096)
+def _gemm_wide_tiling(M, N, K, nbits, group_size):
     if M < GEMM_WIDE_MIN_M:
         return None
     best = None
