@@ -13,12 +13,12 @@ extern "C" {
 #endif
 
 /*
- * qf_pack_weight and qf_pack_zero with the range check of the fields in the same pass: *bad (device memory, may be
- * null) is set to a nonzero value if any value lies outside [0, 2^nbits) and left alone otherwise; the caller clears
- * it first.
+ * qf_pack_weight, qf_transpose_scale and qf_pack_zero of one layer in one launch (scale and zero may be null), with the
+ * range check of the fields and zero-points in the same pass: *bad (device or pinned host memory, may be null) is set to a nonzero
+ * value if any lies outside [0, 2^nbits) and left alone otherwise; the caller clears it first.
  */
-int qf_pack_weight_checked(const int32_t* weight, int8_t* out, int64_t K, int64_t N, int nbits, uint32_t* bad, void* stream);
-int qf_pack_zero_checked(const int32_t* zero, int8_t* out, int64_t G, int64_t N, int nbits, uint32_t* bad, void* stream);
+int qf_pack_layer(const int32_t* weight, int8_t* w_out, const uint16_t* scale, uint16_t* s_out, const int32_t* zero, int8_t* z_out,
+                  int64_t K, int64_t N, int64_t G, int nbits, uint32_t* bad, void* stream);
 
 /*
  * Causal attention of `tokens` positions of every sequence over its cache: q and out (batch, tokens, heads, head_dim)

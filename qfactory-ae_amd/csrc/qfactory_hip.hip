@@ -49,6 +49,11 @@ __host__ __device__ constexpr int field_bit(int e) {
     return B == 8 ? 8 * e : B == 1 ? hi_plane_pos(e) : B * (e / 2 + (e % 2) * (16 / B));
 }
 
+// the word may be host memory: a plain store at system scope
+__device__ __forceinline__ void report(uint32_t* bad) {
+    __hip_atomic_store(bad, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <int NBITS>
 struct PackCfg {
     static constexpr int B = NBITS == 3 ? 2 : NBITS;           // field width of the main plane
@@ -64,13 +69,13 @@ struct PackCfg {
 
 // VEC: N a multiple of four and 16-byte aligned rows, four columns per load; otherwise single words
 template <int NBITS, bool VEC>
-__global__ __launch_bounds__(256) void pack_weight_kernel(const int32_t* __restrict__ weight, uint32_t* __restrict__ out,
-                                                          int64_t K, int64_t N, uint32_t* __restrict__ bad) {
+__device__ __forceinline__ void pack_weight_tile(int64_t bx, int64_t by, const int32_t* __restrict__ weight, uint32_t* __restrict__ out,
+                                                 int64_t K, int64_t N, uint32_t* __restrict__ bad) {
     using C = PackCfg<NBITS>;
     __shared__ uint32_t tile[64][C::PITCH];
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int64_t n0 = (int64_t)blockIdx.x * 64, n = n0 + 4 * tx;
-    const int64_t k_blk = (int64_t)blockIdx.y * C::KB;
+    const int64_t n0 = bx * 64, n = n0 + 4 * tx;
+    const int64_t k_blk = by * C::KB;
     constexpr uint32_t MASK = (1u << NBITS) - 1u;
     uint32_t seen = 0;
 #pragma unroll
@@ -106,16 +111,16 @@ __global__ __launch_bounds__(256) void pack_weight_kernel(const int32_t* __restr
             if constexpr (NBITS == 3) tile[4 * tx + c][C::WORDS + unit] = high[c];
         }
     }
-    if (bad != nullptr && __any((seen & ~MASK) != 0) && (threadIdx.x & 63) == 0) atomicOr(bad, 1u);
+    if (bad != nullptr && __any((seen & ~MASK) != 0) && (threadIdx.x & 63) == 0) report(bad);
     __syncthreads();
     const int64_t row_words = K * NBITS / 32;
-    const int64_t w0 = (int64_t)blockIdx.y * C::WORDS;
+    const int64_t w0 = by * C::WORDS;
     for (int i = threadIdx.x; i < 64 * C::WORDS; i += 256) {
         const int r = i / C::WORDS, w = i % C::WORDS;
         if (n0 + r < N && w0 + w < K / C::P) out[(n0 + r) * row_words + w0 + w] = tile[r][w];
     }
     if constexpr (NBITS == 3) {                                 // the 1-bit plane behind the row's 2-bit plane
-        const int64_t h0 = (int64_t)blockIdx.y * C::HI;
+        const int64_t h0 = by * C::HI;
         for (int i = threadIdx.x; i < 64 * C::HI; i += 256) {
             const int r = i / C::HI, w = i % C::HI;
             if (n0 + r < N && h0 + w < K / 32) out[(n0 + r) * row_words + K / 16 + h0 + w] = tile[r][C::WORDS + w];
@@ -123,20 +128,11 @@ __global__ __launch_bounds__(256) void pack_weight_kernel(const int32_t* __restr
     }
 }
 
-template <int NBITS>
-void launch_pack(const int32_t* weight, int8_t* out, int64_t K, int64_t N, uint32_t* bad, hipStream_t stream) {
-    const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((K + PackCfg<NBITS>::KB - 1) / PackCfg<NBITS>::KB));
-    const bool vec = N % 4 == 0 && (uintptr_t)weight % 16 == 0;
-    hipLaunchKernelGGL((vec ? pack_weight_kernel<NBITS, true> : pack_weight_kernel<NBITS, false>), grid, dim3(256), 0, stream,
-                       weight, (uint32_t*)out, K, N, bad);
-}
-
-__global__ __launch_bounds__(256) void pack_zero_kernel(const int32_t* __restrict__ zero, uint8_t* __restrict__ out,
-                                                        int64_t G, int64_t N, int nbits, int fb,
-                                                        uint32_t* __restrict__ bad) {
+__device__ __forceinline__ void pack_zero_tile(int64_t block, const int32_t* __restrict__ zero, uint8_t* __restrict__ out,
+                                               int64_t G, int64_t N, int nbits, int fb, uint32_t* __restrict__ bad) {
     const int p8 = 8 / fb;
     const int64_t row_bytes = G / p8;
-    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;      // over N * row_bytes, n fastest
+    const int64_t idx = block * 256 + threadIdx.x;      // over N * row_bytes, n fastest
     if (idx >= N * row_bytes) return;
     const int64_t n = idx % N, byte = idx / N;
     const int32_t maxv = (1 << nbits) - 1;
@@ -149,19 +145,74 @@ __global__ __launch_bounds__(256) void pack_zero_kernel(const int32_t* __restric
         v |= (uint32_t)z << (i * fb);
     }
     out[n * row_bytes + byte] = (uint8_t)v;
-    if (bad != nullptr && (seen & ~(uint32_t)maxv) != 0) atomicOr(bad, 1u);
+    if (bad != nullptr && (seen & ~(uint32_t)maxv) != 0) report(bad);
 }
 
-__global__ __launch_bounds__(256) void transpose_u16_kernel(const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
-                                                            int64_t G, int64_t N) {
+__device__ __forceinline__ void transpose_u16_tile(int64_t bx, int64_t by, const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
+                                                   int64_t G, int64_t N) {
     __shared__ uint16_t tile[32][33];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;           // 32 x 8
-    const int64_t n0 = (int64_t)blockIdx.x * 32, g0 = (int64_t)blockIdx.y * 32;
+    const int64_t n0 = bx * 32, g0 = by * 32;
     for (int r = ty; r < 32; r += 8)
         if (g0 + r < G && n0 + tx < N) tile[r][tx] = in[(g0 + r) * N + n0 + tx];
     __syncthreads();
     for (int r = ty; r < 32; r += 8)
         if (n0 + r < N && g0 + tx < G) out[(n0 + r) * G + g0 + tx] = tile[tx][r];
+}
+
+// The three tensors of a layer in one launch: the scale and zero-point blocks come first and run under the weight's (as
+// launches of their own behind it they took 5 and 6 us on 4096 x 22016, almost all of it latency).  Any of the three may
+// have no blocks.
+struct PackJob {
+    const int32_t* weight; uint32_t* w_out;
+    const uint16_t* scale; uint16_t* s_out;
+    const int32_t* zero; uint8_t* z_out;
+    int64_t K, N, G;
+    int nbits, fb;
+    uint32_t* bad;
+    unsigned scale_blocks, zero_blocks;
+};
+
+template <int NBITS, bool VEC>
+__global__ __launch_bounds__(256) void pack_layer_kernel(PackJob j) {
+    unsigned b = blockIdx.x;
+    if (b < j.scale_blocks) {
+        const unsigned columns = (unsigned)((j.N + 31) / 32);
+        transpose_u16_tile(b % columns, b / columns, j.scale, j.s_out, j.G, j.N);
+        return;
+    }
+    b -= j.scale_blocks;
+    if (b < j.zero_blocks) {
+        pack_zero_tile(b, j.zero, j.z_out, j.G, j.N, j.nbits, j.fb, j.bad);
+        return;
+    }
+    b -= j.zero_blocks;
+    const unsigned columns = (unsigned)((j.N + 63) / 64);
+    pack_weight_tile<NBITS, VEC>(b % columns, b / columns, j.weight, j.w_out, j.K, j.N, j.bad);
+}
+
+template <int NBITS>
+int launch_layer(const char* fn, PackJob j, hipStream_t stream) {
+    const int64_t weight_blocks = j.weight ? (j.N + 63) / 64 * ((j.K + PackCfg<NBITS>::KB - 1) / PackCfg<NBITS>::KB) : 0;
+    const int64_t scale_blocks = j.scale ? (j.N + 31) / 32 * ((j.G + 31) / 32) : 0;
+    const int64_t zero_blocks = j.zero ? (j.N * (j.G / (8 / j.fb)) + 255) / 256 : 0;
+    if (weight_blocks + scale_blocks + zero_blocks > 0x7fffffff) return fail(fn, "too many blocks");
+    j.scale_blocks = (unsigned)scale_blocks;
+    j.zero_blocks = (unsigned)zero_blocks;
+    const bool vec = j.N % 4 == 0 && (uintptr_t)j.weight % 16 == 0;
+    hipLaunchKernelGGL((vec ? pack_layer_kernel<NBITS, true> : pack_layer_kernel<NBITS, false>),
+                       dim3((unsigned)(weight_blocks + scale_blocks + zero_blocks)), dim3(256), 0, stream, j);
+    return launched(fn);
+}
+
+int launch_layer(const char* fn, const PackJob& j, hipStream_t stream) {
+    switch (j.nbits) {
+        case 8: return launch_layer<8>(fn, j, stream);
+        case 4: return launch_layer<4>(fn, j, stream);
+        case 3: return launch_layer<3>(fn, j, stream);
+        case 2: return launch_layer<2>(fn, j, stream);
+        default: return fail(fn, "nbits must be 2, 3, 4 or 8");
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -241,49 +292,42 @@ extern "C" int qf_bf16_to_f16(const uint16_t* src, uint16_t* dst, int64_t n, voi
     return launched("qf_bf16_to_f16");
 }
 
-extern "C" int qf_pack_weight_checked(const int32_t* weight, int8_t* out, int64_t K, int64_t N, int nbits, uint32_t* bad,
-                                      void* stream_) {
-    hipStream_t stream = (hipStream_t)stream_;
-    if (!weight || !out) return fail("qf_pack_weight", "null pointer");
-    if (K <= 0 || N <= 0 || K % 32 != 0) return fail("qf_pack_weight", "K must be a positive multiple of 32, N positive");
-    switch (nbits) {
-        case 8: launch_pack<8>(weight, out, K, N, bad, stream); break;
-        case 4: launch_pack<4>(weight, out, K, N, bad, stream); break;
-        case 3: launch_pack<3>(weight, out, K, N, bad, stream); break;
-        case 2: launch_pack<2>(weight, out, K, N, bad, stream); break;
-        default: return fail("qf_pack_weight", "nbits must be 2, 3, 4 or 8");
-    }
-    return launched("qf_pack_weight");
+extern "C" int qf_pack_layer(const int32_t* weight, int8_t* w_out, const uint16_t* scale, uint16_t* s_out, const int32_t* zero,
+                             int8_t* z_out, int64_t K, int64_t N, int64_t G, int nbits, uint32_t* bad, void* stream_) {
+    const char* fn = "qf_pack_layer";
+    if (!weight || !w_out || (scale && !s_out) || (zero && !z_out)) return fail(fn, "null pointer");
+    if (K <= 0 || N <= 0 || K % 32 != 0) return fail(fn, "K must be a positive multiple of 32, N positive");
+    const int fb = nbits == 3 ? 4 : nbits;
+    if ((scale || zero) && G <= 0) return fail(fn, "G must be positive");
+    if (nbits != 2 && nbits != 3 && nbits != 4 && nbits != 8) return fail(fn, "nbits must be 2, 3, 4 or 8");
+    if (zero && G % (8 / fb) != 0) return fail(fn, "G must fill whole bytes of zero-points");
+    return launch_layer(fn, PackJob{weight, (uint32_t*)w_out, scale, s_out, zero, (uint8_t*)z_out, K, N, G, nbits, fb, bad, 0, 0},
+                        (hipStream_t)stream_);
 }
 
 extern "C" int qf_pack_weight(const int32_t* weight, int8_t* out, int64_t K, int64_t N, int nbits, void* stream_) {
-    return qf_pack_weight_checked(weight, out, K, N, nbits, nullptr, stream_);
-}
-
-extern "C" int qf_pack_zero_checked(const int32_t* zero, int8_t* out, int64_t G, int64_t N, int nbits, uint32_t* bad,
-                                    void* stream_) {
-    hipStream_t stream = (hipStream_t)stream_;
-    if (!zero || !out) return fail("qf_pack_zero", "null pointer");
-    if (nbits != 2 && nbits != 3 && nbits != 4 && nbits != 8) return fail("qf_pack_zero", "nbits must be 2, 3, 4 or 8");
-    const int fb = nbits == 3 ? 4 : nbits;
-    if (G <= 0 || N <= 0 || G % (8 / fb) != 0) return fail("qf_pack_zero", "G must fill whole bytes of zero-points");
-    const int64_t total = N * (G / (8 / fb));
-    hipLaunchKernelGGL(pack_zero_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, zero, (uint8_t*)out, G,
-                       N, nbits, fb, bad);
-    return launched("qf_pack_zero");
+    const char* fn = "qf_pack_weight";
+    if (!weight || !out) return fail(fn, "null pointer");
+    if (K <= 0 || N <= 0 || K % 32 != 0) return fail(fn, "K must be a positive multiple of 32, N positive");
+    return launch_layer(fn, PackJob{weight, (uint32_t*)out, nullptr, nullptr, nullptr, nullptr, K, N, 0, nbits, 8, nullptr, 0, 0},
+                        (hipStream_t)stream_);
 }
 
 extern "C" int qf_pack_zero(const int32_t* zero, int8_t* out, int64_t G, int64_t N, int nbits, void* stream_) {
-    return qf_pack_zero_checked(zero, out, G, N, nbits, nullptr, stream_);
+    const char* fn = "qf_pack_zero";
+    if (!zero || !out) return fail(fn, "null pointer");
+    if (nbits != 2 && nbits != 3 && nbits != 4 && nbits != 8) return fail(fn, "nbits must be 2, 3, 4 or 8");
+    const int fb = nbits == 3 ? 4 : nbits;
+    if (G <= 0 || N <= 0 || G % (8 / fb) != 0) return fail(fn, "G must fill whole bytes of zero-points");
+    return launch_layer(fn, PackJob{nullptr, nullptr, nullptr, nullptr, zero, (uint8_t*)out, 0, N, G, nbits, fb, nullptr, 0, 0},
+                        (hipStream_t)stream_);
 }
 
 extern "C" int qf_transpose_scale(const uint16_t* scale, uint16_t* out, int64_t G, int64_t N, void* stream_) {
-    hipStream_t stream = (hipStream_t)stream_;
-    if (!scale || !out) return fail("qf_transpose_scale", "null pointer");
-    if (G <= 0 || N <= 0) return fail("qf_transpose_scale", "G and N must be positive");
-    dim3 grid((unsigned)((N + 31) / 32), (unsigned)((G + 31) / 32));
-    hipLaunchKernelGGL(transpose_u16_kernel, grid, dim3(256), 0, stream, scale, out, G, N);
-    return launched("qf_transpose_scale");
+    const char* fn = "qf_transpose_scale";
+    if (!scale || !out) return fail(fn, "null pointer");
+    if (G <= 0 || N <= 0) return fail(fn, "G and N must be positive");
+    return launch_layer(fn, PackJob{nullptr, nullptr, scale, out, nullptr, nullptr, 0, N, G, 8, 8, nullptr, 0, 0}, (hipStream_t)stream_);
 }
 
 __global__ void empty_kernel(uint32_t* sink) {

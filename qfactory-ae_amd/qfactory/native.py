@@ -44,8 +44,7 @@ SIGNATURES = {
 
 # the same for include/qfactory_hip_ext.h
 EXT_SIGNATURES = {
-    "qf_pack_weight_checked": (_INT, [_P, _P, _I64, _I64, _INT, _P, _P]),
-    "qf_pack_zero_checked": (_INT, [_P, _P, _I64, _I64, _INT, _P, _P]),
+    "qf_pack_layer": (_INT, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _INT, _P, _P]),
     "qf_prefill_attention": (_INT, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P]),
 }
 
@@ -93,27 +92,45 @@ def _check(rc, what):
         raise RuntimeError(f"{what} failed with return code {rc}")
 
 
-def pack_weight(weight, nbits, bad=None):
-    """(K, N) int32 device tensor -> (N, K*nbits/8) int8, bit-identical to convert._transform_weight_basic.  ``bad``: a
-    one-element int32 device tensor, set nonzero if a field lies outside [0, 2^nbits)."""
+def pack_layer(weight, scale, zero, nbits, bad):
+    """The packed tensors of one layer in one launch: weight (K, N) int32, scale (G, N) fp16 or None, zero (G, N) int32 or
+    None -> (w, s, z) as of ``pack_weight``, ``transpose_scale`` and ``pack_zero``.  ``bad``: a one-element int32 tensor on
+    the device or in pinned host memory, set nonzero if a field or zero-point lies outside [0, 2^nbits)."""
+    import torch
+    for t, dtype in ((weight, torch.int32), (scale, torch.float16), (zero, torch.int32)):
+        assert t is None or (t.is_cuda and t.dtype == dtype and t.is_contiguous() and t.dim() == 2 and t.device == weight.device)
+    K, N = weight.shape
+    G = scale.shape[0] if scale is not None else zero.shape[0] if zero is not None else 0
+    fb = 4 if nbits == 3 else nbits
+    assert all(t is None or t.shape == (G, N) for t in (scale, zero))
+    new = lambda *shape, dtype=torch.int8: torch.empty(*shape, dtype=dtype, device=weight.device)
+    w = new(N, K * nbits // 8)
+    s = None if scale is None else new(N, G, dtype=torch.float16)
+    z = None if zero is None else new(N, G * fb // 8)
+    address = lambda t: None if t is None else t.data_ptr()
+    _check(load().qf_pack_layer(weight.data_ptr(), w.data_ptr(), address(scale), address(s), address(zero), address(z), K, N, G,
+                                nbits, bad.data_ptr(), _stream()), "qf_pack_layer")
+    return w, s, z
+
+
+def pack_weight(weight, nbits):
+    """(K, N) int32 device tensor -> (N, K*nbits/8) int8, bit-identical to convert._transform_weight_basic."""
     import torch
     assert weight.is_cuda and weight.dtype == torch.int32 and weight.is_contiguous() and weight.dim() == 2
     K, N = weight.shape
     out = torch.empty(N, K * nbits // 8, dtype=torch.int8, device=weight.device)
-    _check(load().qf_pack_weight_checked(weight.data_ptr(), out.data_ptr(), K, N, nbits, bad.data_ptr() if bad is not None else None,
-                                         _stream()), "qf_pack_weight")
+    _check(load().qf_pack_weight(weight.data_ptr(), out.data_ptr(), K, N, nbits, _stream()), "qf_pack_weight")
     return out
 
 
-def pack_zero(zero, nbits, bad=None):
-    """(G, N) int32 device tensor -> (N, G*fb/8) int8 holding min(zero + 1, 2^nbits - 1); ``bad`` as for ``pack_weight``."""
+def pack_zero(zero, nbits):
+    """(G, N) int32 device tensor -> (N, G*fb/8) int8 holding min(zero + 1, 2^nbits - 1)."""
     import torch
     assert zero.is_cuda and zero.dtype == torch.int32 and zero.is_contiguous() and zero.dim() == 2
     G, N = zero.shape
     fb = 4 if nbits == 3 else nbits
     out = torch.empty(N, G * fb // 8, dtype=torch.int8, device=zero.device)
-    _check(load().qf_pack_zero_checked(zero.data_ptr(), out.data_ptr(), G, N, nbits, bad.data_ptr() if bad is not None else None,
-                                       _stream()), "qf_pack_zero")
+    _check(load().qf_pack_zero(zero.data_ptr(), out.data_ptr(), G, N, nbits, _stream()), "qf_pack_zero")
     return out
 
 

@@ -89,10 +89,18 @@ def test_weight_packer_at_tile_edges(oracle, nbits, K, N, offset):
     store = torch.empty(K * N + offset, dtype=torch.int32, device="cuda")
     dev = store[offset:].view(K, N)
     dev.copy_(weight)
-    bad = torch.zeros(1, dtype=torch.int32, device="cuda")
-    w = native.pack_weight(dev, nbits, bad)
-    assert bad.item() == 0
-    assert np.array_equal(w.cpu().numpy(), oracle.pack_weight(weight.numpy(), nbits))
+    want = oracle.pack_weight(weight.numpy(), nbits)
+    assert np.array_equal(native.pack_weight(dev, nbits).cpu().numpy(), want)
+    G = 8                                            # whole bytes of zero-points at every width
+    scale = torch.rand(G, N, generator=g).to(torch.float16)
+    zero = torch.randint(0, 2 ** nbits, (G, N), dtype=torch.int32, generator=g)
+    for s, z in ((scale, zero), (scale, None), (None, None), (None, zero)):
+        bad = torch.zeros(1, dtype=torch.int32, device="cuda")
+        packed = native.pack_layer(dev, None if s is None else s.cuda(), None if z is None else z.cuda(), nbits, bad)
+        assert bad.item() == 0
+        assert np.array_equal(packed[0].cpu().numpy(), want)
+        assert packed[1] is None if s is None else np.array_equal(packed[1].cpu().numpy(), oracle.transpose_scale(s.numpy()))
+        assert packed[2] is None if z is None else np.array_equal(packed[2].cpu().numpy(), oracle.pack_zero(z.numpy(), nbits))
 
 
 @pytest.mark.parametrize("nbits", [2, 3, 4, 8])
