@@ -71,6 +71,12 @@ def get_qfactory_version(code: str = None) -> str:
     objects of the other kernel families valid when one header changes).  Without ``code``: every header."""
     if code is None:
         code = "".join(f'#include "{f}"\n' for d in include_dirs() for f in sorted(os.listdir(d)) if f.endswith(".h"))
+    # the headers' text is read once per process: so is the digest of what a set of includes reaches (every layer asks,
+    # and hashing 120 KB of headers each time was half of a layer's construction from compiled objects)
+    key = ("version", tuple(include_dirs()), tuple(_INCLUDE_RE.findall(code)))
+    with _lock:
+        if key in _memo:
+            return _memo[key]
     seen, queue = {}, [code]
     while queue:
         for name in _INCLUDE_RE.findall(queue.pop()):
@@ -82,7 +88,9 @@ def get_qfactory_version(code: str = None) -> str:
     for path in sorted(seen):
         md5.update(os.path.basename(path).encode())
         md5.update(seen[path].encode())
-    return md5.hexdigest()[0:12]
+    with _lock:
+        _memo[key] = md5.hexdigest()[0:12]
+        return _memo[key]
 
 
 def get_hipcc_compiler():
