@@ -28,7 +28,7 @@ def _m_bucket(m):
         return 16
     bucket = 32
     # 512 .. 4096: prefill-sized tiles.  Several rounds of blocks pay for 256 x 256 tiles where one round of the
-    # same layer does not (4096 x 11008: 128 x 128 tiles at 1024 rows, 256 x 256 from 4096 rows on, 884 -> 699 us at 8192 rows)
+    # same layer does not (4096 x 11008: 128 x 128 tiles at 1024 rows, 256 x 256 from 4096 rows on: 550 us at 8192 rows)
     while bucket < m and bucket < 4096:
         bucket *= 2
     return bucket
