@@ -339,7 +339,7 @@ def wide_cases():
         (65, 140, 1280, 4, 128, False, (1, 4, 2, 1, 2, 2)), (64, 104, 2816, 4, 64, False, (1, 3, 2, 1, 2, 2)),
         (50, 64, 2048, 2, 128, False, (1, 2, 2, 1, 2, 2)), (70, 132, 640, 8, 64, False, (1, 4, 2, 1, 1, 2)),
         (33, 72, 2816, 4, 128, False, (1, 2, 1, 1, 2, 4)), (40, 33, 3328, 4, 128, False, (1, 1, 1, 1, 2, 4)),
-        (34, 68, 1152, 8, 64, True, (1, 2, 1, 1, 1, 4))]]
+        (34, 68, 1152, 8, 64, True, (1, 2, 1, 1, 1, 4))]] + [_case(256, 12288, 1024)]
 
 
 def search_cases():

@@ -881,8 +881,8 @@ def gemm_wide_valid(cfg, K, nbits, group_size):
 
 def gemm_wide_tiling(M, N, K, nbits, group_size):
     """Tiling of the pipelined kernel for this problem, None where the kernel of gemm_tiling serves: up to 16 rows, 3 bits,
-    and K that is not whole 128-byte windows.  A launch costs its exact number of rounds of blocks plus 40 % of the rounding
-    up (rounds overlap), a single partial round 0.6 + 0.4 x the share of the CUs that get a block; a block row taller than
+    and K that is not whole 128-byte windows.  A launch costs its whole rounds of blocks (one block per CU), each 0.6 + 0.4 x the
+    mean share of the CUs that get a block (a machine that is not full clocks higher and shares L2 among fewer); a block row taller than
     twice the rows is not considered."""
     cfg = _gemm_wide_tiling(M, N, K, nbits, group_size)
     return None if cfg is None else dict(cfg)
@@ -906,10 +906,25 @@ def _gemm_wide_tiling(M, N, K, nbits, group_size):
         else:
             continue
         exact = (-(-N // bn) * -(-M // bm)) / NUM_CUS
-        rounds = exact + 0.4 * (-(-exact // 1) - exact) if exact > 1 else 0.6 + 0.4 * exact
-        if best is None or rounds * per_step < best[0]:
-            best = (rounds * per_step, cfg)
+        whole = -(-exact // 1)
+        cost = (0.6 * whole + 0.4 * exact) * per_step
+        if best is None or cost < best[0]:
+            best = (cost, cfg)
     return None if best is None else best[1]
+
+
+GEMM_WIDE_LOW = (256, 4096)     # row-count buckets whose objects hold a second tiling
+
+
+def gemm_wide_low_tiling(M, N, K, nbits, group_size):
+    """A bucket's object serves every row count above half of it, and 256-row slabs that fit the full bucket compute up to
+    half a slab too much on the others (290 rows on 33088 x 11008: two slabs of 256, 362 us, against three of 128).  Buckets of 256 ...
+    4096 rows therefore carry the tiling of their lower half, 11/16 of the rows, as well; a launch of at most 3/4 of the
+    bucket's rows takes it.  None where the two are the same."""
+    if M & (M - 1) or not GEMM_WIDE_LOW[0] <= M <= GEMM_WIDE_LOW[1]:
+        return None
+    low = gemm_wide_tiling(11 * M // 16, N, K, nbits, group_size)
+    return None if low is None or low == gemm_wide_tiling(M, N, K, nbits, group_size) else low
 
 
 def gemm_wide_cfg_string(problem, t):

@@ -184,7 +184,13 @@ class JITCompiler:
             if counted_waits:
                 isa = "".join(open(os.path.join(work_dir, f)).read() for f in sorted(os.listdir(work_dir))
                               if f.endswith(".s") and "amdgcn" in f)
-                ok, detail = self.check_gemm_waits(isa, qfunc.tiling_configs["PA"])
+                # an object may hold two kernels (a tiling for each half of its row counts): each is checked
+                kernels = [k for k in re.split(r"^\.Lfunc_end\d+:", isa, flags=re.MULTILINE) if re.search(r"^_Z\w+:", k, flags=re.MULTILINE)]
+                ok, detail = False, "no kernel found in the listing"
+                for kernel in kernels:
+                    ok, detail = self.check_gemm_waits(kernel, qfunc.tiling_configs["PA"])
+                    if not ok:
+                        break
                 if not ok:
                     logger.warning(f"GEMM object {runtime_path}: {detail}; rebuilding with a full drain per K-iteration")
                     command = [c for c in command if c != "-save-temps"] + ["-DQF_GEMM_FULL_DRAIN=1"]

@@ -24,7 +24,7 @@ def _launch(runtime, x, layer, out):
     assert rc == 0
 
 
-@pytest.mark.parametrize("case", prebuild.wide_cases(), ids=_id)
+@pytest.mark.parametrize("case", [c for c in prebuild.wide_cases() if "tiling" in c], ids=_id)
 def test_tilings_at_their_edges(oracle, case):
     from qfactory import QLinear
     from qfactory.jit import jit
@@ -53,3 +53,18 @@ def test_tilings_at_their_edges(oracle, case):
         store.fill_(float("nan"))
         _launch(runtime, shifted[:rows], layer, store[:rows])
         assert torch.equal(first[:rows], store[:rows]) and store[rows:].isnan().all()
+
+
+@pytest.mark.parametrize("rows", [129, 192, 193, 256])
+def test_both_tilings_of_a_row_count_bucket(oracle, rows):
+    """The object of the 256-row bucket holds a tiling for launches of at most 192 rows and one for the others."""
+    from qfactory import QLinear
+    from qfactory.core import tiling
+    N, K = 12288, 1024
+    assert tiling.gemm_wide_low_tiling(256, N, K, 4, 128) not in (None, tiling.gemm_wide_tiling(256, N, K, 4, 128))
+    A, weight, scale, zero = make_problem(rows, rows, N, K, 4, 128)
+    layer = QLinear.init(256, K, N, 4, weight.cuda(), 128, scale.cuda(), zero.cuda(), compile_flags=NO_SEARCH)
+    out = layer(A.cuda())
+    columns = list(range(0, N, 97))
+    ref = reference_output(oracle, A, layer.w, layer.s, layer.z, 4, 128, rows=columns)
+    assert_close(oracle, out[:, columns].cpu().numpy(), ref, f"{rows} rows")
