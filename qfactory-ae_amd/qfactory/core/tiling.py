@@ -833,7 +833,7 @@ def gemm_candidates(M, N, K, nbits, group_size):
 # Tilings of the pipelined kernel (qf::GemmWideCfg, include/qf_gemm_wide.hip.h): (WM, WN, MT, NT, KI, WK) -> us per round
 # of blocks and 64 elements of K.  The figures are medians of a sweep of eighteen tilings over 22016 x 4096, 12288 x 4096,
 # 4096 x 4096, 4096 x 11008, 10240 x 8192, 8192 x 28672 and 57344 x 8192 at 32 ... 2048 rows (W4 g128, cold weights): with the
-# round model of gemm_wide_tiling they pick the fastest of the sweep on all but three of its cells (2 - 7 % off there).
+# round model of gemm_wide_tiling they pick the fastest of the sweep on nearly all of its cells (up to 7 % off on the others).
 GEMM_WIDE_COST = {
     (1, 4, 8, 2, 1, 1): 1.547,     # 256 x 256
     (2, 2, 4, 3, 1, 1): 1.289,     # 256 x 192
