@@ -577,7 +577,12 @@ __global__ __launch_bounds__(C::T) void gemm_kernel(
     if constexpr (C::SPREAD == 0) load_super(ringW[0], 2, -1);
     read_packed(cur, is_tail(0) ? C::TAIL_SHIFT : 0);
     wait_loads_and_barrier<0>();
-    if constexpr (C::PREFETCH_A) read_frags(fcur, 0);
+    if constexpr (C::PREFETCH_A) {
+        read_frags(fcur, 0);
+        // Iteration 0 requests tile PA into the buffer of tile 0, and the other waves of the group read that buffer too: all
+        // of them have to have their fragments first (every later request finds its buffer's reads behind an iteration's barrier).
+        wait_loads_and_barrier<0>();
+    }
 
     // The K loop runs whole passes of 2*SUP iterations (the period of the register rings); what is left over is
     // a straight-line tail behind it.  No iteration is skipped by a branch inside the loop, so every path through

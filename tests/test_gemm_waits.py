@@ -56,6 +56,35 @@ def test_wave_counts_that_do_not_divide_the_activation_tile(M, N, K, tile, tmp_p
     assert ok, detail
 
 
+def _barriers_around_the_first_tile(isa):
+    """Fragment reads between the barrier that publishes tile 0 and the next barrier of the GEMM kernel's listing, in the
+    order of the text, and the tile requests among them; None if the wave's own reads may be open at that barrier."""
+    reads, requests, drained, published = 0, 0, False, False
+    for line in (raw.strip() for raw in isa.splitlines()):
+        if line.startswith("s_barrier"):
+            if published:
+                return (reads, requests) if drained else None
+            published = True
+        elif published and line.startswith("ds_read"):
+            reads, drained = reads + 1, False
+        elif published and line.startswith("global_load_lds"):
+            requests += 1
+        elif line.startswith("s_waitcnt") and "lgkmcnt(0)" in line:
+            drained = True
+    raise AssertionError("fewer than two barriers in the listing")
+
+
+@pytest.mark.parametrize("M,N,K,nbits,gs,sets", [(48, 64, 2816, 3, 64, 4), (70, 96, 4224, 4, 32, 4), (128, 4096, 4096, 3, 128, 4),
+                                                (256, 4096, 4096, 3, 128, 8), (512, 10240, 8192, 3, 128, 16), (40, 96, 192, 8, 64, 4)])
+def test_first_tile_is_read_before_its_buffer_is_requested_again(M, N, K, nbits, gs, sets, tmp_path):
+    """Iteration 0 requests tile PA into the buffer of tile 0, which every wave of the group reads: between the barrier
+    that publishes tile 0 and that request each wave has its fragments (four per 32 rows) and has met the others."""
+    q = _gemm_qfunc(M, N, K, nbits, gs)
+    assert "NT32" in q.tiling_configs and q.tiling_configs["BM"] == 8 * sets         # qf_gemm.hip.h, with fragment prefetch
+    found = _barriers_around_the_first_tile(_isa_of(q, tmp_path))
+    assert found is not None and found[0] >= sets and found[1] == 0, found
+
+
 def test_checker_rejects_a_missing_load():
     from qfactory.jit.verify import gemm_waits_hold
     load = "\tglobal_load_dwordx4 v[0:3], v4, s[0:1]"
