@@ -203,7 +203,8 @@ def _packs_in_one_launch(K, weight, scale, zero, nbits):
 def _pack_layer(weight, scale, zero, nbits):
     from . import native
     # pinned host memory: clearing it is no launch and reading it no copy (103 -> 101 us on 4096 x 22016, a first pass 144 -> 128)
-    bad = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    # (on the host by name: only host memory can be pinned, and the caller's default device may be another)
+    bad = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
     packed = native.pack_layer(weight.contiguous(), None if scale is None else scale.contiguous(),
                                None if zero is None else zero.contiguous(), nbits, bad)
     torch.cuda.current_stream().synchronize()                   # the one wait for the device, behind the packing launch

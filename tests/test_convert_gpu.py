@@ -124,3 +124,24 @@ def test_values_out_of_range_are_refused(nbits, value):
     bad[-1, -1] = v
     with pytest.raises(AssertionError):
         convert.convert_params(args, (weight, scale, bad))
+
+
+@pytest.mark.parametrize("nbits", [3, 4])
+def test_conversion_under_a_default_device(oracle, nbits):
+    """A loader that makes its tensors under ``torch.device("cuda")``: the same bytes, the same refusals, and a layer."""
+    from qfactory import QLinear, convert
+    K, N, GS = 512, 68, 64
+    weight, scale, zero = _tensors(nbits, K, N, nbits, GS)
+    args = {"K": K, "N": N, "NBITS": nbits, "GS": GS}
+    with torch.device("cuda"):
+        w, s, z = convert.convert_params(args, (weight.cuda(), scale.cuda(), zero.cuda()))
+        assert all(t.is_cuda for t in (w, s, z))
+        with pytest.raises(AssertionError):
+            convert.convert_params(args, (weight.cuda() + 2 ** nbits, scale.cuda(), zero.cuda()))
+    assert np.array_equal(w.cpu().numpy(), oracle.pack_weight(weight.numpy(), nbits))
+    assert np.array_equal(s.cpu().numpy(), oracle.transpose_scale(scale.numpy()))
+    assert np.array_equal(z.cpu().numpy(), oracle.pack_zero(zero.numpy(), nbits))
+    with torch.device("cuda"):
+        layer = QLinear.init(1, 512, 96, 4, torch.ones(512, 96, dtype=torch.int32), 128, torch.ones(4, 96, dtype=torch.float16),
+                             torch.zeros(4, 96, dtype=torch.int32), compile_flags={})
+        assert torch.equal(layer(torch.ones(1, 512, dtype=torch.float16)), torch.zeros(1, 96, dtype=torch.float16))
