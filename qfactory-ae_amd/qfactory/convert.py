@@ -205,9 +205,11 @@ def _pack_layer(weight, scale, zero, nbits):
     # pinned host memory: clearing it is no launch and reading it no copy (103 -> 101 us on 4096 x 22016, a first pass 144 -> 128)
     # (on the host by name: only host memory can be pinned, and the caller's default device may be another)
     bad = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)
-    packed = native.pack_layer(weight.contiguous(), None if scale is None else scale.contiguous(),
-                               None if zero is None else zero.contiguous(), nbits, bad)
-    torch.cuda.current_stream().synchronize()                   # the one wait for the device, behind the packing launch
+    # on the tensors' own device, which need not be the current one: its stream has filled them
+    with torch.cuda.device(weight.device):
+        packed = native.pack_layer(weight.contiguous(), None if scale is None else scale.contiguous(),
+                                   None if zero is None else zero.contiguous(), nbits, bad)
+        torch.cuda.current_stream().synchronize()               # the one wait for the device, behind the packing launch
     assert bad.item() == 0, "values outside [0, 2^NBITS)"
     return packed
 

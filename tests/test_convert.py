@@ -108,3 +108,30 @@ def test_large_layer_is_fast_enough():
     t = time.perf_counter()
     convert_params({"K": K, "N": N, "NBITS": 4, "GS": 128}, (weight, scale, zero))
     assert time.perf_counter() - t < 20.0
+
+
+def test_device_tensors_are_packed_on_their_own_device(monkeypatch):
+    """The packing launch and the wait behind it belong to the tensors' device (whose stream has filled them), not to
+    whichever device is current: checked with the device calls replaced by a record of them."""
+    import contextlib
+    from qfactory import convert, native
+    seen, current = [], ["another device"]
+
+    @contextlib.contextmanager
+    def device(d):
+        saved, current[0] = current[0], str(d)
+        yield
+        current[0] = saved
+
+    class Stream:
+        def synchronize(self):
+            seen.append(("wait", current[0]))
+
+    real_zeros = torch.zeros
+    monkeypatch.setattr(torch, "zeros", lambda *a, pin_memory=False, **k: real_zeros(*a, **k))
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Stream())
+    monkeypatch.setattr(native, "pack_layer", lambda *a: seen.append(("launch", current[0])) or ("w", "s", "z"))
+    weight, scale, zero = _problem(4, 256, 4, 4, 128)
+    assert convert._pack_layer(weight, scale, zero, 4) == ("w", "s", "z")
+    assert seen == [("launch", str(weight.device)), ("wait", str(weight.device))]
