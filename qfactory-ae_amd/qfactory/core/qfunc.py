@@ -322,12 +322,7 @@ class QMatmulQFunc(QFunc):
             if low is not None and t == tiling.gemm_wide_tiling(p["M"], p["N"], p["K"], p["NBITS"], p["GS"]):
                 cfg += (f";\nusing CfgLow = {tiling.gemm_wide_cfg_string(p, low)};\n"
                         "static int gemm_by_rows(const void* a, const void* w, void* c, const void* s, const void* z, int m, hipStream_t stream) {\n"
-                        "\t// the LDS limit of both kernels is raised by the first launch of either: a later one may come under graph capture\n"
-                        "\tstatic std::atomic<bool> ready{false};\n"
-                        "\tif (!ready.load(std::memory_order_acquire)) {\n"
-                        "\t\tif (hipFuncSetAttribute(reinterpret_cast<const void*>(&qf::gemm_wide_kernel<CfgLow>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)CfgLow::LDS_BYTES) != hipSuccess) return 2;\n"
-                        "\t\tready.store(true, std::memory_order_release);\n\t}\n"
-                        f"\treturn m <= {3 * p['M'] // 4} ? qf::gemm_wide_launch<CfgLow>(a, w, c, s, z, m, stream) : qf::gemm_wide_launch<Cfg>(a, w, c, s, z, m, stream);\n}}\n")
+                        f"\treturn qf::gemm_wide_launch_by_rows<CfgLow, Cfg>(a, w, c, s, z, m, {3 * p['M'] // 4}, stream);\n}}\n")
                 call = "gemm_by_rows"
         elif self.regime == "gemm":
             code += '#include "qf_gemm.hip.h"\n'

@@ -513,6 +513,21 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
     }
 }
 
+// Raises the kernel's limit of LDS, once per object (re-entrant: the call is idempotent, the flag only saves repeats).
+template <class C>
+int gemm_wide_reserve() {
+    static std::atomic<bool> reserved{false};
+    if (C::LDS_BYTES <= 64 * 1024 || reserved.load(std::memory_order_acquire)) return 0;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<C>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS_BYTES);
+    if (e != hipSuccess) {
+        fprintf(stderr, "qfactory gemm: cannot reserve %zu bytes of LDS: %s\n", (size_t)C::LDS_BYTES, hipGetErrorString(e));
+        return 2;
+    }
+    reserved.store(true, std::memory_order_release);
+    return 0;
+}
+
 template <class C>
 int gemm_wide_launch(const void* A, const void* W, void* Cout, const void* S, const void* Zp, int m, hipStream_t stream) {
     const char* why = nullptr;
@@ -538,16 +553,7 @@ int gemm_wide_launch(const void* A, const void* W, void* Cout, const void* S, co
         return 1;
     }
     if (m <= 0) return 0;
-    static std::atomic<bool> attr_set{false};        // launch is re-entrant: the attribute call is idempotent, the flag only saves repeats
-    if (C::LDS_BYTES > 64 * 1024 && !attr_set.load(std::memory_order_acquire)) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_wide_kernel<C>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS_BYTES);
-        if (e != hipSuccess) {
-            fprintf(stderr, "qfactory gemm: cannot reserve %zu bytes of LDS: %s\n", C::LDS_BYTES, hipGetErrorString(e));
-            return 2;
-        }
-        attr_set.store(true, std::memory_order_release);
-    }
+    if (int rc = gemm_wide_reserve<C>()) return rc;
     dim3 grid(C::GRID_X, (m + C::BM - 1) / C::BM);
     hipLaunchKernelGGL(gemm_wide_kernel<C>, grid, dim3(C::T), C::LDS_BYTES, stream, (const uint16_t*)A, (const uint8_t*)W,
                        (uint16_t*)Cout, (const uint16_t*)S, (const uint8_t*)Zp, m);
@@ -557,6 +563,17 @@ int gemm_wide_launch(const void* A, const void* W, void* Cout, const void* S, co
         return 2;
     }
     return 0;
+}
+
+// Two tilings of one problem: Low for launches of at most low_rows rows, C for the others.  The first launch, whatever its
+// rows, raises the LDS limit of both kernels: a later one may come under graph capture.
+template <class Low, class C>
+int gemm_wide_launch_by_rows(const void* A, const void* W, void* Cout, const void* S, const void* Zp, int m, int low_rows,
+                             hipStream_t stream) {
+    if (m <= 0) return 0;
+    if (int rc = gemm_wide_reserve<Low>()) return rc;
+    if (int rc = gemm_wide_reserve<C>()) return rc;
+    return m <= low_rows ? gemm_wide_launch<Low>(A, W, Cout, S, Zp, m, stream) : gemm_wide_launch<C>(A, W, Cout, S, Zp, m, stream);
 }
 
 }  // namespace qf

@@ -14,3 +14,37 @@ def test_the_rule_gives_a_tiling_the_kernel_takes():
                         assert tiling.gemm_wide_lds_bytes(t, nbits) <= 160 * 1024
                     if nbits == 3 or K % (1024 // nbits):
                         assert t is None
+
+
+HIP_CALLS = r"""
+#include <stddef.h>
+#include <stdio.h>
+typedef struct { unsigned x, y, z; } dim3_;
+int hipFuncSetAttribute(const void* f, int attr, int value) { (void)f; printf("attribute %d %d\n", attr, value); fflush(stdout); return 0; }
+int __hipPushCallConfiguration(dim3_ g, dim3_ b, size_t lds, void* s) { (void)g; (void)b; (void)s; printf("launch %zu\n", lds); fflush(stdout); return 1; }
+int hipGetLastError(void) { return 0; }
+"""
+
+
+def test_the_first_launch_of_a_two_tiling_object_raises_both_lds_limits(tmp_path):
+    """Whichever tiling the first launch takes, no later launch (which may come under graph capture) has an attribute
+    left to set.  The object's HIP calls go to stand-ins that print what they are asked for."""
+    import os
+    import subprocess
+    import sys
+    import prebuild
+    from qfactory.core import tiling
+    from qfactory.jit import jit
+    (qfunc,) = prebuild.qfuncs_of(prebuild._case(256, 12288, 1024))
+    sizes = [tiling.gemm_wide_lds_bytes(t, 4) for t in (tiling.gemm_wide_low_tiling(256, 12288, 1024, 4, 128), qfunc.tiling_configs)]
+    assert sizes[0] != sizes[1] and min(sizes) > 64 * 1024
+    (tmp_path / "calls.c").write_text(HIP_CALLS)
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "calls.c"), "-o", str(tmp_path / "calls.so")], check=True)
+    obj = os.path.join(jit.compile(qfunc).path, "kernel.so")
+    probe = ("import ctypes; launch = ctypes.CDLL(%r).launch_m; rc = ctypes.c_int(-1)\n"
+             "for m in %r:\n launch(m, None, None, None, None, None, None, ctypes.byref(rc))\n assert rc.value == 0, rc.value\n")
+    for rows in ((1, 256, 192, 193), (256, 1, 193, 192)):
+        out = subprocess.run([sys.executable, "-c", probe % (obj, rows)], env=dict(os.environ, LD_PRELOAD=str(tmp_path / "calls.so")),
+                             check=True, capture_output=True, text=True, timeout=120).stdout.splitlines()
+        assert sorted(int(line.split()[2]) for line in out[:2] if line.startswith("attribute")) == sorted(sizes), out
+        assert out[2:] == [f"launch {sizes[0] if m <= 192 else sizes[1]}" for m in rows], out
