@@ -21,6 +21,50 @@ int fail(const char* fn, const char* why) {
     return 1;
 }
 
+// One wave's 32 queries, key by key: two lanes (kb = 0, 1) per query, each with half of the dims.
+template <int HD>
+__device__ __forceinline__ void attend_by_key(const f16* q_row, const f16* k_rows, const f16* v_rows, f16* dst, int kb, bool have,
+                                              int my_pos, int last, float scale_log2) {
+    constexpr int UNITS = HD / 16;                                          // eight dims each
+    f16x8 qh[UNITS];
+    float o[HD / 2], m = -INFINITY, l = 0.0f;
+#pragma unroll
+    for (int u = 0; u < UNITS; u++) qh[u] = *reinterpret_cast<const f16x8*>(q_row + kb * (HD / 2) + 8 * u);
+#pragma unroll
+    for (int d = 0; d < HD / 2; d++) o[d] = 0.0f;
+#pragma unroll 1
+    for (int key = 0; key <= last; key++) {
+        const size_t at = (size_t)key * HD + kb * (HD / 2);
+        float score = 0.0f;
+#pragma unroll
+        for (int u = 0; u < UNITS; u++) {
+            const f16x8 kh = *reinterpret_cast<const f16x8*>(k_rows + at + 8 * u);
+#pragma unroll
+            for (int e = 0; e < 8; e++) score += (float)qh[u][e] * (float)kh[e];
+        }
+        score = (score + __shfl_xor(score, 32, 64)) * scale_log2;
+        if (key > my_pos) continue;
+        const float m_new = fmaxf(m, score), base = m_new == -INFINITY ? 0.0f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m - base), p = __builtin_amdgcn_exp2f(score - base);
+        m = m_new;
+        l = l * alpha + p;
+#pragma unroll
+        for (int u = 0; u < UNITS; u++) {
+            const f16x8 vh = *reinterpret_cast<const f16x8*>(v_rows + at + 8 * u);
+#pragma unroll
+            for (int e = 0; e < 8; e++) o[8 * u + e] = o[8 * u + e] * alpha + p * (float)vh[e];
+        }
+    }
+    if (!have) return;
+#pragma unroll
+    for (int u = 0; u < UNITS; u++) {
+        f16x8 r;
+#pragma unroll
+        for (int e = 0; e < 8; e++) r[e] = (f16)(o[8 * u + e] / l);
+        *reinterpret_cast<f16x8*>(dst + kb * (HD / 2) + 8 * u) = r;
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // One block: 128 query rows of one (sequence, head), four waves of 32, over key tiles of 64 positions; on the matrix
 // cores (v_mfma_f32_32x32x16_f16), scores, running maximum and sums in fp32.
@@ -29,8 +73,12 @@ int fail(const char* fn, const char* why) {
 //     partner lane ^ 32 has the other sixteen), so the softmax is arithmetic inside a lane and one exchange, and
 //     the probabilities already are the B operand of O^T += V^T P^T -- the contraction order of an MFMA is free, the
 //     fragments of V^T are read to match: keys 16 s + 4 kb .. + 3 and 16 s + 8 + 4 kb .. + 3.  No probability moves between lanes.
-//   * Probabilities enter the second product as fp16(p) + fp16(p - fp16(p)), twenty-two bits: the product costs twice
-//     the MFMAs, which are idle otherwise.
+//   * Probabilities enter the second product as fp16(p) + fp16(p - fp16(p)), off by at most max(2^-22 p, 2^-25) (the second
+//     half is subnormal below p = 1/4): the product costs twice the MFMAs, which are idle otherwise.
+//   * A key that a query must not see has probability 0, but 0 times an infinity or NaN in its V still reaches the sum.  A
+//     wave with a sum that is not finite (finite values cannot overflow fp32 here) goes through its keys once more, key by
+//     key, and leaves out what a query does not see.  The look at the sums costs 0 - 1.5 % (8 x 128 positions 11.2 -> 11.4 us);
+//     a look at every V on its way to LDS cost 9 - 17 %, a second pass of the block that shares the registers 3 - 15 %.
 //   * K tiles go to LDS as rows, V tiles turned to [dim][key] in 4 x 4 pieces on the way (registers); the next tile is
 //     loaded while this one is used.
 //
@@ -181,9 +229,18 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(
             }
         }
     }
+    f16* dst = out + (((size_t)b * tokens + row) * heads + h) * HD;
+    float look = 0.0f;                                                      // NaN where a sum is not finite
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) look = __builtin_fmaf(o[d][v], 0.0f, look);
+    if (__builtin_expect(__any(have && look != 0.0f), 0)) {
+        attend_by_key<HD>(q_row, k_cache + head * HD, v_cache + head * HD, dst, kb, have, my_pos, last, scale_log2);
+        return;
+    }
     if (!have) return;
     const float inv = 1.0f / (l + __shfl_xor(l, 32, 64));
-    f16* dst = out + (((size_t)b * tokens + row) * heads + h) * HD;
 #pragma unroll
     for (int d = 0; d < DT; d++)
 #pragma unroll

@@ -35,6 +35,39 @@ def test_prefill_attention(hd, B, T, H, max_len, first):
     assert torch.equal(out, again)
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("T,max_len,first", [(70, 256, 0), (129, 200, 3), (33, 100, 60)])
+def test_rows_behind_a_position_never_reach_it(hd, T, max_len, first):
+    """Unwritten cache rows (NaN and infinities behind the last position, in the prompt's last key tile and past it) leave
+    no trace; an infinite or NaN V inside the prompt reaches the tokens from its position on, as it should, and none before."""
+    from qfactory import native
+    print(f"[case] hd{hd} T{T} max_len{max_len} first{first}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T)
+    B, H = 2, 2
+    q = torch.randn(B, T, H, hd, device="cuda", generator=g).half()
+    k, v = (torch.randn(B, H, max_len, hd, device="cuda", generator=g).half() for _ in range(2))
+    pos = torch.arange(first, first + T, device="cuda")
+    ref = _reference(q, k, v, pos)
+    for cache in (k, v):
+        cache[:, :, first + T:] = float("nan")
+        cache[:, :, first + T::3] = float("inf")
+    out = native.prefill_attention(q, k, v, pos, torch.empty_like(q))
+    assert (out.double().cpu() - ref).norm() / ref.norm() <= 4e-4
+    dims = {0: float("inf"), 5: float("-inf"), hd - 1: float("nan")}
+    at = first + T // 2
+    for d, value in dims.items():
+        v[1, 0, at, d] = value
+    odd = native.prefill_attention(q, k, v, pos, torch.empty_like(q)).double().cpu()
+    want = ref.clone()
+    for d, value in dims.items():
+        want[1, T // 2:, 0, d] = value
+        assert torch.equal(odd[..., d][~want[..., d].isfinite()].nan_to_num(nan=-1.0),
+                           want[..., d][~want[..., d].isfinite()].nan_to_num(nan=-1.0))
+    seen = want.isfinite()
+    assert odd[seen].isfinite().all()
+    assert (odd[seen] - ref[seen]).norm() / ref[seen].norm() <= 4e-4
+
+
 def test_positions_in_any_order():
     from qfactory import native
     g = torch.Generator(device="cuda").manual_seed(5)
