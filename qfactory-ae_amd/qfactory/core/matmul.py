@@ -164,7 +164,13 @@ class QMatmul:
         predefined = _load_predefined(shape)
         if predefined is not None:
             logger.info(f"[Profile] Using predefined config for {shape}")
-            self.qfuncs = [apply_config(self.qfuncs[0], predefined)]
+            stored = apply_config(self.qfuncs[0].clone(), predefined)
+            if self.output_epilogue == "silu_mul" and stored.regime == "gemm" and not stored.pairs_whole():
+                # the entry was stored for the plain projection (the key names no epilogue): its kernel would refuse the
+                # launch, the default tiling's takes it
+                logger.info(f"[Profile] The predefined config for {shape} does not take the SwiGLU epilogue")
+            else:
+                self.qfuncs = [stored]
         else:
             if enable_transform:
                 self.qfuncs = list(chain.from_iterable(q.transform() for q in self.qfuncs))

@@ -173,6 +173,12 @@ class QMatmulQFunc(QFunc):
             ("stream", torch.cuda.streams.Stream),
         ]
 
+    def pairs_whole(self):
+        """Does every wave of this GEMM tiling hold whole (gate, up) pairs, as the SwiGLU epilogue needs?  The pipelined
+        kernel clamps by pairs and stores four at a time; the other one takes whole tiles of a wave."""
+        n = self.problem["N"]
+        return n % (8 if "WM" in self.tiling_configs else 32 * self.tiling_configs["NT32"]) == 0
+
     # -- search space -------------------------------------------------------------------------
     def decode_strategies(self):
         """Decode strategies this problem's kernel family implements, its default first.

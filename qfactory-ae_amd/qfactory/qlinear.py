@@ -146,8 +146,9 @@ class GPTQLinear(torch.nn.Module):
 
     def fuses_silu_mul(self, m, dtype=torch.float16):
         """Does ``forward_silu_mul`` on ``m`` rows run as one launch?  Where the dot2 GEMV kernel serves and its
-        rows come in pairs, or the A-stationary kernel and gate and up are whole 16-row tiles, or the GEMM kernel
-        and every wave holds whole (gate, up) pairs of its own (N a multiple of the wave's weight rows)."""
+        rows come in pairs, or the A-stationary kernel and gate and up are whole 16-row tiles, or a GEMM kernel and
+        every wave holds whole (gate, up) pairs of its own (N a multiple of eight; of the wave's weight rows where
+        the pipelined kernel does not serve)."""
         bucket = _m_bucket(m)
         if dtype != torch.float16 or self.out_features % 2:
             return False

@@ -25,6 +25,23 @@ def test_config_round_trip_selects_the_stored_tiling(tmp_path, monkeypatch):
     assert "WN=1" in func.runtime.description and "STEPS=2" in func.runtime.description
 
 
+def test_stored_tiling_that_cannot_pair_columns_gives_way_to_the_default(tmp_path, monkeypatch):
+    """An entry stored for a layer's plain projection is looked up for its SwiGLU form too.  Where the stored kernel takes
+    whole wave tiles only and N is not one (the default takes any multiple of eight), the default serves the SwiGLU form."""
+    from qfactory import tune
+    from qfactory.core import QMatmul, tiling
+    old = {"BM": 64, "NT32": 1, "WN": 2, "WK": 1, "PA": 3}
+    path = tmp_path / "best_config.json"
+    for n in (200, 192):
+        tune.update_config(str(path), {tune.shape_key(4, 64, n, 1024, 128): {"regime": "gemm", "tiling_configs": old}})
+    monkeypatch.setenv("QFACTORY_CONFIG", str(path))
+    for n, epilogue, stored in ((200, "none", True), (200, "silu_mul", False), (192, "silu_mul", True)):
+        op = QMatmul(64, n, 1024, 4, False, torch.float16, torch.int8, 128, output_epilogue=epilogue)
+        op.compile_profile()
+        want = old if stored else tiling.gemm_wide_tiling(64, n, 1024, 4, 128)
+        assert op.best_qfunc.tiling_configs == want and op.best_qfunc.output_epilogue == epilogue
+
+
 @pytest.mark.gpu
 def test_search_on_device_and_latency_harness(tmp_path):
     from qfactory import testing, tune
