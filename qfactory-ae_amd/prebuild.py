@@ -343,8 +343,9 @@ def wide_cases():
 
 
 def search_cases():
-    """Problems whose whole tiling search space is compiled (tests/test_tune.py searches on the device)."""
-    return [_case(1, 64, 256, 4, 128)]
+    """Problems whose whole tiling search space is compiled (tests/test_tune.py and tests/test_gemm_wide_gpu.py search and
+    check it on the device)."""
+    return [_case(1, 64, 256, 4, 128), _case(64, 100, 1280, 4, 64)]
 
 
 def drain_cases(base=None):

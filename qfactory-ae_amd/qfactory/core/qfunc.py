@@ -202,6 +202,8 @@ class QMatmulQFunc(QFunc):
 
     def schedule(self) -> List[QFunc]:
         smem = (False, True) if self.regime == "gemv" and self.output_epilogue == "none" else (False,)
+        if self.regime == "gemm" and "WM" in self.tiling_configs:
+            return [self.clone(l2cache_a=True, l2cache_b=False)]         # its loads go straight to LDS, in one form
         return [self.clone(l2cache_a=True, l2cache_b=b, smem_quant=s) for b in (False, True) for s in smem]
 
     def lower(self) -> List[QFunc]:
@@ -213,10 +215,12 @@ class QMatmulQFunc(QFunc):
         elif self.regime == "skinny":
             cands = tiling.skinny_candidates(p["M"], p["N"], p["K"], p["NBITS"], p["GS"])
         elif self.regime == "gemm":
-            cands = tiling.gemm_candidates(p["M"], p["N"], p["K"], p["NBITS"], p["GS"])
+            shape = (p["M"], p["N"], p["K"], p["NBITS"], p["GS"])
+            cands = tiling.gemm_wide_candidates(*shape)
+            # where the pipelined kernel serves, its tilings and, to measure them against, the other kernel's default
+            cands = cands + [tiling.gemm_tiling(*shape)] if cands else tiling.gemm_candidates(*shape)
             default = self.default_tiling("gemm")
-            if default not in cands:
-                cands = [default] + cands
+            cands = [default] + [c for c in cands if c != default]
         else:
             cands = tiling.mfma_candidates(p["M"], p["N"], p["K"], p["NBITS"], p["GS"])
         return [self.clone(tiling_configs=c) for c in cands]

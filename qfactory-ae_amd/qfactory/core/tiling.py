@@ -863,7 +863,8 @@ def gemm_wide_lds_bytes(cfg, nbits):
 
 
 def gemm_wide_valid(cfg, K, nbits, group_size):
-    """Mirror of the static checks in gemm_wide_launch (qf_gemm_wide.hip.h)."""
+    """The static checks of gemm_wide_launch (qf_gemm_wide.hip.h) on everything but the packed tensors and the epilogue, and one
+    limit more: five iterations."""
     if nbits not in (2, 4, 8):
         return False
     supk = 1024 // nbits
@@ -875,8 +876,26 @@ def gemm_wide_valid(cfg, K, nbits, group_size):
         return False
     if (supk % group_size) if group_size < supk else (group_size % supk):
         return False
+    threads = 64 * cfg["WM"] * cfg["WN"] * cfg["WK"]
+    if threads > 1024 or cfg["MT"] * cfg["NT"] * (4 if threads > 512 else 2 if threads > 256 else 1) > 16:
+        return False                   # a block's threads; a wave's accumulators beside the other waves of its SIMD
     ngs = max(1, supk // group_size)
     return ngs <= 8 and ngs * nbits <= 32 and gemm_wide_lds_bytes(cfg, nbits) <= 160 * 1024
+
+
+def gemm_wide_candidates(M, N, K, nbits, group_size):
+    """Tilings of the pipelined kernel for an on-device search: every tile of ``GEMM_WIDE_COST`` of less than twice the rows,
+    one and two steps per iteration, one to four groups along K, one wave per SIMD where a wave holds eight tiles or more
+    (two waves of that size spill and measured 8 - 50 % slower)."""
+    out = []
+    for wm, wn, mt, nt, _, _ in GEMM_WIDE_COST:
+        for ki in (2, 1):
+            for wk in (1, 2, 4):
+                cfg = {"BM": 32 * mt * wm, "WM": wm, "WN": wn, "MT": mt, "NT": nt, "KI": ki, "WK": wk, "PA": 3}
+                crowded = mt * nt >= 8 and wm * wn * wk > 4
+                if M >= GEMM_WIDE_MIN_M and cfg["BM"] < 2 * M and not crowded and gemm_wide_valid(cfg, K, nbits, group_size):
+                    out.append(cfg)
+    return out
 
 
 def gemm_wide_tiling(M, N, K, nbits, group_size):

@@ -55,6 +55,26 @@ def test_tilings_at_their_edges(oracle, case):
         assert torch.equal(first[:rows], store[:rows]) and store[rows:].isnan().all()
 
 
+def test_every_tiling_of_a_search(oracle):
+    """All candidates of a search on a ragged problem (windows of K that do not deal evenly over the groups among them)
+    against the oracle: a search may pick any."""
+    from qfactory import QLinear
+    from qfactory.jit import jit
+    case = prebuild.search_cases()[1]
+    M, N, K, nbits, GS = (case[k] for k in ("M", "N", "K", "NBITS", "GS"))
+    rows = M - 3
+    A, weight, scale, zero = make_problem(91, rows, N, K, nbits, GS)
+    layer = QLinear.init(1, K, N, nbits, weight.cuda(), GS, scale.cuda(), zero.cuda(), compile_flags=NO_SEARCH)
+    ref = reference_output(oracle, A, layer.w, layer.s, layer.z, nbits, GS)
+    x = A.cuda()
+    (qfunc,) = prebuild.qfuncs_of(case)
+    for cand in qfunc.lower():
+        print(f"[case] {cand.tiling_configs}", flush=True)
+        out = torch.full((rows, N), float("nan"), dtype=torch.float16, device="cuda")
+        _launch(jit.compile(cand), x, layer, out)
+        assert_close(oracle, out.cpu().numpy(), ref, str(cand.tiling_configs))
+
+
 @pytest.mark.parametrize("rows", [129, 192, 193, 256])
 def test_both_tilings_of_a_row_count_bucket(oracle, rows):
     """The object of the 256-row bucket holds a tiling for launches of at most 192 rows and one for the others."""

@@ -1,4 +1,5 @@
 """The rule that picks a tiling of the pipelined GEMM kernel: host logic, no GPU."""
+import pytest
 
 
 def test_the_rule_gives_a_tiling_the_kernel_takes():
@@ -14,6 +15,40 @@ def test_the_rule_gives_a_tiling_the_kernel_takes():
                         assert tiling.gemm_wide_lds_bytes(t, nbits) <= 160 * 1024
                     if nbits == 3 or K % (1024 // nbits):
                         assert t is None
+
+
+def _qfunc(M, N, K, nbits, gs):
+    import torch
+    from qfactory.core.qfunc import QMatmulQFunc
+    from qfactory.core.qtile import AsymQTile, QTile
+    return QMatmulQFunc(QTile((M, K), torch.float16, 16), AsymQTile((N, K), torch.int8, nbits, (1, gs)), "nt")
+
+
+@pytest.mark.parametrize("M,N,K,nbits,gs", [(32, 9280, 4608, 2, 128), (64, 22016, 4096, 4, 128), (256, 12288, 4096, 4, 128),
+                                           (512, 8192, 8192, 8, 128), (64, 4096, 1024, 4, 32)])
+def test_search_space_is_the_pipelined_kernels_where_it_serves(M, N, K, nbits, gs):
+    """``lower`` offers the default first, the tiles of the rule's table in their forms, and one tiling of the other GEMM
+    kernel to measure against; the schedule has nothing to add (the kernel has one load path)."""
+    from qfactory.core import tiling
+    q = _qfunc(M, N, K, nbits, gs)
+    cands = [c.tiling_configs for c in q.lower()]
+    wide = [t for t in cands if "WM" in t]
+    assert cands[0] == tiling.gemm_wide_tiling(M, N, K, nbits, gs) and len(wide) == len(cands) - 1 >= 8
+    assert cands[-1] == tiling.gemm_tiling(M, N, K, nbits, gs)
+    assert all(tiling.gemm_wide_valid(t, K, nbits, gs) and t["BM"] < 2 * M for t in wide)
+    assert len({tuple(sorted(t.items())) for t in cands}) == len(cands)
+    tiles = {tuple(t[k] for k in ("WM", "WN", "MT", "NT")) for t in wide}
+    assert tiles == {key[:4] for key in tiling.GEMM_WIDE_COST if 32 * key[0] * key[2] < 2 * M
+                     and any(tiling.gemm_wide_valid(dict(zip(("WM", "WN", "MT", "NT", "KI", "WK"), key[:4] + (ki, 1))), K, nbits, gs) for ki in (1, 2))}
+    assert [s.l2cache_b for s in q.schedule()] == [False]
+
+
+def test_search_space_of_the_other_gemm_kernel_is_as_it_was():
+    from qfactory.core import tiling
+    for shape in ((64, 4096, 4096, 3, 128), (64, 4096, 4224, 4, 32)):
+        q = _qfunc(*shape)
+        assert [c.tiling_configs for c in q.lower()] == tiling.gemm_candidates(*shape)
+        assert [s.l2cache_b for s in q.schedule()] == [False, True]
 
 
 HIP_CALLS = r"""

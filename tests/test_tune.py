@@ -50,3 +50,10 @@ def test_search_on_device_and_latency_harness(tmp_path):
     tq, td, ratio = testing.speedup_over_dense(1, 512, 1024)
     assert 0 < tq < 1e-3 and 0 < td < 1e-3 and ratio > 0
     assert testing.CuBLASLatencyTest is testing.DenseLatencyTest
+
+
+@pytest.mark.gpu
+def test_search_on_device_where_the_pipelined_gemm_kernel_serves():
+    from qfactory import tune
+    key, entry = tune.tune_shape(4, 64, 100, 1280, 64)
+    assert key == "4-64-100-1280-64" and entry["regime"] == "gemm" and "WM" in entry["tiling_configs"]
