@@ -95,9 +95,10 @@ def gemm_waits_hold(isa: str, pa: int):
     checked, exact = 0, True
     budget = [200000]
 
-    def min_loads(block, upto, waits_left):
+    def min_loads(block, upto, waits_left, walked=frozenset()):
         """Fewest loads issued on any path ending just before event index `upto` of `block`, going back over
-        `waits_left` waits; None if every such path crosses a full drain first."""
+        `waits_left` waits; None if every such path crosses a full drain first.  `walked`: whole blocks without a wait on
+        the way so far -- a path that comes round to one of them again issues no fewer loads than the path without the round."""
         budget[0] -= 1
         if budget[0] < 0:
             raise RuntimeError("control flow too tangled to enumerate")
@@ -116,8 +117,12 @@ def gemm_waits_hold(isa: str, pa: int):
         best = None
         if not preds[block]:
             return None                                               # the kernel's entry: nothing older is in flight
+        if upto == len(events) and "W" not in [ev[0] for ev in events]:
+            walked = walked | {(block, waits_left)}
         for p in preds[block]:
-            r = min_loads(p, len(blocks[p][0]), waits_left)
+            if (p, waits_left) in walked:
+                continue
+            r = min_loads(p, len(blocks[p][0]), waits_left, walked)
             if r is not None and (best is None or r < best):
                 best = r
         return None if best is None else count + best

@@ -103,6 +103,15 @@ def test_checker_rejects_a_missing_load():
     skipping = iteration * 2 + [load, "\ts_cbranch_vccnz .LBB0_3", load, ".LBB0_3:", load, "\ts_waitcnt vmcnt(3) lgkmcnt(0)"]
     assert not gemm_waits_hold(listing(skipping), 3)[0]
     assert not gemm_waits_hold("s_endpgm", 3)[0]                                    # no kernel, no counted wait
+    # a loop without a wait of its own between two waits (a load the compiler puts into one): at least one trip, and
+    # round and round again issues no fewer loads
+    looping = [load, ".LBB0_4:", load, "\ts_cbranch_execnz .LBB0_4", load, "\ts_waitcnt vmcnt(3) lgkmcnt(0)"]
+    assert gemm_waits_hold(listing(iteration * 2 + looping + iteration), 3) == (True, "3 counted waits hold on every path")
+    assert not gemm_waits_hold(listing(iteration * 2 + looping[1:] + iteration), 3)[0]
+    # a loop that holds a wait is walked round for the wait before it
+    waiting = [".LBB0_6:", load, load, load, "\ts_waitcnt vmcnt(6) lgkmcnt(0)", "\ts_cbranch_scc1 .LBB0_6"]
+    assert gemm_waits_hold(listing(iteration * 3 + waiting), 4)[0]
+    assert not gemm_waits_hold(listing(iteration * 3 + waiting[:2] + waiting[3:]), 4)[0]
 
 
 def test_jit_falls_back_to_a_full_drain_when_the_count_fails(tmp_path, monkeypatch):
