@@ -154,7 +154,9 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
     // the group's window w and its iteration `it` in the whole row; past the end the last ones
     auto window_of = [&](int w) { return min(w * C::WK + grp, C::NSUP - 1); };
     auto request_a = [&](int buf, int it, int part, int parts) {
-        const uint32_t at = ((uint32_t)window_of(it / SUP) * SUP + (uint32_t)(it % SUP)) * (128u * C::KI);
+        // the same for all lanes, and said so: where the compiler had formed it with vector instructions (short rows of K),
+        // every request became a loop over the values of the lanes
+        const uint32_t at = __builtin_amdgcn_readfirstlane(((uint32_t)window_of(it / SUP) * SUP + (uint32_t)(it % SUP)) * (128u * C::KI));
         uint8_t* dst = as_b + (size_t)buf * C::A_TILE;
 #pragma unroll
         for (int p = 0; p < C::UA; p++)
@@ -172,9 +174,10 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
     const buffer_rsrc w_rows = rows_from(W + (size_t)n_first * C::RB);
     auto request_w = [&](int slot, int sup, int part) {
         uint8_t* dst = ws_b + slot * C::W_TILE;
+        const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)sup * 128u);      // a scalar operand of the request, as in request_a
 #pragma unroll
         for (int p = 0; p < C::UW; p++)
-            if (part < 0 || p % C::PARTS == part) buffer_to_lds_16(w_rows, w_off[p], (uint32_t)sup * 128u, dst + min(p * WAVES + wave, C::WB - 1) * 1024);
+            if (part < 0 || p % C::PARTS == part) buffer_to_lds_16(w_rows, w_off[p], at, dst + min(p * WAVES + wave, C::WB - 1) * 1024);
     };
 
     // the first windows and tiles go out before anything else is computed

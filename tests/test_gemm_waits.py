@@ -85,6 +85,19 @@ def test_first_tile_is_read_before_its_buffer_is_requested_again(M, N, K, nbits,
     assert found is not None and found[0] >= sets and found[1] == 0, found
 
 
+@pytest.mark.parametrize("M,N,K,nbits,gs", [(256, 12288, 1024, 4, 128), (512, 4112, 1024, 4, 128), (64, 4096, 4096, 4, 128), (1024, 8192, 8192, 8, 128)])
+def test_every_request_is_one_instruction(M, N, K, nbits, gs, tmp_path):
+    """The wave-uniform offsets of the pipelined kernel's requests are scalar operands: the compiler puts a request whose
+    offset it holds in a vector register into a loop over the lanes' values."""
+    from qfactory.core.qfunc import QMatmulQFunc
+    from qfactory.core.qtile import AsymQTile, QTile
+    from qfactory.jit.verify import _blocks_of
+    q = QMatmulQFunc(QTile((M, K), torch.float16, 16), AsymQTile((N, K), torch.int8, nbits, (1, gs)), "nt")
+    assert "WM" in q.tiling_configs
+    kernels = [k for k in _isa_of(q, tmp_path).split(".Lfunc_end") if "buffer_load_dwordx4" in k]
+    assert kernels and not [name for k in kernels for name, (events, succ) in _blocks_of(k).items() if name in succ and events == ["L"]]
+
+
 def test_checker_rejects_a_missing_load():
     from qfactory.jit.verify import gemm_waits_hold
     load = "\tglobal_load_dwordx4 v[0:3], v4, s[0:1]"
