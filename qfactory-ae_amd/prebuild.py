@@ -234,6 +234,10 @@ def silu_mul_cases():
     cases += [_case(M, 22016, 4096) for M in (64, 128, 256, 512, 1024, 2048, 4096)]
     cases += [_case(64, 1024, 256, 4, 64), _case(100, 4128, 2048, 3, 64), _case(40, 160, 4096, 2, 128, True),
               _case(200, 2208, 2048, 8, 128), _case(33, 96, 1024, 4, 128)]
+    # the pipelined GEMM kernel on columns that are not whole wave tiles: stores of four elements (N / 2 a multiple of four
+    # only) and of eight, pairs clamped in the last 32-row tile, one to three weight tiles per wave
+    cases += [_case(64, 1032, 1024), _case(200, 2200, 2048, 8, 128), _case(300, 1000, 1024, 2, 128, True), _case(512, 4112, 1024),
+              _case(40, 24, 2048, 4, 64), _case(2048, 5768, 1024)]
     return [dict(c, epilogue="silu_mul") for c in cases]
 
 
@@ -325,8 +329,8 @@ def odd_wave_cases():
 
 
 def wide_cases():
-    """The pipelined GEMM kernel (tests/test_gemm_wide_gpu.py): every tiling of its table at ragged rows and columns,
-    pinned explicitly; windows of K that do not deal evenly over the groups, the fewest iterations, three window buffers
+    """The pipelined GEMM kernel (tests/test_gemm_wide_gpu.py): every tiling of its table, and the forms with fewer steps
+    and groups that the rule falls back to, at ragged rows and columns, pinned explicitly; windows of K that do not deal evenly over the groups, the fewest iterations, three window buffers
     (8 bits, two steps per iteration), one step per iteration, N that is not a multiple of four or eight, every bit
     width, groups from 32 elements to a whole window."""
     def tile(wm, wn, mt, nt, ki, wk):
@@ -339,7 +343,14 @@ def wide_cases():
         (65, 140, 1280, 4, 128, False, (1, 4, 2, 1, 2, 2)), (64, 104, 2816, 4, 64, False, (1, 3, 2, 1, 2, 2)),
         (50, 64, 2048, 2, 128, False, (1, 2, 2, 1, 2, 2)), (70, 132, 640, 8, 64, False, (1, 4, 2, 1, 1, 2)),
         (33, 72, 2816, 4, 128, False, (1, 2, 1, 1, 2, 4)), (40, 33, 3328, 4, 128, False, (1, 1, 1, 1, 2, 4)),
-        (34, 68, 1152, 8, 64, True, (1, 2, 1, 1, 1, 4))]] + [_case(256, 12288, 1024)]
+        (34, 68, 1152, 8, 64, True, (1, 2, 1, 1, 1, 4)),
+        # seven waves: the 1 KB blocks of an activation tile do not divide over them
+        (100, 230, 1280, 4, 128, False, (1, 7, 2, 1, 2, 1)), (33, 452, 2048, 2, 64, True, (1, 7, 1, 1, 2, 1)),
+        (45, 227, 1280, 8, 64, False, (1, 7, 1, 1, 1, 1)), (70, 450, 1024, 8, 128, True, (1, 7, 2, 1, 1, 1)),
+        # fewer steps per iteration and groups than the table's form
+        (70, 100, 1152, 8, 64, False, (1, 3, 2, 1, 1, 2)), (49, 72, 1408, 8, 64, True, (1, 2, 2, 1, 1, 2)),
+        (39, 40, 896, 8, 32, False, (1, 2, 1, 1, 1, 2)), (34, 36, 1152, 8, 64, False, (1, 1, 1, 1, 1, 4)),
+        (66, 130, 1280, 4, 128, False, (1, 4, 2, 1, 1, 1))]] + [_case(256, 12288, 1024)]
 
 
 def search_cases():
@@ -349,8 +360,8 @@ def search_cases():
 
 
 def drain_cases(base=None):
-    """One problem (the cheapest) per distinct GEMM tiling x bit width among the problems above: the GEMM kernel
-    with counted waits is compared bit for bit with its full-drain build (tests/test_gemm_drain_gpu.py)."""
+    """One problem (the cheapest) per distinct GEMM tiling (or pair of tilings, where an object holds two) x bit width
+    among the problems above: the GEMM kernel with counted waits is compared bit for bit with its full-drain build (tests/test_gemm_drain_gpu.py)."""
     best = {}
     for c in (base if base is not None else all_cases(with_drain=False)):
         if c.get("act") or c.get("smem_quant") or c.get("epilogue") or c.get("drain") or c["GS"] == -1:
@@ -358,7 +369,8 @@ def drain_cases(base=None):
         for q in qfuncs_of(c):
             if getattr(q, "regime", None) != "gemm":
                 continue
-            key = (tuple(sorted(q.tiling_configs.items())), c["NBITS"])
+            low = q.low_tiling()
+            key = (tuple(sorted(q.tiling_configs.items())), None if low is None else tuple(sorted(low.items())), c["NBITS"])
             cost = c["M"] * c["N"] * c["K"]
             if key not in best or cost < best[key][0]:
                 best[key] = (cost, c)

@@ -173,6 +173,15 @@ class QMatmulQFunc(QFunc):
             ("stream", torch.cuda.streams.Stream),
         ]
 
+    def low_tiling(self):
+        """The second tiling that a pipelined GEMM object of the default tiling holds for launches of at most 3/4 of its
+        rows, or None."""
+        p = self.problem
+        shape = (p["M"], p["N"], p["K"], p["NBITS"], p["GS"])
+        if self.regime != "gemm" or "WM" not in self.tiling_configs or self.tiling_configs != tiling.gemm_wide_tiling(*shape):
+            return None
+        return tiling.gemm_wide_low_tiling(*shape)
+
     def pairs_whole(self):
         """Does every wave of this GEMM tiling hold whole (gate, up) pairs, as the SwiGLU epilogue needs?  The pipelined
         kernel clamps by pairs and stores four at a time; the other one takes whole tiles of a wave."""
@@ -328,8 +337,8 @@ class QMatmulQFunc(QFunc):
             code += '#include "qf_gemm.hip.h"\n#include "qf_gemm_wide.hip.h"\n'
             cfg = tiling.gemm_wide_cfg_string(p, t)
             call = "qf::gemm_wide_launch<Cfg>"
-            low = tiling.gemm_wide_low_tiling(p["M"], p["N"], p["K"], p["NBITS"], p["GS"])
-            if low is not None and t == tiling.gemm_wide_tiling(p["M"], p["N"], p["K"], p["NBITS"], p["GS"]):
+            low = self.low_tiling()
+            if low is not None:
                 cfg += (f";\nusing CfgLow = {tiling.gemm_wide_cfg_string(p, low)};\n"
                         "static int gemm_by_rows(const void* a, const void* w, void* c, const void* s, const void* z, int m, hipStream_t stream) {\n"
                         f"\treturn qf::gemm_wide_launch_by_rows<CfgLow, Cfg>(a, w, c, s, z, m, {3 * p['M'] // 4}, stream);\n}}\n")

@@ -5,7 +5,7 @@ import pytest
 def test_the_rule_gives_a_tiling_the_kernel_takes():
     """Every problem the rule accepts passes the host-side mirror of the kernel's own checks."""
     from qfactory.core import tiling
-    for M in (33, 64, 100, 128, 256, 512, 1024, 4096):
+    for M in (17, 32, 33, 64, 100, 128, 256, 512, 1024, 4096):
         for N in (1, 64, 1000, 4096, 22016, 57344):
             for K in (256, 512, 896, 1024, 4096, 11008, 28672):
                 for nbits, gs in ((4, 128), (4, 32), (8, 128), (8, 32), (2, 64), (3, 128)):
@@ -15,6 +15,24 @@ def test_the_rule_gives_a_tiling_the_kernel_takes():
                         assert tiling.gemm_wide_lds_bytes(t, nbits) <= 160 * 1024
                     if nbits == 3 or K % (1024 // nbits):
                         assert t is None
+
+
+def test_where_the_rule_takes_over():
+    """From 17 rows on, at 2, 4 and 8 bits, on rows of whole 128-byte windows and five iterations: never None there, always None
+    elsewhere; the specialisation of such a problem is built on it."""
+    from qfactory.core import tiling
+    for N, K in ((12288, 4096), (4096, 11264), (8192, 28672), (77, 2560), (1, 5120)):
+        for nbits in (2, 4, 8):
+            assert tiling.gemm_wide_tiling(16, N, K, nbits, 128) is None
+            for M in (17, 32, 33, 64, 256, 4096):
+                assert tiling.gemm_wide_tiling(M, N, K, nbits, 128) is not None, (M, N, K, nbits)
+        assert tiling.gemm_wide_tiling(64, N, K, 3, 128) is None
+    for K, nbits, gs in ((11008, 2, 128), (4224, 4, 128), (8256, 8, 64), (768, 2, 128), (4096, 4, 16)):
+        assert tiling.gemm_wide_tiling(64, 4096, K, nbits, gs) is None, (K, nbits)
+    for M, N, K, nbits in ((32, 9280, 4608, 2), (64, 22016, 4096, 4), (1024, 8192, 8192, 8)):
+        q = _qfunc(M, N, K, nbits, 128)
+        assert q.regime == "gemm" and q.tiling_configs == tiling.gemm_wide_tiling(M, N, K, nbits, 128)
+        assert "qf::GemmWideCfg<" in q.emit()
 
 
 def _qfunc(M, N, K, nbits, gs):
