@@ -834,6 +834,8 @@ def gemm_candidates(M, N, K, nbits, group_size):
 # of blocks and 64 elements of K.  The figures are medians of a sweep of eighteen tilings over 22016 x 4096, 12288 x 4096,
 # 4096 x 4096, 4096 x 11008, 10240 x 8192, 8192 x 28672 and 57344 x 8192 at 32 ... 2048 rows (W4 g128, cold weights): with the
 # round model of gemm_wide_tiling they pick the fastest of the sweep on nearly all of its cells (up to 7 % off on the others).
+# At 8 bits (ten shapes at 24 ... 1024 rows, the forms of _gemm_wide_tiling) the same figures pick within 7 % of the fastest on 97 of
+# 104 cells, 8 - 16 % off on six, and 63 % off on one (2432 x 20480 at 96 rows, where two rounds of 32 x 32 tiles share CUs).
 GEMM_WIDE_COST = {
     (1, 4, 8, 2, 1, 1): 1.547,     # 256 x 256
     (2, 2, 4, 3, 1, 1): 1.289,     # 256 x 192
@@ -917,8 +919,12 @@ def _gemm_wide_tiling(M, N, K, nbits, group_size):
         if bm >= 2 * M:
             continue
         cfg = {"BM": bm, "WM": wm, "WN": wn, "MT": mt, "NT": nt, "KI": ki, "WK": wk, "PA": 3}
-        # 8 bits (three windows do not fit beside the tiles) and short rows: one step per iteration, fewer groups
-        for ki, wk in ((ki, wk), (1, wk), (1, -(-wk // 2)), (1, 1)):
+        # Where the form of the table does not fit.  8 bits (two steps per iteration take three window buffers): half the
+        # groups first -- two steps in half the groups against one step in all of them, ten shapes at 24 ... 512 rows: less
+        # time by 5 - 15 % wherever the rule has that choice (10240 x 8192 at 24 rows 32.1 -> 28.9 us, 4096 x 11008 at 128 39.1 -> 33.5, 23552 x 11776 at
+        # 64 98.0 -> 87.5).  Short rows: one step per iteration, fewer groups.
+        halved = ((ki, wk // 2),) if nbits == 8 and wk > 1 else ()
+        for ki, wk in ((ki, wk),) + halved + ((1, wk), (1, -(-wk // 2)), (1, 1)):
             cfg.update(KI=ki, WK=wk)
             if gemm_wide_valid(cfg, K, nbits, group_size):
                 break

@@ -29,6 +29,9 @@ def test_where_the_rule_takes_over():
         assert tiling.gemm_wide_tiling(64, N, K, 3, 128) is None
     for K, nbits, gs in ((11008, 2, 128), (4224, 4, 128), (8256, 8, 64), (768, 2, 128), (4096, 4, 16)):
         assert tiling.gemm_wide_tiling(64, 4096, K, nbits, gs) is None, (K, nbits)
+    # 8 bits, where the table's form does not fit in LDS: two steps per iteration in half the groups
+    assert [tiling.gemm_wide_tiling(M, N, 4096, 8, 128)[k] for M, N in ((32, 12288), (128, 12288)) for k in ("WN", "MT", "KI", "WK")] == \
+        [2, 1, 2, 2, 4, 2, 2, 1]
     for M, N, K, nbits in ((32, 9280, 4608, 2), (64, 22016, 4096, 4), (1024, 8192, 8192, 8)):
         q = _qfunc(M, N, K, nbits, 128)
         assert q.regime == "gemm" and q.tiling_configs == tiling.gemm_wide_tiling(M, N, K, nbits, 128)
