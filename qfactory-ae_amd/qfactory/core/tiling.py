@@ -853,6 +853,11 @@ GEMM_WIDE_COST = {
     (1, 1, 1, 1, 2, 4): 0.100,     # 32 x 32
 }
 GEMM_WIDE_MIN_M = 17           # the 32-row bucket: 9280 x 4608 at 2 bits 13.9 -> 11.6 us, 8192 x 28672 49.8 -> 46.3, 8192 x 8192 level
+# ... but not in more than one and up to two and a half rounds of blocks there: its blocks fill a CU's LDS, so a second round
+# starts when the first has ended, where the other kernel's smaller blocks share CUs.  Other kernel against this one, 24 rows:
+# 19008 x 14592 at 4 bits 54.9 against 65.4 us, 24576 x 4352 21.4 / 24.4, 23552 x 11776 at 8 bits 80.4 / 89.0; of random problems
+# at 17 - 32 rows 26 of 28 in that range took longer here (up to 21 %), four of five past 2.5 rounds 9 - 10 % less.
+GEMM_WIDE_NOT_AT_32 = (NUM_CUS, 2.5 * NUM_CUS)
 
 
 def gemm_wide_lds_bytes(cfg, nbits):
@@ -901,8 +906,8 @@ def gemm_wide_candidates(M, N, K, nbits, group_size):
 
 
 def gemm_wide_tiling(M, N, K, nbits, group_size):
-    """Tiling of the pipelined kernel for this problem, None where the kernel of gemm_tiling serves: up to 16 rows, 3 bits,
-    and K that is not whole 128-byte windows.  A launch costs its whole rounds of blocks (one block per CU), each 0.6 + 0.4 x the
+    """Tiling of the pipelined kernel for this problem, None where the kernel of gemm_tiling serves: up to 16 rows, up to 32
+    on some widths (GEMM_WIDE_NOT_AT_32), 3 bits, and K that is not whole 128-byte windows.  A launch costs its whole rounds of blocks (one block per CU), each 0.6 + 0.4 x the
     mean share of the CUs that get a block (a machine that is not full clocks higher and shares L2 among fewer); a block row taller than
     twice the rows is not considered."""
     cfg = _gemm_wide_tiling(M, N, K, nbits, group_size)
@@ -934,8 +939,10 @@ def _gemm_wide_tiling(M, N, K, nbits, group_size):
         whole = -(-exact // 1)
         cost = (0.6 * whole + 0.4 * exact) * per_step
         if best is None or cost < best[0]:
-            best = (cost, cfg)
-    return None if best is None else best[1]
+            best = (cost, cfg, exact * NUM_CUS)
+    if best is None or (M <= 32 and GEMM_WIDE_NOT_AT_32[0] < best[2] <= GEMM_WIDE_NOT_AT_32[1]):
+        return None
+    return best[1]
 
 
 GEMM_WIDE_LOW = (256, 4096)     # row-count buckets whose objects hold a second tiling

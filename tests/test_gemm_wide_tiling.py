@@ -29,6 +29,11 @@ def test_where_the_rule_takes_over():
         assert tiling.gemm_wide_tiling(64, N, K, 3, 128) is None
     for K, nbits, gs in ((11008, 2, 128), (4224, 4, 128), (8256, 8, 64), (768, 2, 128), (4096, 4, 16)):
         assert tiling.gemm_wide_tiling(64, 4096, K, nbits, gs) is None, (K, nbits)
+    # at 17 .. 32 rows: one round of blocks, or more than two and a half
+    for N, takes in ((16384, True), (16385, False), (19008, False), (40960, False), (40961, True)):
+        assert (tiling.gemm_wide_tiling(32, N, 4352, 4, 128) is not None) == takes, N
+        assert tiling.gemm_wide_tiling(33, N, 4352, 4, 128) is not None
+    assert _qfunc(32, 19008, 14592, 4, 128).tiling_configs == tiling.gemm_tiling(32, 19008, 14592, 4, 128)
     # 8 bits, where the table's form does not fit in LDS: two steps per iteration in half the groups
     assert [tiling.gemm_wide_tiling(M, N, 4096, 8, 128)[k] for M, N in ((32, 12288), (128, 12288)) for k in ("WN", "MT", "KI", "WK")] == \
         [2, 1, 2, 2, 4, 2, 2, 1]
