@@ -25,8 +25,8 @@ prefill row count) and `decode` (configs[4]: the Llama-2-7B-shaped decode loop a
 Other modes (each prints its own JSON and exits): `--counter-pass` and `--counter-pass-matrix` (a few eager
 launches of the GEMV kernels / of the matrix-core kernels beside a copy of known size, for `rocprofv3 --pmc`),
 `--shape-sets` (the reference's figure 6 / 9 / 10 and table 3 shape sets: achieved bandwidth and speed-up over the
-dense fp16 GEMM), `--launch-floor` (an empty kernel and a pure streaming read), `--ablation` (each kernel family
-beside timing builds of itself that leave one part out).
+dense fp16 GEMM), `--launch-floor` (an empty kernel and a pure streaming read), `--ablation` (the kernels
+of up to 16 rows beside timing builds of themselves that leave one part out).
 
 Every per-kernel timing rotates over at least 512 MB of distinct packed weights (twice the 256 MB
 Infinity Cache), so each launch streams its weights from HBM.
@@ -455,7 +455,7 @@ def small_m_report():
 
 
 def ablation_report():
-    """Where the time of a launch goes: per kernel family, the product's object beside timing builds of the same
+    """Where the time of a launch goes at 1 and 16 rows: the product's object beside timing builds of the same
     tiling that leave one part out (`prebuild.ABLATIONS`: the headers' `QF_*_EXPERIMENT` knobs; their results are wrong
     by design and nothing but this mode compiles them), and a pure streaming read of the same bytes.  Cold weights,
     timed like every other kernel here."""
@@ -751,8 +751,8 @@ def main():
                     help="the same for the matrix-core kernels: gate_up and down at M = 16, the four GEMMs at M = 256, qkv and "
                          "gate_up at 8192 rows")
     ap.add_argument("--ablation", action="store_true",
-                    help="only the phase ablation: each kernel family's object beside timing builds that leave one part "
-                         "out, on the 7B layers at M = 1 and 16 and three GEMM problems; prints one JSON object")
+                    help="only the phase ablation: the dot2 GEMV and A-stationary kernels' objects beside timing builds that leave "
+                         "one part out, on the 7B layers at M = 1 and 16; prints one JSON object")
     ap.add_argument("--shape-sets", action="store_true",
                     help="only the reference's bandwidth tables: its `squares` and `operator` shape sets at M in {1, 2, 4}, "
                          "8 / 4 / 2 bits, with and without groups; prints one JSON object, writes gpurun_out/shape_sets.json")

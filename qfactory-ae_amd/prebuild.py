@@ -441,7 +441,7 @@ class TimingBuild:
     """A specialisation compiled with its kernel header's timing knob set (``QF_*_EXPERIMENT``: parts of the kernel
     left out, results wrong by design), for ``bench.py --ablation`` only.  The code generator refuses these knobs;
     this wrapper writes them, and the define the headers ask for, in front of the generated translation unit."""
-    KNOBS = {"gemv": "QF_GEMV_EXPERIMENT", "mgemv": "QF_MGEMV_EXPERIMENT", "gemm": "QF_GEMM_EXPERIMENT"}
+    KNOBS = {"gemv": "QF_GEMV_EXPERIMENT", "mgemv": "QF_MGEMV_EXPERIMENT"}
 
     def __init__(self, qfunc, bits):
         assert bits != 0 and qfunc.regime in self.KNOBS
@@ -453,7 +453,7 @@ class TimingBuild:
         return getattr(self.qfunc, name)
 
     @property
-    def regime(self):                                 # not "gemm": the counted waits of a timing build are not re-counted
+    def regime(self):
         return self.qfunc.regime + "-timing"
 
     def emit(self):
@@ -469,12 +469,8 @@ ABLATIONS = {
               (16, "loads in their order, LDS hand-off + decode + MFMAs replaced by an XOR"),
               (48, "... and without scale / zero-point loads"), (8, "without the weight loads"),
               (1, "without the activation loads")],
-    "gemm": [(0, "kernel"), (1, "without dequantisation arithmetic"), (4, "without MFMAs"), (5, "without both"),
-             (72, "without activation tile requests and their wait"), (32, "without weight / scale / zero-point loads"),
-             (16, "without the block barrier of the K loop")],
 }
-ABLATION_PROBLEMS = ([(1, N, K) for N, K in LLAMA2_7B] + [(16, 22016, 4096), (16, 12288, 4096), (16, 4096, 11008), (16, 57344, 8192)]
-                     + [(256, 8192, 8192), (256, 57344, 8192), (8192, 4096, 4096)])
+ABLATION_PROBLEMS = ([(1, N, K) for N, K in LLAMA2_7B] + [(16, 22016, 4096), (16, 12288, 4096), (16, 4096, 11008), (16, 57344, 8192)])
 
 
 def ablation_builds(M, N, K):
@@ -486,10 +482,6 @@ def ablation_builds(M, N, K):
     op = QMatmul(_m_bucket(M), N, K, 4, False, torch.float16, torch.int8, 128)
     op.init_qfuncs()
     q = op.qfuncs[0]
-    if "WM" in q.tiling_configs:
-        # the timing knobs are those of qf_gemm.hip.h: the problem on that kernel
-        from qfactory.core import tiling
-        q = q.clone(tiling_configs=tiling.gemm_tiling(_m_bucket(M), N, K, 4, 128))
     return op, q.regime, [(bits, label, q if bits == 0 else TimingBuild(q, bits)) for bits, label in ABLATIONS[q.regime]]
 
 

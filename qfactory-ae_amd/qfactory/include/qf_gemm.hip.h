@@ -37,16 +37,6 @@
 #include <cstdio>
 #include "qf_dequant.hip.h"
 
-// Timing experiments (results are wrong when non-zero): bit 0 skips the dequantisation arithmetic,
-// bit 1 the activation fragment reads, bit 2 the MFMAs, bit 3 the activation tile requests, bit 4 the block
-// barrier of the K loop, bit 5 the global weight / scale / zero loads, bit 6 the wait for the activation tiles.
-#ifndef QF_GEMM_EXPERIMENT
-#define QF_GEMM_EXPERIMENT 0
-#endif
-#if QF_GEMM_EXPERIMENT != 0 && !defined(QF_ALLOW_TIMING_EXPERIMENTS)
-#error "QF_GEMM_EXPERIMENT gives wrong results: timing builds only (define QF_ALLOW_TIMING_EXPERIMENTS)"
-#endif
-
 // 1: the wait in front of the K loop's barrier drains every vector-memory load of the wave (vmcnt(0)) instead of
 // letting the counted younger loads stay in flight.  The counted wait is only right if the compiled code issues
 // exactly the loads `loads_since` counts, in order; the JIT checks that on the generated ISA of every object and
@@ -178,11 +168,11 @@ constexpr int waitcnt_imm(int vmcnt, int lgkmcnt) {
 // Wait until at most ALLOWED of this wave's vector-memory loads (in issue order) and none of its
 // LDS operations are outstanding, then meet the block's other waves.  A bare s_barrier: the
 // fence of __syncthreads() would wait for every outstanding load.
-template <int ALLOWED, bool BARRIER = true>
+template <int ALLOWED>
 __device__ __forceinline__ void wait_loads_and_barrier() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(waitcnt_imm(ALLOWED, 0));
-    if constexpr (BARRIER) __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 }
 
@@ -295,7 +285,6 @@ __global__ __launch_bounds__(C::T) void gemm_kernel(
     const uint8_t* a_slab = reinterpret_cast<const uint8_t*>(A + (size_t)m_blk * C::K);
     // tile `it` of the group into LDS buffer `buf`, asynchronously
     auto load_a = [&](int buf, int it) {
-        if (QF_GEMM_EXPERIMENT & 8) return;
         const uint8_t* base = a_slab + (size_t)k_of(it) * 2;
         uint8_t* dst = as_b + (size_t)buf * BM * C::ROWB;
 #pragma unroll
@@ -334,7 +323,6 @@ __global__ __launch_bounds__(C::T) void gemm_kernel(
     const uint8_t* z_rows = Zp + (size_t)n_base * C::ZRB;
     // instalment `part` of the super (part < 0: all of it)
     auto load_super = [&](WStage& st, int sup_local, int part) {
-        if (QF_GEMM_EXPERIMENT & 32) return;
         const int sup = min(sup_local * WK + grp, C::NSUP - 1);
         // byte offset of the super's window in the main plane (half of it in the 1-bit plane); wave-uniform, and
         // opaque: requests past the end clamp to the same window and must not be merged (see the end of the K loop)
@@ -358,7 +346,6 @@ __global__ __launch_bounds__(C::T) void gemm_kernel(
         }
     };
     auto load_quant = [&](Quant& qu, int sup_local) {
-        if (QF_GEMM_EXPERIMENT & 32) return;
         const int sup = min(sup_local * WK + grp, C::NSUP - 1);
         // first group of the super's window (a partial last super: the window ends at the last group); opaque, as in load_super
         int g0 = __builtin_amdgcn_readfirstlane(is_tail(sup_local) ? (C::K - C::SUPK) / C::GS : sup * C::SUPK / C::GS);
@@ -472,10 +459,7 @@ __global__ __launch_bounds__(C::T) void gemm_kernel(
 #pragma unroll
         for (int i = 0; i < MT32; i++)
 #pragma unroll
-            for (int ks = 0; ks < 4; ks++) {
-                if (QF_GEMM_EXPERIMENT & 2) fr.f[i][ks] = __builtin_bit_cast(f16x8, u32x4{(uint32_t)buf, 1u, 2u, 3u});
-                else fr.f[i][ks] = frag_of(buf, i, ks);
-            }
+            for (int ks = 0; ks < 4; ks++) fr.f[i][ks] = frag_of(buf, i, ks);
     };
 
     WStage ringW[2];            // packed words of the two supers after the one in LDS
@@ -516,15 +500,12 @@ __global__ __launch_bounds__(C::T) void gemm_kernel(
 #pragma unroll
                 for (int i = 0; i < MT32; i++) {
                     if constexpr (C::PREFETCH_A) af[i] = fcur.f[i][ks];
-                    else if (QF_GEMM_EXPERIMENT & 2) af[i] = __builtin_bit_cast(f16x8, u32x4{(uint32_t)b0, 1u, 2u, 3u});
                     else af[i] = frag_of(b0, i, ks);
                 }
 #pragma unroll
                 for (int j = 0; j < NT32; j++) {
                     const QConst qc = qconst_of(ringQ[pslot], j, q, tail);
-                    if constexpr ((QF_GEMM_EXPERIMENT & 1) != 0) {
-                        wf[j] = __builtin_bit_cast(f16x8, u32x4{cur.w[j][0], cur.w[j][1], cur.w[j][2], cur.w[j][3] + (uint32_t)ks});
-                    } else if constexpr (C::NBITS == 3) {
+                    if constexpr (C::NBITS == 3) {
                         const uint32_t w4[4] = {cur.w[j][0], cur.w[j][1], 0u, 0u};
                         wf[j] = ks == 0 ? DequantStep3::run<0>(w4, cur.h[j], qc) : ks == 1 ? DequantStep3::run<1>(w4, cur.h[j], qc)
                               : ks == 2 ? DequantStep3::run<2>(w4, cur.h[j], qc) : DequantStep3::run<3>(w4, cur.h[j], qc);
@@ -541,8 +522,7 @@ __global__ __launch_bounds__(C::T) void gemm_kernel(
                 for (int j = 0; j < NT32; j++)
 #pragma unroll
                     for (int i = 0; i < MT32; i++)
-                        if (QF_GEMM_EXPERIMENT & 4) acc[j][i][ks] += (float)wf[j][0] * (float)af[i][0];
-                        else acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[j], af[i], acc[j][i], 0, 0, 0);
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[j], af[i], acc[j][i], 0, 0, 0);
             }
         }
         if constexpr (C::PREFETCH_A) load_a(b0, min(it + C::PA, C::ITERS - 1));
@@ -563,7 +543,7 @@ __global__ __launch_bounds__(C::T) void gemm_kernel(
         // wave has issued in those iterations (activation tiles and whole supers) may stay in
         // flight.  Loads return in order; what the requesting iteration itself issued next to the
         // request is not counted, wherever the compiler placed it.
-        wait_loads_and_barrier<QF_GEMM_FULL_DRAIN ? 0 : ((QF_GEMM_EXPERIMENT & (8 | 64)) ? 63 : loads_since<C>(s, C::PA - 2)), !(QF_GEMM_EXPERIMENT & 16)>();
+        wait_loads_and_barrier<QF_GEMM_FULL_DRAIN ? 0 : loads_since<C>(s, C::PA - 2)>();
     };
 
     // ---- prologue: supers 0, 1 (with the early request: then 2) and activation tiles 0 .. PA-1 requested, all complete at the barrier ----

@@ -1,4 +1,4 @@
-// Dequant-fused low-bit GEMM on the gfx950 matrix cores, one software-pipelined wave per SIMD (M > 32).
+// Dequant-fused low-bit GEMM on the gfx950 matrix cores, one software-pipelined wave per SIMD (from 17 rows on).
 //
 //   C[m][n] = fp16( sum_k A[m][k] * DQ[n][k] ),   DQ[n][k] = fp16_rn((q[n][k] - Z[n][k/GS]) * s[n][k/GS])
 //
