@@ -692,7 +692,8 @@ def gemm_tuned(M, N, K, nbits, group_size):
     """The winner of the on-device sweep over ``gemm_candidates`` for this exact problem, where the sweep was run
     and beat the model below by 3 % or more (``gemm_tuned_gfx950.json`` beside this file: the reference times its
     candidates at every first construction, qfunc.py:110-131; here that was done once for the reference's own
-    shape list at M = 32 .. 256, W4 g128).  None for any other problem."""
+    shape list at M = 32 .. 256, W4 g128).  None for any other problem.  The pipelined kernel serves these problems by
+    default; a search there measures against this tiling."""
     global _GEMM_TUNED
     if _GEMM_TUNED is None:
         import json
