@@ -75,6 +75,13 @@ def test_add_rmsnorm_matches_torch(rows, hidden, with_delta):
     assert ((out.float() - want.float()).norm() / want.float().norm()).item() <= 2e-4
 
 
+@pytest.mark.parametrize("with_delta", [False, True])
+@pytest.mark.parametrize("rows,hidden", [(3, 2048), (3, 2056), (1, 4104), (512, 8192), (513, 8192), (512, 8200), (513, 8200), (513, 16384)])
+def test_add_rmsnorm_at_the_edges_of_its_block_sizes(rows, hidden, with_delta):
+    """One and several vectors per thread, rows that end inside a block's last vectors, few rows and many."""
+    test_add_rmsnorm_matches_torch(rows, hidden, with_delta)
+
+
 @pytest.mark.parametrize("B,H,hd,max_len,pos", [(1, 32, 128, 256, 0), (2, 4, 64, 32, 8), (16, 32, 128, 256, 200),
                                                 (3, 5, 32, 40, 39), (2, 2, 256, 300, 299), (40, 32, 64, 64, 50)])
 def test_rope_cache_append_and_attention_match_torch(B, H, hd, max_len, pos):
