@@ -165,17 +165,17 @@ __global__ __launch_bounds__(kThreads) void rope_kv_store_kernel(const f16* __re
 // store them), k and v are appended to the cache, and the new position is served from LDS rather than
 // re-read from memory the block has just written.
 // ---------------------------------------------------------------------------------------------
-// 8 waves per block and the first 8 positions of every group requested up front, at every batch size.  Measured with 32
-// heads of 128 at 130 / 191 / 250 cache positions, cold caches: 5.4 / 5.6 / 6.0 us at batch 1, 10.4 / 12.4 / 14.9 at
-// batch 16, 28.9 / 37.1 / 47.3 at batch 64 (there the kernel reads 200 MB of cache per launch and is HBM-bound).
-// Against it: 16 waves walking the cache two positions at a time 5.6 / 6.2 / 6.8 and 11.5 / 14.2 / 16.7 at batch 1 and 16;
+// 8 waves per block and up to the first 8 positions of every group requested up front, at every batch size.  Measured with
+// 8 of them always, 32 heads of 128 at 130 / 191 / 250 cache positions, cold caches: 5.4 / 5.6 / 6.0 us at batch 1, 10.4 / 12.4 /
+// 14.9 at batch 16, 28.9 / 37.1 / 47.3 at batch 64 (there the kernel reads 200 MB of cache per launch and is HBM-bound).
+// Against that: 16 waves walking the cache two positions at a time 5.6 / 6.2 / 6.8 and 11.5 / 14.2 / 16.7 at batch 1 and 16;
 // 4 waves per block and one pass with a running maximum (the variant that served 1024 pairs and more) 8.7 / 10.8 /
 // 13.7 at batch 4, 11.8 / 14.9 / 18.0 at batch 16, 30.8 / 41.9 / 52.8 at batch 64, and 5 - 7 % behind at 500 and 900
 // positions too.  Every wave repeats the rotation of q and the merge steps, so more waves cost vector issue; a launch
 // costs 4.0 us before it touches the cache (the position, then the new token's q / k / v, then the stores: three
 // dependent round trips behind a 1.7 us launch).
 constexpr int kAttnThreads = 512;
-constexpr int kAttnPrefetch = 8;          // positions per group requested up front (256 at 128-wide heads)
+constexpr int kAttnPrefetch = 8;          // positions per group requested up front at most (256 at 128-wide heads)
 
 __device__ __forceinline__ f16x8 rotate8(const f16x8 x, const float* __restrict__ c, const float* __restrict__ s) {
 #pragma clang fp contract(off)                                // same roundings as rope_kv_store_kernel
@@ -225,12 +225,15 @@ __global__ __launch_bounds__(kThreads) void rope_kv_store_rows_kernel(const f16*
     *reinterpret_cast<f16x8*>(v_cache + cache_off) = v;
 }
 
-// PRE: how many of a group's first positions are requested before anything else -- before the position itself is
-// known (rows are clamped to the cache; what lies past the sequence is fetched and never used) and before q has
-// been rotated -- so that the cache rows, the position and the new token's q / k / v travel together instead of one
-// after the other.  For the few-blocks variant only: with many blocks the rows past a short sequence would cost
-// real bandwidth.
-template <int LPK, bool FUSED, int THREADS, int PRE>
+template <int V> struct Tag { static constexpr int value = V; };
+
+// PRE: how many positions of a group are requested before anything is computed -- before the new token's q has been
+// rotated -- so that the cache rows and the new token's q / k / v travel together instead of one after the other.  The kernel
+// takes as many as the sequence has (its position is known on the device only, so all forms are in the one kernel): stages
+// past the end cost requests, registers and arithmetic, and only the last stage has to look for the end of the sequence.
+// 32 heads of 128, cold caches, against eight stages for every sequence: 190 positions at batch 1 / 16 / 64 4.85 / 11.8 / 36.0
+// -> 4.24 / 11.3 / 35.7 us, 60 positions at batch 96 26.6 -> 19.4; past 256 positions level.
+template <int LPK, bool FUSED, int THREADS, int MOST>
 __global__ __launch_bounds__(THREADS) void decode_attention_kernel(const f16* __restrict__ q_or_qkv, f16* __restrict__ k_cache,
                                                                         f16* __restrict__ v_cache, const int64_t* __restrict__ pos_ptr,
                                                                         const float* __restrict__ cos_t, const float* __restrict__ sin_t,
@@ -249,137 +252,151 @@ __global__ __launch_bounds__(THREADS) void decode_attention_kernel(const f16* __
     if (pos < 0 || (FUSED && pos >= max_len)) return;          // uniform over the block; nothing is written
     const int n = (int)(pos < max_len ? pos + 1 : max_len);    // keys 0 .. n-1
 
-    // Everything the block needs from memory is requested here, in one go, before anything is computed: the new
-    // token's q / k / v and angles first (they come from L2 and are needed first), then the group's first PRE
-    // cache positions (rows past the sequence are clamped to its last row: one row per wave, never used).
-    f16x8 qraw, kraw, vraw;
-    float c[4], s[4];
-    if constexpr (FUSED) {
-        const f16* row = q_or_qkv + (size_t)b * 3 * heads * HD + (size_t)h * HD + j * 8;
+    auto attend = [&](auto pre_tag) __attribute__((always_inline)) {
+        constexpr int PRE = decltype(pre_tag)::value;
+        // Everything the block needs from memory is requested here, in one go, before anything is computed: the new
+        // token's q / k / v and angles first (they come from L2 and are needed first), then the group's first PRE
+        // cache positions.  The new position, and the end of the sequence, lie in the last of these stages or behind it.
+        f16x8 qraw, kraw, vraw;
+        float c[4], s[4];
+        if constexpr (FUSED) {
+            const f16* row = q_or_qkv + (size_t)b * 3 * heads * HD + (size_t)h * HD + j * 8;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            c[i] = cos_t[pos * (HD / 2) + j * 4 + i];
-            s[i] = sin_t[pos * (HD / 2) + j * 4 + i];
+            for (int i = 0; i < 4; i++) {
+                c[i] = cos_t[pos * (HD / 2) + j * 4 + i];
+                s[i] = sin_t[pos * (HD / 2) + j * 4 + i];
+            }
+            qraw = *reinterpret_cast<const f16x8*>(row);
+            if (g == 0) {
+                kraw = *reinterpret_cast<const f16x8*>(row + (size_t)heads * HD);
+                vraw = *reinterpret_cast<const f16x8*>(row + (size_t)2 * heads * HD);
+            }
+        } else {
+            qraw = *reinterpret_cast<const f16x8*>(q_or_qkv + head * HD + j * 8);
         }
-        qraw = *reinterpret_cast<const f16x8*>(row);
-        if (g == 0) {
-            kraw = *reinterpret_cast<const f16x8*>(row + (size_t)heads * HD);
-            vraw = *reinterpret_cast<const f16x8*>(row + (size_t)2 * heads * HD);
-        }
-    } else {
-        qraw = *reinterpret_cast<const f16x8*>(q_or_qkv + head * HD + j * 8);
-    }
-    f16x8 kpre[PRE > 0 ? PRE : 1], vpre[PRE > 0 ? PRE : 1];
+        f16x8 kpre[PRE], vpre[PRE];
 #pragma unroll
-    for (int i = 0; i < PRE; i++) {
-        // a position past the sequence, and the new position itself (which the block is about to write and serves
-        // from LDS), fetch row 0 instead: a row that is being read anyway, and never the line that is being written
-        const int p = (g + i * GROUPS < (FUSED ? n - 1 : n)) ? g + i * GROUPS : 0;
-        kpre[i] = *reinterpret_cast<const f16x8*>(kc + (size_t)p * HD + j * 8);
-        vpre[i] = *reinterpret_cast<const f16x8*>(vc + (size_t)p * HD + j * 8);
-    }
-    f16x8 qv = qraw;
-    if constexpr (FUSED) {
-        qv = rotate8(qraw, c, s);
-        if (g == 0) {
-            const f16x8 kr = rotate8(kraw, c, s);
-            *reinterpret_cast<f16x8*>(kc + (size_t)pos * HD + j * 8) = kr;
-            *reinterpret_cast<f16x8*>(vc + (size_t)pos * HD + j * 8) = vraw;
-            *reinterpret_cast<f16x8*>(new_k + j * 8) = kr;
-            *reinterpret_cast<f16x8*>(new_v + j * 8) = vraw;
+        for (int i = 0; i < PRE; i++) {
+            // a position past the sequence, and the new position itself (which the block is about to write and serves
+            // from LDS), fetch row 0 instead: a row that is being read anyway, and never the line that is being written
+            const int p = i < PRE - 1 || g + i * GROUPS < (FUSED ? n - 1 : n) ? g + i * GROUPS : 0;
+            kpre[i] = *reinterpret_cast<const f16x8*>(kc + (size_t)p * HD + j * 8);
+            vpre[i] = *reinterpret_cast<const f16x8*>(vc + (size_t)p * HD + j * 8);
         }
-        __syncthreads();
-    }
-    float qf[8];
+        f16x8 qv = qraw;
+        if constexpr (FUSED) {
+            qv = rotate8(qraw, c, s);
+            if (g == 0) {
+                const f16x8 kr = rotate8(kraw, c, s);
+                *reinterpret_cast<f16x8*>(kc + (size_t)pos * HD + j * 8) = kr;
+                *reinterpret_cast<f16x8*>(vc + (size_t)pos * HD + j * 8) = vraw;
+                *reinterpret_cast<f16x8*>(new_k + j * 8) = kr;
+                *reinterpret_cast<f16x8*>(new_v + j * 8) = vraw;
+            }
+            __syncthreads();
+        }
+        float qf[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) qf[e] = (float)qv[e] * scale;
+        for (int e = 0; e < 8; e++) qf[e] = (float)qv[e] * scale;
 
-    // one pass over the cache with a running maximum: key and value row of a position are requested together
-    float m = -INFINITY, l = 0.f;
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    auto visit = [&](const f16x8 kv, const f16x8 vv) {
-        float d = 0.f;
+        // one pass over the cache with a running maximum: key and value row of a position are requested together
+        float m = -INFINITY, l = 0.f;
+        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        auto visit = [&](const f16x8 kv, const f16x8 vv) {
+            float d = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; e++) d += qf[e] * (float)kv[e];
-        d = group_sum<LPK>(d);                                                  // stays inside the group: all its lanes are here
-        const float m_new = fmaxf(m, d);
-        const float keep = __expf(m - m_new), w = __expf(d - m_new);           // m = -inf the first time: keep = 0
-        l = l * keep + w;
+            for (int e = 0; e < 8; e++) d += qf[e] * (float)kv[e];
+            d = group_sum<LPK>(d);                                                  // stays inside the group: all its lanes are here
+            const float m_new = fmaxf(m, d);
+            const float keep = __expf(m - m_new), w = __expf(d - m_new);           // m = -inf the first time: keep = 0
+            l = l * keep + w;
 #pragma unroll
-        for (int e = 0; e < 8; e++) acc[e] = acc[e] * keep + w * (float)vv[e];
-        m = m_new;
-    };
-    if constexpr (PRE > 0) {
-        // the positions requested at the top, all at once: their scores are independent of each other, so the dot
-        // products and the lane exchanges of the PRE positions overlap, and one maximum serves them all (no
-        // rescaling chain from position to position)
-        float d[PRE];
-        f16x8 vsel[PRE];
-#pragma unroll
-        for (int i = 0; i < PRE; i++) {
-            const bool fresh = FUSED && g + i * GROUPS == (int)pos;             // the block has just written this row: serve it from LDS
-            const f16x8 kv = fresh ? *reinterpret_cast<const f16x8*>(new_k + j * 8) : kpre[i];
-            vsel[i] = fresh ? *reinterpret_cast<const f16x8*>(new_v + j * 8) : vpre[i];
-            d[i] = 0.f;
-#pragma unroll
-            for (int e = 0; e < 8; e++) d[i] += qf[e] * (float)kv[e];
-        }
-#pragma unroll
-        for (int i = 0; i < PRE; i++) d[i] = group_sum<LPK>(d[i]);
-#pragma unroll
-        for (int i = 0; i < PRE; i++) {
-            if (g + i * GROUPS >= n) d[i] = -INFINITY;                          // past the sequence (row 0 was fetched instead)
-            m = fmaxf(m, d[i]);
-        }
-        if (m != -INFINITY) {
+            for (int e = 0; e < 8; e++) acc[e] = acc[e] * keep + w * (float)vv[e];
+            m = m_new;
+        };
+        {
+            // the positions requested at the top, all at once: their scores are independent of each other, so the dot
+            // products and the lane exchanges of the PRE positions overlap, and one maximum serves them all (no
+            // rescaling chain from position to position)
+            float d[PRE];
+            f16x8 vsel[PRE];
 #pragma unroll
             for (int i = 0; i < PRE; i++) {
-                const float w = __expf(d[i] - m);                               // 0 for a position past the sequence
-                l += w;
+                const bool fresh = FUSED && i == PRE - 1 && g + i * GROUPS == (int)pos;     // the block has just written this row: serve it from LDS
+                const f16x8 kv = fresh ? *reinterpret_cast<const f16x8*>(new_k + j * 8) : kpre[i];
+                vsel[i] = fresh ? *reinterpret_cast<const f16x8*>(new_v + j * 8) : vpre[i];
+                d[i] = 0.f;
 #pragma unroll
-                for (int e = 0; e < 8; e++) acc[e] += w * (float)vsel[i][e];
+                for (int e = 0; e < 8; e++) d[i] += qf[e] * (float)kv[e];
+            }
+#pragma unroll
+            for (int i = 0; i < PRE; i++) d[i] = group_sum<LPK>(d[i]);
+#pragma unroll
+            for (int i = 0; i < PRE; i++) {
+                if (i == PRE - 1 && g + i * GROUPS >= n) d[i] = -INFINITY;          // past the sequence (row 0 was fetched instead)
+                m = fmaxf(m, d[i]);
+            }
+            if (m != -INFINITY) {
+#pragma unroll
+                for (int i = 0; i < PRE; i++) {
+                    const float w = __expf(d[i] - m);                               // 0 for a position past the sequence
+                    l += w;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) acc[e] += w * (float)vsel[i][e];
+                }
             }
         }
-    }
 #pragma unroll 2
-    for (int p = g + PRE * GROUPS; p < n; p += GROUPS) {
-        const bool fresh = FUSED && p == (int)pos;
-        visit(fresh ? *reinterpret_cast<const f16x8*>(new_k + j * 8) : *reinterpret_cast<const f16x8*>(kc + (size_t)p * HD + j * 8),
-              fresh ? *reinterpret_cast<const f16x8*>(new_v + j * 8) : *reinterpret_cast<const f16x8*>(vc + (size_t)p * HD + j * 8));
-    }
-    // merge the 64/LPK groups of a wave (lanes that differ in the bits above log2(LPK)) ...
-#pragma unroll
-    for (int o = LPK; o < 64; o <<= 1) {
-        const float m_o = __shfl_xor(m, o, 64), l_o = __shfl_xor(l, o, 64);
-        const float top = fmaxf(m, m_o);
-        const float a = (m == -INFINITY) ? 0.f : __expf(m - top), b = (m_o == -INFINITY) ? 0.f : __expf(m_o - top);
-        l = l * a + l_o * b;
-#pragma unroll
-        for (int e = 0; e < 8; e++) acc[e] = acc[e] * a + __shfl_xor(acc[e], o, 64) * b;
-        m = top;
-    }
-    // ... and the waves through LDS
-    if ((threadIdx.x & 63) < LPK) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) part[(threadIdx.x >> 6) * HD + j * 8 + e] = acc[e];
-        if (j == 0) {
-            part_m[threadIdx.x >> 6] = m;
-            part_l[threadIdx.x >> 6] = l;
+        for (int p = g + PRE * GROUPS; p < n; p += GROUPS) {
+            const bool fresh = FUSED && p == (int)pos;
+            visit(fresh ? *reinterpret_cast<const f16x8*>(new_k + j * 8) : *reinterpret_cast<const f16x8*>(kc + (size_t)p * HD + j * 8),
+                  fresh ? *reinterpret_cast<const f16x8*>(new_v + j * 8) : *reinterpret_cast<const f16x8*>(vc + (size_t)p * HD + j * 8));
         }
-    }
-    __syncthreads();
-    for (int d = threadIdx.x; d < HD; d += THREADS) {
-        float top = -INFINITY;
+        // merge the 64/LPK groups of a wave (lanes that differ in the bits above log2(LPK)) ...
 #pragma unroll
-        for (int w = 0; w < WAVES; w++) top = fmaxf(top, part_m[w]);
-        float num = 0.f, den = 0.f;
+        for (int o = LPK; o < 64; o <<= 1) {
+            const float m_o = __shfl_xor(m, o, 64), l_o = __shfl_xor(l, o, 64);
+            const float top = fmaxf(m, m_o);
+            const float a = (m == -INFINITY) ? 0.f : __expf(m - top), b = (m_o == -INFINITY) ? 0.f : __expf(m_o - top);
+            l = l * a + l_o * b;
 #pragma unroll
-        for (int w = 0; w < WAVES; w++) {
-            const float f = (part_m[w] == -INFINITY) ? 0.f : __expf(part_m[w] - top);
-            num += part[w * HD + d] * f;
-            den += part_l[w] * f;
+            for (int e = 0; e < 8; e++) acc[e] = acc[e] * a + __shfl_xor(acc[e], o, 64) * b;
+            m = top;
         }
-        out[head * HD + d] = (f16)(num / den);
+        // ... and the waves through LDS
+        if ((threadIdx.x & 63) < LPK) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) part[(threadIdx.x >> 6) * HD + j * 8 + e] = acc[e];
+            if (j == 0) {
+                part_m[threadIdx.x >> 6] = m;
+                part_l[threadIdx.x >> 6] = l;
+            }
+        }
+        __syncthreads();
+        for (int d = threadIdx.x; d < HD; d += THREADS) {
+            float top = -INFINITY;
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) top = fmaxf(top, part_m[w]);
+            float num = 0.f, den = 0.f;
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) {
+                const float f = (part_m[w] == -INFINITY) ? 0.f : __expf(part_m[w] - top);
+                num += part[w * HD + d] * f;
+                den += part_l[w] * f;
+            }
+            out[head * HD + d] = (f16)(num / den);
+        }
+    };
+    static_assert(MOST == 8, "one form per number of stages");
+    switch (min((n + GROUPS - 1) / GROUPS, MOST)) {
+        case 1: attend(Tag<1>{}); break;
+        case 2: attend(Tag<2>{}); break;
+        case 3: attend(Tag<3>{}); break;
+        case 4: attend(Tag<4>{}); break;
+        case 5: attend(Tag<5>{}); break;
+        case 6: attend(Tag<6>{}); break;
+        case 7: attend(Tag<7>{}); break;
+        default: attend(Tag<8>{});
     }
 }
 

@@ -127,6 +127,13 @@ def test_rope_cache_append_and_attention_match_torch(B, H, hd, max_len, pos):
     assert (att.float() - want_att).abs().max() <= 1e-2 * want_att.abs().max() + 2e-3
 
 
+@pytest.mark.parametrize("hd,pos", [(128, p) for p in (30, 31, 32, 63, 64, 96, 127, 159, 160, 191, 223, 224, 254, 255, 256, 257, 319)]
+                         + [(64, 63), (64, 64), (64, 319), (32, 127), (32, 128), (256, 15), (256, 16), (256, 127), (256, 128), (256, 200)])
+def test_attention_at_the_ends_of_its_stages(hd, pos):
+    """The last key of a stage, the first of the next, and sequences longer than all stages: every number of stages."""
+    test_rope_cache_append_and_attention_match_torch(2, 3, hd, 320, pos)
+
+
 def test_rope_and_cache_write_of_a_whole_prompt():
     """``qf_rope_kv_store_rows`` (prefill): every token of every sequence gets the rotation and the cache rows the
     one-position kernel gives it, bit for bit, and what the PyTorch ops of ``QuantLlama.forward`` give within the
