@@ -124,6 +124,35 @@ template <int NBITS> struct DequantStep {
     }
 };
 
+// Elements 2P, 2P + 1 of the same eight, from the word that holds them (2 bits: shifted so that they lie in its even bytes).
+template <int NBITS> struct DequantPair;
+
+template <> struct DequantPair<4> {
+    template <int P>
+    __device__ __forceinline__ static f16x2 run(uint32_t w, const QConst& c) {
+        const uint32_t x = P >= 2 ? w >> 8 : w, mg = magic_register();
+        if constexpr (P % 2 == 0) return (as_f16x2(and_or<0x000F000Fu>(x, mg)) + c.z.off[0]) * c.s2;
+        else return __builtin_elementwise_fma(as_f16x2(and_or<0x00F000F0u>(x, mg)), f16x2{(_Float16)0.0625f, (_Float16)0.0625f}, c.z.off[1]) * c.s2;
+    }
+};
+
+template <> struct DequantPair<2> {
+    template <int P>
+    __device__ __forceinline__ static f16x2 run(uint32_t w, const QConst& c) {
+        const float inv = Decode<2>::inv_scale(P);
+        return __builtin_elementwise_fma(as_f16x2(and_or<0x00030003u << (2 * P)>(w, magic_register())), f16x2{(_Float16)inv, (_Float16)inv}, c.z.off[P]) * c.s2;
+    }
+};
+
+template <> struct DequantPair<8> {
+    template <int P>
+    __device__ __forceinline__ static f16x2 run(uint32_t w, const QConst& c) {
+        uint32_t x[2];
+        Decode<8>::word(w, x);
+        return (as_f16x2(x[P % 2]) + c.z.off[0]) * c.s2;
+    }
+};
+
 template <int T>
 __device__ __forceinline__ f16x8 DequantStep3::run(const uint32_t (&w)[4], uint32_t h, const QConst& c) {
     const f16x8 s8 = f16x8{c.s2.x, c.s2.y, c.s2.x, c.s2.y, c.s2.x, c.s2.y, c.s2.x, c.s2.y};

@@ -15,15 +15,16 @@
 //     packed weight windows (BN rows x 128 bytes = 1024/NBITS elements, WS buffers), both in the same XOR-swizzled form.
 //     No packed word waits in a register on its way, which is what leaves room for the accumulators.
 //   * A K-iteration of KI x 64 elements is 4 * KI segments, one MFMA k-step each.  Segment g issues the MFMAs of k-step g,
-//     dequantises the weight fragments of g + 1 and reads the activation fragments of g + AHEAD, interleaved instruction
-//     by instruction (sched_group_barrier): nothing is waited for in front of an MFMA.  The one block barrier of an
-//     iteration stands in front of the first segment that reads the next tile, not at its end, so the MFMAs of the
-//     last AHEAD segments run behind it on registers.
+//     dequantises the weight fragments of g + 1 and reads the activation fragments of g + AHEAD, dealt out behind the
+//     MFMAs: nothing is waited for in front of an MFMA.  The one block barrier of an iteration stands in front of the first
+//     segment that reads the next tile, not at its end, so the MFMAs of the last AHEAD segments run behind it on registers.
 //   * Reuse and arrival: the barrier of iteration t is passed when every wave has read all of tile t (its LDS reads have
-//     returned) and its own requests for tile t + 1 have landed.  Tile t + 2 is requested in iteration t, behind the
-//     barrier of t - 1, into the buffer of tile t - 1; packed windows likewise, a window ahead.  The wait allows the
-//     requests of the current iteration to stay in flight and counts nothing else, so loads that the compiler places
-//     itself (scales, zero-points) can only make it stricter.
+//     returned) and its own requests for tile t + 1 have landed.  Between the barriers of t - 1 and t tile t + 2 is
+//     requested, into the buffer of tile t - 1, an equal share in every segment (all in the segments of iteration t in
+//     front of its barrier, the four waves of a CU asked for more at a time than its address unit takes, and waited to
+//     issue: 1 - 4 % of a launch); packed windows in front of the barrier, a window ahead.  The wait allows the requests since
+//     the barrier before it to stay in flight and counts nothing else, so loads that the compiler places itself (scales,
+//     zero-points) can only make it stricter.
 //   * WK groups of waves deal the windows of K between them where a launch has few tiles; their sums meet in LDS.
 #pragma once
 
@@ -76,13 +77,13 @@ struct GemmWideCfg {
     static constexpr size_t LDS_BYTES = WK * LDS_TILES > LDS_END ? WK * LDS_TILES : LDS_END;
 };
 
+// first of n pieces of work that falls to slot i of `slots`, dealt out evenly from the first slot on
+constexpr int wide_first(int i, int n, int slots) { return i < slots ? (i * n + slots - 1) / slots : n; }
+// pieces that fall to `part` of `parts` where piece p belongs to part p % parts
+constexpr int wide_part(int n, int part, int parts) { return (n - part + parts - 1) / parts; }
 // requests for packed words a wave issues in iteration q of a window
 template <class C>
-constexpr int wide_window_requests(int q) {
-    int n = 0;
-    for (int p = 0; p < C::UW; p++) n += p % C::PARTS == q ? 1 : 0;
-    return n;
-}
+constexpr int wide_window_requests(int q) { return q < C::PARTS ? wide_part(C::UW, q, C::PARTS) : 0; }
 
 // 16 bytes per lane from global memory straight into LDS, address = base + per-lane offset + wave-uniform offset: the
 // buffer form adds them in the address unit (the flat form costs a 64-bit vector add and a register pair per request)
@@ -153,15 +154,13 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
     const buffer_rsrc a_slab = rows_from(A + (size_t)m_blk * C::K);
     // the group's window w and its iteration `it` in the whole row; past the end the last ones
     auto window_of = [&](int w) { return min(w * C::WK + grp, C::NSUP - 1); };
-    auto request_a = [&](int buf, int it, int part, int parts) {
-        // the same for all lanes, and said so: where the compiler had formed it with vector instructions (short rows of K),
-        // every request became a loop over the values of the lanes
-        const uint32_t at = __builtin_amdgcn_readfirstlane(((uint32_t)window_of(it / SUP) * SUP + (uint32_t)(it % SUP)) * (128u * C::KI));
-        uint8_t* dst = as_b + (size_t)buf * C::A_TILE;
-#pragma unroll
-        for (int p = 0; p < C::UA; p++)
-            if (p % parts == part)
-                buffer_to_lds_16(a_slab, a_off[p], at, dst + min(p * WAVES + wave, C::AB - 1) * 1024);
+    // byte offset in a row of the group's iteration `it`: the same for all lanes, and said so: where the compiler had formed it
+    // with vector instructions (short rows of K), every request became a loop over the values of the lanes
+    auto tile_at = [&](int it) {
+        return __builtin_amdgcn_readfirstlane(((uint32_t)window_of(it / SUP) * SUP + (uint32_t)(it % SUP)) * (128u * C::KI));
+    };
+    auto request_a = [&](int buf, uint32_t at, int p) __attribute__((always_inline)) {
+        buffer_to_lds_16(a_slab, a_off[p], at, as_b + (size_t)buf * C::A_TILE + min(p * WAVES + wave, C::AB - 1) * 1024);
     };
     // byte offset of the lane's unit from the block's first packed row (gate+up: from the first gate row; below 4 GiB, checked by the host)
     const int n_first = SILU ? min(n_blk >> 1, C::N / 2 - 1) : min(n_blk, C::N - 1);
@@ -172,20 +171,19 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
         w_off[p] = (uint32_t)(packed_row(row) - n_first) * C::RB + c * 16;
     }
     const buffer_rsrc w_rows = rows_from(W + (size_t)n_first * C::RB);
-    auto request_w = [&](int slot, int sup, int part) {
-        uint8_t* dst = ws_b + slot * C::W_TILE;
-        const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)sup * 128u);      // a scalar operand of the request, as in request_a
-#pragma unroll
-        for (int p = 0; p < C::UW; p++)
-            if (part < 0 || p % C::PARTS == part) buffer_to_lds_16(w_rows, w_off[p], at, dst + min(p * WAVES + wave, C::WB - 1) * 1024);
+    auto window_at = [&](int sup) { return __builtin_amdgcn_readfirstlane((uint32_t)sup * 128u); };      // a scalar operand, as tile_at
+    auto request_w = [&](int slot, uint32_t at, int p) __attribute__((always_inline)) {
+        buffer_to_lds_16(w_rows, w_off[p], at, ws_b + slot * C::W_TILE + min(p * WAVES + wave, C::WB - 1) * 1024);
     };
 
     // the first windows and tiles go out before anything else is computed
 #pragma unroll
     for (int w = 0; w < C::WS - 1; w++)
-        if (w < C::NWIN) request_w(w, window_of(w), -1);
-    request_a(0, 0, 0, 1);
-    if (C::ITERS > 1) request_a(1, 1, 0, 1);
+        if (w < C::NWIN)
+#pragma unroll
+            for (int p = 0; p < C::UW; p++) request_w(w, window_at(window_of(w)), p);
+#pragma unroll
+    for (int p = 0; p < C::UA; p++) request_a(0, tile_at(0), p);
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- scales and zero-points of the wave's rows, one window in registers and the next on its way ----
@@ -228,24 +226,21 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
         }
     };
     QConst qc[NT];
-    auto make_consts = [&](const Quant& qu, int q) {
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            uint32_t sbits, zero;
-            if constexpr (C::GS >= C::SUPK) {
-                sbits = qu.s[j][0] & 0xFFFFu;
-                zero = qu.z[j] & ZMASK;
-            } else if constexpr (C::GS >= 64) {
-                const int gi = q * 64 / C::GS;
-                sbits = (qu.s[j][gi / 2] >> (16 * (gi % 2))) & 0xFFFFu;
-                zero = (qu.z[j] >> (gi * C::NBITS)) & ZMASK;
-            } else {                                           // GS == 32: group 2q + kb
-                sbits = kb ? (qu.s[j][q] >> 16) : (qu.s[j][q] & 0xFFFFu);
-                zero = (qu.z[j] >> ((2 * q + kb) * C::NBITS)) & ZMASK;
-            }
-            if constexpr (C::SYM) zero = 1u << (C::NBITS - 1);
-            qc[j] = make_qconst<C::NBITS>((uint16_t)sbits, zero);
+    auto make_consts = [&](const Quant& qu, int q, int j) __attribute__((always_inline)) {
+        uint32_t sbits, zero;
+        if constexpr (C::GS >= C::SUPK) {
+            sbits = qu.s[j][0] & 0xFFFFu;
+            zero = qu.z[j] & ZMASK;
+        } else if constexpr (C::GS >= 64) {
+            const int gi = q * 64 / C::GS;
+            sbits = (qu.s[j][gi / 2] >> (16 * (gi % 2))) & 0xFFFFu;
+            zero = (qu.z[j] >> (gi * C::NBITS)) & ZMASK;
+        } else {                                               // GS == 32: group 2q + kb
+            sbits = kb ? (qu.s[j][q] >> 16) : (qu.s[j][q] & 0xFFFFu);
+            zero = (qu.z[j] >> ((2 * q + kb) * C::NBITS)) & ZMASK;
         }
+        if constexpr (C::SYM) zero = 1u << (C::NBITS - 1);
+        qc[j] = make_qconst<C::NBITS>((uint16_t)sbits, zero);
     };
 
     f32x16 acc[NT][MT];
@@ -271,104 +266,112 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
 
     // packed fields of the lane for iteration q of a window: 32 fields = 4*NBITS bytes per tile
     struct Packed { uint32_t w[NT][C::NBITS]; };
-    auto read_packed = [&](Packed& pk, int slot, int q) __attribute__((always_inline)) {
-        const uint32_t lane_at = opaque(w_lane);
+    auto read_packed = [&](Packed& pk, uint32_t lane_at, int slot, int q, int j) __attribute__((always_inline)) {
+        const uint8_t* tile = smem + slot * C::W_TILE + j * 4096;
+        if constexpr (C::NBITS == 2) {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(tile + (lane_at ^ (16 * q)));
+            pk.w[j][0] = v.x; pk.w[j][1] = v.y;
+        } else {
 #pragma unroll
-        for (int j = 0; j < NT; j++) {
-            const uint8_t* tile = smem + slot * C::W_TILE + j * 4096;
-            if constexpr (C::NBITS == 4) {
-                const u32x4 v = *reinterpret_cast<const u32x4*>(tile + (lane_at ^ (32 * q)));
-                pk.w[j][0] = v.x; pk.w[j][1] = v.y; pk.w[j][2] = v.z; pk.w[j][3] = v.w;
-            } else if constexpr (C::NBITS == 8) {
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const u32x4 v = *reinterpret_cast<const u32x4*>(tile + (lane_at ^ (64 * q + 16 * h)));
-                    pk.w[j][4 * h] = v.x; pk.w[j][4 * h + 1] = v.y; pk.w[j][4 * h + 2] = v.z; pk.w[j][4 * h + 3] = v.w;
-                }
-            } else {
-                const u32x2 v = *reinterpret_cast<const u32x2*>(tile + (lane_at ^ (16 * q)));
-                pk.w[j][0] = v.x; pk.w[j][1] = v.y;
+            for (int h = 0; h < C::NBITS / 4; h++) {
+                const u32x4 v = *reinterpret_cast<const u32x4*>(tile + (lane_at ^ (8 * C::NBITS * q + 16 * h)));
+                pk.w[j][4 * h] = v.x; pk.w[j][4 * h + 1] = v.y; pk.w[j][4 * h + 2] = v.z; pk.w[j][4 * h + 3] = v.w;
             }
         }
     };
     f16x8 af[C::SETS][MT], wf[2][NT];
     Packed pk[2];
-    auto read_frags = [&](f16x8 (&f)[MT], int buf, int seg) __attribute__((always_inline)) {
-        const uint32_t lane_at = (opaque(a_lane) ^ (16 * (seg % 4))) + (uint32_t)buf * C::A_TILE + (seg / 4) * C::BM * 128;
-#pragma unroll
-        for (int i = 0; i < MT; i++) f[i] = *reinterpret_cast<const f16x8*>(smem + lane_at + i * 4096);
+    auto frags_at = [&](int buf, int seg) __attribute__((always_inline)) {
+        return (opaque(a_lane) ^ (16 * (seg % 4))) + (uint32_t)buf * C::A_TILE + (seg / 4) * C::BM * 128;
     };
-    auto dequant = [&](f16x8 (&f)[NT], const Packed& pk, int ks) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            uint32_t w4[4];
-            if constexpr (C::NBITS == 8) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) w4[e] = pk.w[j][4 * (ks / 2) + e];
-                f[j] = DequantStep<8>::run(w4, ks % 2, qc[j]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; e++) w4[e] = e < C::NBITS ? pk.w[j][e] : 0u;
-                f[j] = DequantStep<C::NBITS>::run(w4, ks, qc[j]);
-            }
-        }
+    auto read_frag = [&](f16x8 (&f)[MT], uint32_t lane_at, int i) __attribute__((always_inline)) {
+        f[i] = *reinterpret_cast<const f16x8*>(smem + lane_at + i * 4096);
     };
-    auto multiply = [&](const f16x8 (&w)[NT], const f16x8 (&a)[MT]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < MT; i++)
-#pragma unroll
-            for (int j = 0; j < NT; j++)
-                acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[j], a[i], acc[j][i], 0, 0, 0);
+    // half a weight fragment: four of the lane's eight elements of k-step ks, six or seven instructions
+    auto dequant_half = [&](f16x8& f, const Packed& pk, int ks, int j, auto h_tag) __attribute__((always_inline)) {
+        constexpr int h = decltype(h_tag)::value;
+        const uint32_t word = C::NBITS == 8 ? pk.w[j][2 * ks + h]
+                            : C::NBITS == 4 ? pk.w[j][ks]
+                            : ks % 2 != 0   ? pk.w[j][ks / 2] >> 8 : pk.w[j][ks / 2];
+        const f16x2 v0 = DequantPair<C::NBITS>::template run<2 * h>(word, qc[j]), v1 = DequantPair<C::NBITS>::template run<2 * h + 1>(word, qc[j]);
+        f[4 * h] = v0.x; f[4 * h + 1] = v0.y; f[4 * h + 2] = v1.x; f[4 * h + 3] = v1.y;
     };
-    // The instruction mix of a segment, dealt out evenly: behind every MFMA a share of the LDS reads, of the vector
-    // instructions and of the requests.
-    auto interleave = [&](auto reads_tag) __attribute__((always_inline)) {
-        constexpr int MF = MT * NT, VALU = NT * 13 + 4, READS = decltype(reads_tag)::value;
-#pragma unroll
-        for (int i = 0; i < MF; i++) {
+
+    // How a segment's work is dealt out behind its MFMAs.  One weight tile per wave: by hand, each MFMA followed by its share
+    // and a fence.  More: the scheduler deals out the mix named here -- behind every MFMA a share of the LDS reads and of
+    // the vector instructions, the requests at equal distances.  Both ways measured on all tilings, three layers, 32 ... 2048
+    // rows: with one weight tile by hand 1 - 7 % less, mean 4 % (half a fragment's six or seven instructions fit behind
+    // one MFMA, and the scheduler's groups let them pile up behind the last one); with two and three 2 - 5 % more (there
+    // halves leave every second or third MFMA without work and its neighbour with too much).
+    auto interleave = [&](auto reads_tag, auto requests_tag) __attribute__((always_inline)) {
+        constexpr int MF = MT * NT, VALU = NT * 13 + 4, READS = decltype(reads_tag)::value, REQUESTS = decltype(requests_tag)::value;
+        static_for<0, MF>([&](auto i_tag) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_tag)::value, here = (i + 1) * REQUESTS / MF - i * REQUESTS / MF;
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                         // one MFMA
             __builtin_amdgcn_sched_group_barrier(0x100, (READS + MF - 1) / MF, 0);     // LDS reads
             __builtin_amdgcn_sched_group_barrier(0x002, (VALU + MF - 1) / MF, 0);      // vector instructions
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);                         // a request
-        }
+            if constexpr (here > 0) __builtin_amdgcn_sched_group_barrier(0x020, here, 0);
+        });
         __builtin_amdgcn_sched_barrier(0);
     };
 
+    constexpr bool BY_HAND = NT == 1;
     constexpr int AHEAD = C::AHEAD, SEGS = C::SEGS, KI = C::KI, WS = C::WS, STEPS = C::STEPS;
     constexpr int LAST_BEFORE = SEGS - AHEAD - 1;              // the barrier follows this segment: the next ones read the next tile
     Quant quant[WS];
+    auto part_of = [](int g) constexpr { return (g - LAST_BEFORE - 1 + SEGS) % SEGS; };       // segments since the last barrier
     // iteration `it` of the group; s = it % PASS a constant, live 0: nothing to multiply (a group with one window less), left:
     // iterations behind this one, where that is known to be few (tiles and windows past the end are not requested, and the
-    // last iteration reads nothing ahead and meets nobody); b0, b1, b2 the buffers of tiles it, it + 1 and it + 2
+    // last iteration reads nothing ahead and meets nobody); b0, b1, b2 the buffers of tiles it (and, behind its barrier,
+    // it + 3), it + 1 and it + 2
     auto iteration = [&](int it, auto s_tag, auto live_tag, auto left_tag, int b0, int b1, int b2) __attribute__((always_inline)) {
         constexpr int s = decltype(s_tag)::value, left = decltype(left_tag)::value;
         constexpr int q = s % SUP, win = s / SUP;              // iteration of the window; window counted inside a pass
-        constexpr bool next_tile = left >= 1, request_tile = left >= 2, request_window = (left + q) / SUP >= WS - 1;
+        constexpr bool next_tile = left >= 1, request_tile = left >= 2, request_later = left >= 3, request_window = (left + q) / SUP >= WS - 1;
         constexpr int requests = (request_tile ? C::UA : 0) + (request_window ? wide_window_requests<C>(q) : 0);
         const int sup = it / SUP;
         static_for<0, SEGS>([&](auto g_tag) __attribute__((always_inline)) {
             constexpr int g = decltype(g_tag)::value, step = s * KI + g / 4;
-            // fragments of segment g + AHEAD
-            if constexpr (g + AHEAD < SEGS) read_frags(af[(g + AHEAD) % C::SETS], b0, g + AHEAD);
-            else if constexpr (next_tile) read_frags(af[(g + AHEAD) % C::SETS], b1, g + AHEAD - SEGS);
-            // packed words of the next 64-element step, in front of the first segment that dequantises them
+            // what the segment does beside its MFMAs: reads of the fragments of segment g + AHEAD; of the packed words of the next
+            // 64-element step, in front of the first segment that dequantises them; the weight fragments of segment g + 1; requests
             constexpr int next = step + 1, next_win = next / STEPS % WS;
+            constexpr bool frags_here = next_tile || g + AHEAD < SEGS;
             constexpr bool packed_here = g % 4 == 4 - AHEAD && (next_tile || g + 4 < SEGS);
-            if constexpr (packed_here) read_packed(pk[next % 2], next_win, next % STEPS);
-            // weight fragments of segment g + 1
-            if constexpr (g == SEGS - 1 && !next_tile) {
-            } else if constexpr (g % 4 == 3) {
-                constexpr int qn = next % STEPS;
-                if constexpr (qn * 64 % C::GS == 0 || qn == 0) make_consts(quant[next_win], qn);
-                dequant(wf[(g + 1) % 2], pk[next % 2], 0);
-            } else {
-                dequant(wf[(g + 1) % 2], pk[step % 2], g % 4 + 1);
-            }
+            constexpr bool dequant_here = g < SEGS - 1 || next_tile, new_step = g % 4 == 3;
+            constexpr bool consts_here = dequant_here && new_step && (next % STEPS * 64 % C::GS == 0 || next % STEPS == 0);
+            constexpr int reads = (frags_here ? MT : 0) + (packed_here ? NT : 0);
+            constexpr int chunks = dequant_here ? (consts_here ? 3 : 2) * NT : 0;
+            constexpr int of_tile = (g <= LAST_BEFORE ? request_tile : request_later) ? wide_part(C::UA, part_of(g), SEGS) : 0;
+            constexpr int of_window = request_window && g == LAST_BEFORE ? wide_window_requests<C>(q) : 0;
+            constexpr int MF = MT * NT;
+            uint32_t frags_from = 0, packed_from = 0, tile_from = 0, window_from = 0;
+            if constexpr (frags_here) frags_from = g + AHEAD < SEGS ? frags_at(b0, g + AHEAD) : frags_at(b1, g + AHEAD - SEGS);
+            if constexpr (packed_here) packed_from = opaque(w_lane);
+            if constexpr (of_tile > 0) tile_from = tile_at(g <= LAST_BEFORE ? it + 2 : it + 3);
+            if constexpr (of_window > 0) window_from = window_at(window_of(sup + WS - 1));
             if constexpr (request_window && g == 0 && q == 0) load_quant(quant[(win + WS - 1) % WS], window_of(sup + WS - 1));
-            if constexpr (request_window && g == LAST_BEFORE && wide_window_requests<C>(q) > 0) request_w((win + WS - 1) % WS, window_of(sup + WS - 1), q);
-            if constexpr (request_tile && g <= LAST_BEFORE) request_a(b2, it + 2, g, LAST_BEFORE + 1);
-            if constexpr (decltype(live_tag)::value != 0) multiply(wf[g % 2], af[g % C::SETS]);
-            interleave(IntTag<(next_tile || g + AHEAD < SEGS ? MT : 0) + (packed_here ? NT * (C::NBITS == 8 ? 2 : 1) : 0)>{});
+            static_for<0, MF>([&](auto slot_tag) __attribute__((always_inline)) {
+                constexpr int slot = decltype(slot_tag)::value, i = slot / NT, j = slot % NT;
+                if constexpr (decltype(live_tag)::value != 0)
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[g % 2][j], af[g % C::SETS][i], acc[j][i], 0, 0, 0);
+                static_for<wide_first(slot, reads, MF), wide_first(slot + 1, reads, MF)>([&](auto r_tag) __attribute__((always_inline)) {
+                    constexpr int r = decltype(r_tag)::value;
+                    if constexpr (packed_here && r < NT) read_packed(pk[next % 2], packed_from, next_win, next % STEPS, r);
+                    else read_frag(af[(g + AHEAD) % C::SETS], frags_from, r - (packed_here ? NT : 0));
+                });
+                static_for<wide_first(slot, chunks, MF), wide_first(slot + 1, chunks, MF)>([&](auto c_tag) __attribute__((always_inline)) {
+                    constexpr int per = consts_here ? 3 : 2, tile = decltype(c_tag)::value / per, part = decltype(c_tag)::value % per - (consts_here ? 1 : 0);
+                    if constexpr (part < 0) make_consts(quant[next_win], next % STEPS, tile);
+                    else dequant_half(wf[(g + 1) % 2][tile], pk[new_step ? next % 2 : step % 2], new_step ? 0 : g % 4 + 1, tile, IntTag<part>{});
+                });
+                static_for<wide_first(slot, of_tile + of_window, MF), wide_first(slot + 1, of_tile + of_window, MF)>([&](auto r_tag) __attribute__((always_inline)) {
+                    constexpr int r = decltype(r_tag)::value;
+                    if constexpr (r < of_tile) request_a(g <= LAST_BEFORE ? b2 : b0, tile_from, part_of(g) + r * SEGS);
+                    else request_w((win + WS - 1) % WS, window_from, q + (r - of_tile) * C::PARTS);
+                });
+                if constexpr (BY_HAND) __builtin_amdgcn_sched_barrier(0);
+            });
+            if constexpr (!BY_HAND) interleave(IntTag<(frags_here ? MT : 0) + (packed_here ? NT * (C::NBITS == 8 ? 2 : 1) : 0)>{}, IntTag<of_tile + of_window>{});
             if constexpr (g == LAST_BEFORE && next_tile) {
                 wait_loads_and_barrier<QF_GEMM_FULL_DRAIN ? 0 : requests>();
                 __builtin_amdgcn_sched_barrier(0);
@@ -378,12 +381,30 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
 
 #pragma unroll
     for (int w = 0; w < WS - 1; w++) load_quant(quant[w], window_of(w));
-    wait_loads_and_barrier<0>();
-    read_packed(pk[0], 0, 0);
+    // tile 1 is younger than all that the first iteration needs and stays in flight over the wait
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (C::ITERS > 1) {
 #pragma unroll
-    for (int g = 0; g < AHEAD; g++) read_frags(af[g], 0, g);
-    make_consts(quant[0], 0);
-    dequant(wf[0], pk[0], 0);
+        for (int p = 0; p < C::UA; p++) request_a(1, tile_at(1), p);
+    }
+    wait_loads_and_barrier<QF_GEMM_FULL_DRAIN || C::ITERS < 2 ? 0 : C::UA>();
+    static_for<0, NT>([&](auto j_tag) __attribute__((always_inline)) {
+        constexpr int j = decltype(j_tag)::value;
+        read_packed(pk[0], opaque(w_lane), 0, 0, j);
+        make_consts(quant[0], 0, j);
+    });
+#pragma unroll
+    for (int g = 0; g < AHEAD; g++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) read_frag(af[g], frags_at(0, g), i);
+    static_for<0, 2 * NT>([&](auto c_tag) __attribute__((always_inline)) {
+        dequant_half(wf[0][decltype(c_tag)::value / 2], pk[0], 0, decltype(c_tag)::value / 2, IntTag<decltype(c_tag)::value % 2>{});
+    });
+    if constexpr (C::ITERS > 2)
+        static_for<LAST_BEFORE + 1, SEGS>([&](auto g_tag) __attribute__((always_inline)) {
+#pragma unroll
+            for (int p = part_of(decltype(g_tag)::value); p < C::UA; p += SEGS) request_a(2, tile_at(2), p);
+        });
 
     // The accumulators stay in the accumulation registers from here to the stores: left to itself the compiler moves all of
     // them to vector registers behind the loop and, short of those, spills the loop's addresses.
@@ -396,10 +417,12 @@ __global__ __launch_bounds__(C::T) void gemm_wide_kernel(
         }
     };
     pin();
-    // Whole passes (the period of the buffers and register sets) and a straight-line rest of at least two iterations, which
-    // also holds the window that some groups do not have: those meet the same barriers and requests without multiplying.
+    // Whole passes (the period of the buffers and register sets) and a straight-line rest, at least as long as the requests
+    // run ahead, which also holds the window that some groups do not have: those meet the same barriers and requests without
+    // multiplying.
     constexpr int PASS = (WS == 3 ? 6 : 2) * SUP;
-    constexpr int FULL_PASSES = C::ITERS / PASS - (C::ITERS >= PASS && C::ITERS % PASS < 2 ? 1 : 0);
+    constexpr int REST_MIN = (WS - 2) * SUP + 1 > 3 ? (WS - 2) * SUP + 1 : 3;
+    constexpr int FULL_PASSES = C::ITERS > REST_MIN ? (C::ITERS - REST_MIN) / PASS : 0;
     constexpr int REST = C::ITERS - FULL_PASSES * PASS, SHARED = C::ODD != 0 ? SUP : 0;
     int b0 = 0, b1 = 1, b2 = 2;
     auto step = [&](int it, auto s_tag, auto live_tag, auto left_tag) __attribute__((always_inline)) {
