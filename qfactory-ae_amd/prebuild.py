@@ -344,6 +344,10 @@ def wide_cases():
         (50, 64, 2048, 2, 128, False, (1, 2, 2, 1, 2, 2)), (70, 132, 640, 8, 64, False, (1, 4, 2, 1, 1, 2)),
         (33, 72, 2816, 4, 128, False, (1, 2, 1, 1, 2, 4)), (40, 33, 3328, 4, 128, False, (1, 1, 1, 1, 2, 4)),
         (34, 68, 1152, 8, 64, True, (1, 2, 1, 1, 1, 4)),
+        # two groups of two waves with two weight tiles each: windows that deal evenly over the groups and not, all widths
+        (129, 260, 1536, 4, 128, False, (1, 2, 4, 2, 1, 2)), (100, 77, 1792, 4, 64, True, (1, 2, 4, 2, 1, 2)),
+        (97, 130, 3584, 2, 64, False, (1, 2, 3, 2, 1, 2)), (66, 136, 1408, 8, 32, True, (1, 2, 3, 2, 1, 2)),
+        (90, 300, 1280, 4, 128, False, (1, 4, 3, 2, 1, 1)), (193, 258, 640, 8, 64, False, (1, 4, 3, 2, 1, 1)),
         # seven waves: the 1 KB blocks of an activation tile do not divide over them
         (100, 230, 1280, 4, 128, False, (1, 7, 2, 1, 2, 1)), (33, 452, 2048, 2, 64, True, (1, 7, 1, 1, 2, 1)),
         (45, 227, 1280, 8, 64, False, (1, 7, 1, 1, 1, 1)), (70, 450, 1024, 8, 128, True, (1, 7, 2, 1, 1, 1)),

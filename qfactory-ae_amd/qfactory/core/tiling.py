@@ -832,29 +832,41 @@ def gemm_candidates(M, N, K, nbits, group_size):
 
 
 # Tilings of the pipelined kernel (qf::GemmWideCfg, include/qf_gemm_wide.hip.h): (WM, WN, MT, NT, KI, WK) -> us per round
-# of blocks and 64 elements of K.  The figures are medians of a sweep of eighteen tilings over 22016 x 4096, 12288 x 4096,
-# 4096 x 4096, 4096 x 11008, 10240 x 8192, 8192 x 28672 and 57344 x 8192 at 32 ... 2048 rows (W4 g128, cold weights): with the
-# round model of gemm_wide_tiling they pick the fastest of the sweep on nearly all of its cells (up to 7 % off on the others).
+# of blocks and 64 elements of K.  The figures are medians of a sweep of eighteen tilings over 22016 x 4096, 4096 x 11008 and
+# 10240 x 8192 at 32 ... 2048 rows (W4 g128, cold weights): with the round model of gemm_wide_tiling they pick the fastest of the
+# sweep on 23 of its 27 cells (up to 3 % off on the others).
 # At 8 bits (ten shapes at 24 ... 1024 rows, the forms of _gemm_wide_tiling) the same figures pick within 7 % of the fastest on 97 of
 # 104 cells, 8 - 16 % off on six, and 63 % off on one (2432 x 20480 at 96 rows, where two rounds of 32 x 32 tiles share CUs).
 GEMM_WIDE_COST = {
-    (1, 4, 8, 2, 1, 1): 1.547,     # 256 x 256
-    (2, 2, 4, 3, 1, 1): 1.289,     # 256 x 192
-    (1, 4, 6, 2, 1, 1): 1.212,     # 192 x 256
-    (1, 4, 4, 2, 1, 1): 0.952,     # 128 x 256
-    (1, 4, 4, 1, 2, 1): 0.572,     # 128 x 128
-    (1, 3, 4, 1, 2, 1): 0.505,     # 128 x 96
-    (1, 4, 3, 1, 2, 1): 0.462,     # 96 x 128
-    (1, 7, 2, 1, 2, 1): 0.620,     # 64 x 224: 57344 columns are 256 of them
-    (1, 4, 2, 1, 2, 2): 0.338,     # 64 x 128
-    (1, 3, 2, 1, 2, 2): 0.307,     # 64 x 96
-    (1, 2, 2, 1, 2, 2): 0.217,     # 64 x 64
-    (1, 7, 1, 1, 2, 1): 0.528,     # 32 x 224
-    (1, 2, 1, 1, 2, 4): 0.148,     # 32 x 64
-    (1, 1, 1, 1, 2, 4): 0.100,     # 32 x 32
+    (1, 4, 8, 2, 1, 1): 1.520,     # 256 x 256
+    (2, 2, 4, 3, 1, 1): 1.258,     # 256 x 192
+    (1, 4, 6, 2, 1, 1): 1.167,     # 192 x 256
+    (1, 4, 4, 2, 1, 1): 0.914,     # 128 x 256
+    (1, 4, 3, 2, 1, 1): 0.742,     # 96 x 256
+    (1, 4, 4, 1, 2, 1): 0.541,     # 128 x 128 ...
+    (1, 2, 4, 2, 1, 2): 0.511,     # ... as two groups of two 128 x 64 waves: half the LDS reads per MFMA
+    (1, 3, 4, 1, 2, 1): 0.472,     # 128 x 96
+    (1, 4, 3, 1, 2, 1): 0.437,     # 96 x 128 ...
+    (1, 2, 3, 2, 1, 2): 0.408,     # ... as two groups of two 96 x 64 waves
+    (1, 7, 2, 1, 2, 1): 0.564,     # 64 x 224: 57344 columns are 256 of them
+    (1, 4, 2, 1, 2, 2): 0.319,     # 64 x 128
+    (1, 3, 2, 1, 2, 2): 0.290,     # 64 x 96
+    (1, 2, 2, 1, 2, 2): 0.198,     # 64 x 64
+    (1, 7, 1, 1, 2, 1): 0.418,     # 32 x 224
+    (1, 2, 1, 1, 2, 4): 0.149,     # 32 x 64
+    (1, 1, 1, 1, 2, 4): 0.103,     # 32 x 32
 }
+# Where those figures do not hold.  8 bits, 32 x 224: 30 rows on 43648 x 9984 103 us as 32 x 64, 114 as 32 x 224 (2 and 4 bits, 23 ... 28
+# rows on 39360 ... 41984 columns: 7 - 19 % less as 32 x 224).
+GEMM_WIDE_COST_8BIT = {(1, 7, 1, 1, 2, 1): 0.528}
+# Two groups of two waves of two weight tiles: from six windows of K on, not at 8 bits.  Of random problems at 17 - 2500 rows those with
+# fewer windows took 1 - 9 % longer than as four waves of one weight tile (462 rows on 6528 x 1024 10.5 -> 11.5 us), at 8 bits
+# ten of fifteen up to 10 % longer (542 rows on 3904 x 3584 25.1 -> 27.2); the others 0 - 17 % less (194 rows on 8576 x 1536
+# level, 394 on 8192 x 4096 36.5 -> 34.2, 1010 on 3648 x 12288 101 -> 89).  An odd window leaves one group without work: 918 rows on
+# 2240 x 1792, seven windows, 12.5 -> 13.4.
+GEMM_WIDE_PAIR_WINDOWS = 6
 GEMM_WIDE_MIN_M = 17           # the 32-row bucket: 9280 x 4608 at 2 bits 13.9 -> 11.6 us, 8192 x 28672 49.8 -> 46.3, 8192 x 8192 level
-# ... but not in more than one and up to two and a half rounds of blocks there: its blocks fill a CU's LDS, so a second round
+# ... but not in more than one and up to two and a half rounds of 32 x 64 blocks there: its blocks fill a CU's LDS, so a second round
 # starts when the first has ended, where the other kernel's smaller blocks share CUs.  Other kernel against this one, 24 rows:
 # 19008 x 14592 at 4 bits 54.9 against 65.4 us, 24576 x 4352 21.4 / 24.4, 23552 x 11776 at 8 bits 80.4 / 89.0; of random problems
 # at 17 - 32 rows 26 of 28 in that range took longer here (up to 21 %), four of five past 2.5 rounds 9 - 10 % less.
@@ -924,15 +936,23 @@ def _gemm_wide_tiling(M, N, K, nbits, group_size):
         bm, bn = 32 * mt * wm, 32 * nt * wn
         if bm >= 2 * M:
             continue
+        if nt == 2 and wk == 2:
+            windows = K * nbits // 1024
+            if nbits == 8 or windows < GEMM_WIDE_PAIR_WINDOWS:
+                continue
+            per_step *= (windows + windows % 2) / windows
+        if nbits == 8:
+            per_step = GEMM_WIDE_COST_8BIT.get((wm, wn, mt, nt, ki, wk), per_step)
         cfg = {"BM": bm, "WM": wm, "WN": wn, "MT": mt, "NT": nt, "KI": ki, "WK": wk, "PA": 3}
         # Where the form of the table does not fit.  8 bits (two steps per iteration take three window buffers): half the
         # groups first -- two steps in half the groups against one step in all of them, ten shapes at 24 ... 512 rows: less
         # time by 5 - 15 % wherever the rule has that choice (10240 x 8192 at 24 rows 32.1 -> 28.9 us, 4096 x 11008 at 128 39.1 -> 33.5, 23552 x 11776 at
         # 64 98.0 -> 87.5).  Short rows: one step per iteration, fewer groups.
         halved = ((ki, wk // 2),) if nbits == 8 and wk > 1 else ()
+        # (not down to fewer than four waves where a wave holds two weight tiles: SIMDs would have none)
         for ki, wk in ((ki, wk),) + halved + ((1, wk), (1, -(-wk // 2)), (1, 1)):
             cfg.update(KI=ki, WK=wk)
-            if gemm_wide_valid(cfg, K, nbits, group_size):
+            if gemm_wide_valid(cfg, K, nbits, group_size) and (nt == 1 or wm * wn * wk >= 4):
                 break
         else:
             continue
@@ -940,8 +960,8 @@ def _gemm_wide_tiling(M, N, K, nbits, group_size):
         whole = -(-exact // 1)
         cost = (0.6 * whole + 0.4 * exact) * per_step
         if best is None or cost < best[0]:
-            best = (cost, cfg, exact * NUM_CUS)
-    if best is None or (M <= 32 and GEMM_WIDE_NOT_AT_32[0] < best[2] <= GEMM_WIDE_NOT_AT_32[1]):
+            best = (cost, cfg)
+    if best is None or (M <= 32 and GEMM_WIDE_NOT_AT_32[0] < -(-N // 64) <= GEMM_WIDE_NOT_AT_32[1]):
         return None
     return best[1]
 
