@@ -26,12 +26,13 @@ int launched(const char* fn) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Weight repack, bound by memory: four bytes are read per field.  A block takes 64 columns n and 32 main-plane words
-// of K (16 threads x 4 columns side by side, 16 units of K): a thread reads 16 bytes of every k of its unit -- 256
-// contiguous bytes per k and 16 threads, all of a unit's loads in flight -- builds four columns' words in registers,
-// and the words change their orientation through LDS, so that a row of the output is written 128 bytes at a time
-// (a 4-byte word per thread straight to its row left 32-byte pieces: 22016 x 4096 at 4 bits 102 us = 4.0 TB/s; this
-// form 76 us = 5.4 TB/s).  Both planes of the 3-bit layout come out of one read of the fields.
+// Weight repack, bound by memory: four bytes are read per field.  A block takes 128 columns n and 32 main-plane words
+// of K (32 threads x 4 columns side by side, 16 units of K): a thread reads 16 bytes of every k of its unit -- 512
+// contiguous bytes per k and 32 threads -- builds four columns' words in registers, and the words change their orientation
+// through LDS, so that a row of the output is written 128 bytes at a time.  (A 4-byte word per thread straight to its row left
+// 32-byte pieces: 22016 x 4096 at 4 bits 102 us = 4.0 TB/s.  Through LDS by columns of a block, 22016 x 4096 / 4096 x 4096 / 8192 x
+// 28672 at 4 bits: 32 columns 81 / 16.7 / 210 us, 64 73 / 15.1 / 190, 128 with 256 threads 71 / 14.1 / 183, 128 with 512 70.6 / 13.8 /
+// 178 = 5.8 TB/s, 256 71 / 18.6 / 188.)  Both planes of the 3-bit layout come out of one read of the fields.
 // Position j of a word holds element (j < P/2 ? 2j : 2(j - P/2) + 1) of its P = 32/b elements
 // (identity for 8-bit): evens in the low half-word, odds in the high half-word.  The 1-bit plane
 // of the 3-bit layout has its own order (hi_plane_pos): every high bit sits where one shift of
@@ -54,6 +55,8 @@ __device__ __forceinline__ void report(uint32_t* bad) {
     __hip_atomic_store(bad, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+constexpr int kPackThreads = 512;
+
 template <int NBITS>
 struct PackCfg {
     static constexpr int B = NBITS == 3 ? 2 : NBITS;           // field width of the main plane
@@ -61,6 +64,7 @@ struct PackCfg {
     static constexpr int UNIT = NBITS == 3 ? 32 : (P < 8 ? 8 : P);      // elements of K per thread and pass
     static constexpr int UW = UNIT / P;                        // main-plane words per unit
     static constexpr int WORDS = 32;                           // main-plane words of a block
+    static constexpr int COLS = kPackThreads / 4;              // its columns: sixteen units of K side by side
     static constexpr int PASSES = WORDS / UW / 16;
     static constexpr int KB = WORDS * P;                       // elements of K of a block
     static constexpr int HI = NBITS == 3 ? WORDS / 2 : 0;      // 1-bit-plane words of a block
@@ -72,9 +76,9 @@ template <int NBITS, bool VEC>
 __device__ __forceinline__ void pack_weight_tile(int64_t bx, int64_t by, const int32_t* __restrict__ weight, uint32_t* __restrict__ out,
                                                  int64_t K, int64_t N, uint32_t* __restrict__ bad) {
     using C = PackCfg<NBITS>;
-    __shared__ uint32_t tile[64][C::PITCH];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int64_t n0 = bx * 64, n = n0 + 4 * tx;
+    __shared__ uint32_t tile[C::COLS][C::PITCH];
+    const int tx = threadIdx.x % (C::COLS / 4), ty = threadIdx.x / (C::COLS / 4);
+    const int64_t n0 = bx * C::COLS, n = n0 + 4 * tx;
     const int64_t k_blk = by * C::KB;
     constexpr uint32_t MASK = (1u << NBITS) - 1u;
     uint32_t seen = 0;
@@ -115,13 +119,13 @@ __device__ __forceinline__ void pack_weight_tile(int64_t bx, int64_t by, const i
     __syncthreads();
     const int64_t row_words = K * NBITS / 32;
     const int64_t w0 = by * C::WORDS;
-    for (int i = threadIdx.x; i < 64 * C::WORDS; i += 256) {
+    for (int i = threadIdx.x; i < C::COLS * C::WORDS; i += kPackThreads) {
         const int r = i / C::WORDS, w = i % C::WORDS;
         if (n0 + r < N && w0 + w < K / C::P) out[(n0 + r) * row_words + w0 + w] = tile[r][w];
     }
     if constexpr (NBITS == 3) {                                 // the 1-bit plane behind the row's 2-bit plane
         const int64_t h0 = by * C::HI;
-        for (int i = threadIdx.x; i < 64 * C::HI; i += 256) {
+        for (int i = threadIdx.x; i < C::COLS * C::HI; i += kPackThreads) {
             const int r = i / C::HI, w = i % C::HI;
             if (n0 + r < N && h0 + w < K / 32) out[(n0 + r) * row_words + K / 16 + h0 + w] = tile[r][C::WORDS + w];
         }
@@ -132,7 +136,7 @@ __device__ __forceinline__ void pack_zero_tile(int64_t block, const int32_t* __r
                                                int64_t G, int64_t N, int nbits, int fb, uint32_t* __restrict__ bad) {
     const int p8 = 8 / fb;
     const int64_t row_bytes = G / p8;
-    const int64_t idx = block * 256 + threadIdx.x;      // over N * row_bytes, n fastest
+    const int64_t idx = block * kPackThreads + threadIdx.x;      // over N * row_bytes, n fastest
     if (idx >= N * row_bytes) return;
     const int64_t n = idx % N, byte = idx / N;
     const int32_t maxv = (1 << nbits) - 1;
@@ -151,12 +155,12 @@ __device__ __forceinline__ void pack_zero_tile(int64_t block, const int32_t* __r
 __device__ __forceinline__ void transpose_u16_tile(int64_t bx, int64_t by, const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
                                                    int64_t G, int64_t N) {
     __shared__ uint16_t tile[32][33];
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;           // 32 x 8
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;           // 32 x 16
     const int64_t n0 = bx * 32, g0 = by * 32;
-    for (int r = ty; r < 32; r += 8)
+    for (int r = ty; r < 32; r += kPackThreads / 32)
         if (g0 + r < G && n0 + tx < N) tile[r][tx] = in[(g0 + r) * N + n0 + tx];
     __syncthreads();
-    for (int r = ty; r < 32; r += 8)
+    for (int r = ty; r < 32; r += kPackThreads / 32)
         if (n0 + r < N && g0 + tx < G) out[(n0 + r) * G + g0 + tx] = tile[tx][r];
 }
 
@@ -174,7 +178,7 @@ struct PackJob {
 };
 
 template <int NBITS, bool VEC>
-__global__ __launch_bounds__(256) void pack_layer_kernel(PackJob j) {
+__global__ __launch_bounds__(kPackThreads) void pack_layer_kernel(PackJob j) {
     unsigned b = blockIdx.x;
     if (b < j.scale_blocks) {
         const unsigned columns = (unsigned)((j.N + 31) / 32);
@@ -187,21 +191,21 @@ __global__ __launch_bounds__(256) void pack_layer_kernel(PackJob j) {
         return;
     }
     b -= j.zero_blocks;
-    const unsigned columns = (unsigned)((j.N + 63) / 64);
+    const unsigned columns = (unsigned)((j.N + PackCfg<NBITS>::COLS - 1) / PackCfg<NBITS>::COLS);
     pack_weight_tile<NBITS, VEC>(b % columns, b / columns, j.weight, j.w_out, j.K, j.N, j.bad);
 }
 
 template <int NBITS>
 int launch_layer(const char* fn, PackJob j, hipStream_t stream) {
-    const int64_t weight_blocks = j.weight ? (j.N + 63) / 64 * ((j.K + PackCfg<NBITS>::KB - 1) / PackCfg<NBITS>::KB) : 0;
+    const int64_t weight_blocks = j.weight ? (j.N + PackCfg<NBITS>::COLS - 1) / PackCfg<NBITS>::COLS * ((j.K + PackCfg<NBITS>::KB - 1) / PackCfg<NBITS>::KB) : 0;
     const int64_t scale_blocks = j.scale ? (j.N + 31) / 32 * ((j.G + 31) / 32) : 0;
-    const int64_t zero_blocks = j.zero ? (j.N * (j.G / (8 / j.fb)) + 255) / 256 : 0;
+    const int64_t zero_blocks = j.zero ? (j.N * (j.G / (8 / j.fb)) + kPackThreads - 1) / kPackThreads : 0;
     if (weight_blocks + scale_blocks + zero_blocks > 0x7fffffff) return fail(fn, "too many blocks");
     j.scale_blocks = (unsigned)scale_blocks;
     j.zero_blocks = (unsigned)zero_blocks;
     const bool vec = j.N % 4 == 0 && (uintptr_t)j.weight % 16 == 0;
     hipLaunchKernelGGL((vec ? pack_layer_kernel<NBITS, true> : pack_layer_kernel<NBITS, false>),
-                       dim3((unsigned)(weight_blocks + scale_blocks + zero_blocks)), dim3(256), 0, stream, j);
+                       dim3((unsigned)(weight_blocks + scale_blocks + zero_blocks)), dim3(kPackThreads), 0, stream, j);
     return launched(fn);
 }
 
