@@ -83,8 +83,11 @@ def load():
 
 
 def _stream():
+    """Handle of the current device's current HIP stream, by the C-level query: ``torch.cuda.current_stream()`` builds a
+    Python object on every call (2.9 us of the 15 that a repacking call spent on the host in front of its launch)."""
     import torch
-    return torch.cuda.current_stream().cuda_stream
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return raw(torch.cuda.current_device()) if raw is not None else torch.cuda.current_stream().cuda_stream
 
 
 def _check(rc, what):
