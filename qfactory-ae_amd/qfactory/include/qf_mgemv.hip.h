@@ -285,27 +285,19 @@ __global__ __launch_bounds__(C::THREADS) void mgemv_kernel(
         // behind the LDS round trips below they would each expose a full L2 latency), then the
         // chunks pass through the wave's LDS buffer one after another
         constexpr int LPC = 16 / RPIA;                   // loads per chunk
-        // A lane whose row or chunk is not the wave's reads past the end of the buffer: it gets zeros and asks memory for
-        // nothing, and the address is 32 bits.  Against 64-bit addresses clamped to the last row (which moved all 16 rows
-        // through the L1 of every CU whatever the launch had) and zeroed afterwards: 4096 x 11008 at 4 / 8 / 16 rows 9.1 / 9.3 /
-        // 9.6 -> 8.7 / 8.7 / 9.1 us, 4096 x 4096 at 20 rows 7.0 -> 6.5, 8192 x 8192 at 2 bits and 4 rows 10.9 -> 10.6, at 3 bits and 5
-        // rows 13.3 -> 12.5; layers of 12288 columns and more level.
-        const int m_here = min(m_total - m0, C::BM);
-        const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(A + (size_t)m0 * C::K), 0, m_here * C::K * 2, 0x00020000);
         u32x4 raw[MT16][CH][LPC];
 #pragma unroll
         for (int mt = 0; mt < MT16; mt++)
 #pragma unroll
-            for (int c = 0; c < CH; c++) {
-                const bool own = (lo + c >= own_from) && (lo + c < min(own_from + CH, own_end));
+            for (int c = 0; c < CH; c++)
 #pragma unroll
                 for (int i = 0; i < LPC; i++) {
-                    const int m = 16 * mt + i * RPIA + lane / LPRA;
-                    const uint32_t at = own && m < m_here ? (uint32_t)(m * C::K + (lo + c) * CHUNK + (lane % LPRA) * 8) * 2u : 0xFFFFFFF0u;
+                    const int row = i * RPIA + lane / LPRA;
+                    const int m = m0 + 16 * mt + row;
+                    const uint16_t* ap = A + (size_t)min(m, m_total - 1) * C::K + (size_t)(lo + c) * CHUNK + (lane % LPRA) * 8;
                     if (QF_MGEMV_EXPERIMENT & 1) raw[mt][c][i] = u32x4{(uint32_t)lane, 1u, 2u, 3u};
-                    else raw[mt][c][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rows, at, 0, 0));
+                    else raw[mt][c][i] = *reinterpret_cast<const u32x4*>(ap);
                 }
-            }
 #if QF_MGEMV_PIN_FIRST_LOADS
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -403,9 +395,15 @@ __global__ __launch_bounds__(C::THREADS) void mgemv_kernel(
         for (int mt = 0; mt < MT16; mt++) {
 #pragma unroll
             for (int c = 0; c < CH; c++) {
+                const bool own = (lo + c >= own_from) && (lo + c < min(own_from + CH, own_end));
 #pragma unroll
-                for (int i = 0; i < LPC; i++)
-                    *reinterpret_cast<u32x4*>(wbuf + (i * RPIA + lane / LPRA) * PITCH_A + (lane % LPRA) * 16) = act_unit(raw[mt][c][i]);
+                for (int i = 0; i < LPC; i++) {
+                    const int row = i * RPIA + lane / LPRA;
+                    const int m = m0 + 16 * mt + row;
+                    u32x4 v = act_unit(raw[mt][c][i]);
+                    if (!(own && m < m_total)) v = u32x4{0, 0, 0, 0};
+                    *reinterpret_cast<u32x4*>(wbuf + row * PITCH_A + (lane % LPRA) * 16) = v;
+                }
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
                 for (int t = 0; t < KSTEPS; t++)
