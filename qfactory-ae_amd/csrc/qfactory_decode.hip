@@ -233,7 +233,7 @@ template <int V> struct Tag { static constexpr int value = V; };
 // takes as many as the sequence has (its position is known on the device only, so all forms are in the one kernel): stages
 // past the end cost requests, registers and arithmetic, and only the last stage has to look for the end of the sequence.
 // 32 heads of 128, cold caches, against eight stages for every sequence: 190 positions at batch 1 / 16 / 64 4.85 / 11.8 / 36.0
-// -> 4.24 / 11.3 / 35.7 us, 60 positions at batch 96 26.6 -> 19.4; past 256 positions level.
+// -> 4.24 / 11.3 / 35.7 us, 60 positions at batch 96 26.6 -> 19.4.
 template <int LPK, bool FUSED, int THREADS, int MOST>
 __global__ __launch_bounds__(THREADS) void decode_attention_kernel(const f16* __restrict__ q_or_qkv, f16* __restrict__ k_cache,
                                                                         f16* __restrict__ v_cache, const int64_t* __restrict__ pos_ptr,
@@ -352,11 +352,14 @@ __global__ __launch_bounds__(THREADS) void decode_attention_kernel(const f16* __
                 }
             }
         }
+        // The positions behind the stages.  The new one is the last of its group's and served from LDS behind the loop: looked for
+        // in the loop, the compiler put branches around the loads.  32 heads of 128, batch 1, 500 / 900 / 2000 / 4000 positions
+        // 8.5 / 17.9 / 43.1 / 83.6 -> 8.0 / 16.5 / 39.2 / 75.2 us, batch 4 at 2000 43.7 -> 39.9, 16 at 900 41.1 -> 40.7.
+        if constexpr (PRE == MOST) {
 #pragma unroll 2
-        for (int p = g + PRE * GROUPS; p < n; p += GROUPS) {
-            const bool fresh = FUSED && p == (int)pos;
-            visit(fresh ? *reinterpret_cast<const f16x8*>(new_k + j * 8) : row_of(kc, p),
-                  fresh ? *reinterpret_cast<const f16x8*>(new_v + j * 8) : row_of(vc, p));
+            for (int p = g + PRE * GROUPS; p < (FUSED ? n - 1 : n); p += GROUPS) visit(row_of(kc, p), row_of(vc, p));
+            if (FUSED && n > PRE * GROUPS && (n - 1) % GROUPS == g)
+                visit(*reinterpret_cast<const f16x8*>(new_k + j * 8), *reinterpret_cast<const f16x8*>(new_v + j * 8));
         }
         // merge the 64/LPK groups of a wave (lanes that differ in the bits above log2(LPK)) ...
 #pragma unroll
