@@ -28,6 +28,18 @@ int qf_pack_layer(const int32_t* weight, int8_t* w_out, const uint16_t* scale, u
 int qf_prefill_attention(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, const int64_t* pos, uint16_t* out,
                          int64_t batch, int64_t tokens, int64_t heads, int64_t head_dim, int64_t max_len, void* stream);
 
+/*
+ * qf_decode_attention and qf_rope_decode_attention with the number of launches of this shape, each on caches of its own, that lie between
+ * one launch on these caches and the next: the layers of the model (0: not known, taken as 8).  Where the rows that they read together
+ * are more than the 256 MB of the Infinity Cache, they are loaded past it.  The results are the same.
+ */
+int qf_decode_attention_layers(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, const int64_t* pos,
+                               uint16_t* out, int64_t batch, int64_t heads, int64_t head_dim, int64_t max_len, int64_t layers,
+                               void* stream);
+int qf_rope_decode_attention_layers(const uint16_t* qkv, const int64_t* pos, const float* cos_table, const float* sin_table,
+                                    uint16_t* k_cache, uint16_t* v_cache, uint16_t* out, int64_t batch, int64_t heads,
+                                    int64_t head_dim, int64_t max_len, int64_t layers, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

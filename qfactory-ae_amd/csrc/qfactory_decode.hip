@@ -10,6 +10,7 @@
 #include <stdint.h>
 
 #include "qfactory_hip.h"
+#include "qfactory_hip_ext.h"
 
 namespace {
 
@@ -175,7 +176,9 @@ __global__ __launch_bounds__(kThreads) void rope_kv_store_kernel(const f16* __re
 // costs 4.0 us before it touches the cache (the position, then the new token's q / k / v, then the stores: three
 // dependent round trips behind a 1.7 us launch).
 constexpr int kAttnThreads = 512;
-constexpr int64_t kReadOnceBytes = 32 << 20;
+constexpr int64_t kCacheBytes = 256 << 20;      // the Infinity Cache
+constexpr int64_t kMostLayers = 1 << 20;
+constexpr int kUsualLayers = 8;                 // where the caller does not say how many
 constexpr int kAttnPrefetch = 8;          // positions per group requested up front at most (256 at 128-wide heads)
 
 __device__ __forceinline__ f16x8 rotate8(const f16x8 x, const float* __restrict__ c, const float* __restrict__ s) {
@@ -238,7 +241,7 @@ template <int LPK, bool FUSED, int THREADS, int MOST>
 __global__ __launch_bounds__(THREADS) void decode_attention_kernel(const f16* __restrict__ q_or_qkv, f16* __restrict__ k_cache,
                                                                         f16* __restrict__ v_cache, const int64_t* __restrict__ pos_ptr,
                                                                         const float* __restrict__ cos_t, const float* __restrict__ sin_t,
-                                                                        f16* __restrict__ out, int heads, int max_len, float scale) {
+                                                                        f16* __restrict__ out, int heads, int max_len, float scale, int once_from) {
     constexpr int HD = LPK * 8;
     constexpr int GROUPS = THREADS / LPK;
     constexpr int WAVES = THREADS / 64;
@@ -409,11 +412,9 @@ __global__ __launch_bounds__(THREADS) void decode_attention_kernel(const f16* __
             default: attend(Tag<8>{}, once_tag);
         }
     };
-    // From 32 MB of cache rows a launch (256 MB in eight layers, what the Infinity Cache holds) they are marked as read once:
-    // rows that will not be there at the next step are faster when they pass it by, rows that will be are not.  Cold caches, 190
-    // positions at batch 16 / 64 11.3 / 35.9 -> 10.4 / 32.0 us (6.3 TB/s), 60 at batch 96 24.4 -> 22.4, 700 at batch 32 69.7 -> 64.5;
-    // a decode step of one sequence, whose eight layers' 25 MB stay, 280 us without and 285 with.
-    if ((int64_t)gridDim.x * gridDim.y * n * HD * 4 >= kReadOnceBytes) attend_in_stages(Tag<1>{});
+    // Rows that will not be in the Infinity Cache at the next step are faster when they pass it by, rows that will be are not; the
+    // line is read_once_from.
+    if (n >= once_from) attend_in_stages(Tag<1>{});
     else attend_in_stages(Tag<0>{});
 }
 
@@ -493,31 +494,45 @@ __global__ __launch_bounds__(kPickThreads) void greedy_next_kernel(const f16* __
     }
 }
 
+// Length of the sequences from which their cache rows are marked as read once: where the rows of all `layers` launches of a
+// step are more than the Infinity Cache holds.  Decode steps of a 7B shape, 32 heads of 128, rows cached / read once in us: 96 ...
+// 190 MB of rows in 2, 4, 8 or 32 layers 236 / 239 (12 sequences, 4 layers), 150 / 167 (4 at 1500 positions, 2 layers), 402 / 472 (one
+// at 1500, 8 layers), 1062 / 1068 (one at 190, 32 layers); 191 ... 256 MB within 1 % (16 at 800 in one layer 101 / 104); 286 and more 1520 / 1501 (3
+// sequences, 32 layers), 1607 / 1562 (8), 480 / 465 (16, 8 layers), 884 / 854 (64).  Above 32 sequences the projections' weights go through that
+// cache too, and one or two layers lose 3 - 7 % below the line (64 sequences in one layer 140 / 131).
+int read_once_from(int64_t batch, int64_t heads, int64_t head_dim, int64_t layers) {
+    const int64_t position = batch * heads * head_dim * 4;
+    if (position >= kCacheBytes) return 1;
+    const int64_t step = position * (layers ? layers : kUsualLayers);
+    return (int)((kCacheBytes + step - 1) / step);
+}
+
 template <int LPK, bool FUSED>
 int launch_attention(const char* fn, const f16* q_or_qkv, f16* k, f16* v, const int64_t* pos, const float* cos_t, const float* sin_t,
-                     f16* out, int batch, int heads, int max_len, hipStream_t stream) {
+                     f16* out, int batch, int heads, int max_len, int64_t layers, hipStream_t stream) {
     constexpr int HD = LPK * 8;
     const float scale = 1.0f / sqrtf((float)HD);
     hipLaunchKernelGGL((decode_attention_kernel<LPK, FUSED, kAttnThreads, kAttnPrefetch>), dim3(heads, batch), dim3(kAttnThreads), 0,
-                       stream, q_or_qkv, k, v, pos, cos_t, sin_t, out, heads, max_len, scale);
+                       stream, q_or_qkv, k, v, pos, cos_t, sin_t, out, heads, max_len, scale, read_once_from(batch, heads, HD, layers));
     return launched(fn);
 }
 
 template <bool FUSED>
 int dispatch_attention(const char* fn, const uint16_t* q_or_qkv, uint16_t* k_cache, uint16_t* v_cache, const int64_t* pos,
                        const float* cos_t, const float* sin_t, uint16_t* out, int64_t batch, int64_t heads, int64_t head_dim,
-                       int64_t max_len, void* stream) {
+                       int64_t max_len, int64_t layers, void* stream) {
     if (batch <= 0 || heads <= 0 || max_len <= 0 || batch > 65535 || heads > 0x7fffffff || max_len > 0x7fffffff)
         return fail(fn, "batch in 1..65535, heads and max_len positive");
+    if (layers < 0 || layers > kMostLayers) return fail(fn, "layers in 0..1048576");
     const f16* qp = (const f16*)q_or_qkv;
     f16 *kp = (f16*)k_cache, *vp = (f16*)v_cache, *op = (f16*)out;
     hipStream_t s = (hipStream_t)stream;
     const int B = (int)batch, H = (int)heads, L = (int)max_len;
     switch (head_dim) {
-        case 32: return launch_attention<4, FUSED>(fn, qp, kp, vp, pos, cos_t, sin_t, op, B, H, L, s);
-        case 64: return launch_attention<8, FUSED>(fn, qp, kp, vp, pos, cos_t, sin_t, op, B, H, L, s);
-        case 128: return launch_attention<16, FUSED>(fn, qp, kp, vp, pos, cos_t, sin_t, op, B, H, L, s);
-        case 256: return launch_attention<32, FUSED>(fn, qp, kp, vp, pos, cos_t, sin_t, op, B, H, L, s);
+        case 32: return launch_attention<4, FUSED>(fn, qp, kp, vp, pos, cos_t, sin_t, op, B, H, L, layers, s);
+        case 64: return launch_attention<8, FUSED>(fn, qp, kp, vp, pos, cos_t, sin_t, op, B, H, L, layers, s);
+        case 128: return launch_attention<16, FUSED>(fn, qp, kp, vp, pos, cos_t, sin_t, op, B, H, L, layers, s);
+        case 256: return launch_attention<32, FUSED>(fn, qp, kp, vp, pos, cos_t, sin_t, op, B, H, L, layers, s);
         default: return fail(fn, "head_dim must be 32, 64, 128 or 256");
     }
 }
@@ -568,20 +583,32 @@ extern "C" int qf_rope_kv_store_rows(const uint16_t* qkv, const int64_t* pos, co
     return launched("qf_rope_kv_store_rows");
 }
 
-extern "C" int qf_decode_attention(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, const int64_t* pos,
-                                   uint16_t* out, int64_t batch, int64_t heads, int64_t head_dim, int64_t max_len, void* stream) {
+extern "C" int qf_decode_attention_layers(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, const int64_t* pos,
+                                          uint16_t* out, int64_t batch, int64_t heads, int64_t head_dim, int64_t max_len,
+                                          int64_t layers, void* stream) {
     if (!q || !k_cache || !v_cache || !pos || !out) return fail("qf_decode_attention", "null pointer");
     // the caches are only read on this path
     return dispatch_attention<false>("qf_decode_attention", q, const_cast<uint16_t*>(k_cache), const_cast<uint16_t*>(v_cache), pos,
-                                     nullptr, nullptr, out, batch, heads, head_dim, max_len, stream);
+                                     nullptr, nullptr, out, batch, heads, head_dim, max_len, layers, stream);
+}
+
+extern "C" int qf_decode_attention(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, const int64_t* pos,
+                                   uint16_t* out, int64_t batch, int64_t heads, int64_t head_dim, int64_t max_len, void* stream) {
+    return qf_decode_attention_layers(q, k_cache, v_cache, pos, out, batch, heads, head_dim, max_len, 0, stream);
+}
+
+extern "C" int qf_rope_decode_attention_layers(const uint16_t* qkv, const int64_t* pos, const float* cos_table, const float* sin_table,
+                                               uint16_t* k_cache, uint16_t* v_cache, uint16_t* out, int64_t batch, int64_t heads,
+                                               int64_t head_dim, int64_t max_len, int64_t layers, void* stream) {
+    if (!qkv || !pos || !cos_table || !sin_table || !k_cache || !v_cache || !out) return fail("qf_rope_decode_attention", "null pointer");
+    return dispatch_attention<true>("qf_rope_decode_attention", qkv, k_cache, v_cache, pos, cos_table, sin_table, out, batch, heads,
+                                    head_dim, max_len, layers, stream);
 }
 
 extern "C" int qf_rope_decode_attention(const uint16_t* qkv, const int64_t* pos, const float* cos_table, const float* sin_table,
                                         uint16_t* k_cache, uint16_t* v_cache, uint16_t* out, int64_t batch, int64_t heads,
                                         int64_t head_dim, int64_t max_len, void* stream) {
-    if (!qkv || !pos || !cos_table || !sin_table || !k_cache || !v_cache || !out) return fail("qf_rope_decode_attention", "null pointer");
-    return dispatch_attention<true>("qf_rope_decode_attention", qkv, k_cache, v_cache, pos, cos_table, sin_table, out, batch, heads,
-                                    head_dim, max_len, stream);
+    return qf_rope_decode_attention_layers(qkv, pos, cos_table, sin_table, k_cache, v_cache, out, batch, heads, head_dim, max_len, 0, stream);
 }
 
 extern "C" int qf_silu_mul(const uint16_t* gate_up, uint16_t* out, int64_t rows, int64_t mlp, void* stream) {

@@ -206,7 +206,7 @@ class QuantLlama:
             # and the qkv and gate+up projections normalise it in front of their dot products
             for li, layer in enumerate(self.layers):
                 qkv = layer["qkv"].forward_add_rmsnorm(x, None, layer["norm1"], shape.eps)
-                native.rope_decode_attention(qkv, pos, self.cos, self.sin, self.k_cache[li], self.v_cache[li], self._att)
+                native.rope_decode_attention(qkv, pos, self.cos, self.sin, self.k_cache[li], self.v_cache[li], self._att, shape.layers)
                 layer["o"].forward_accumulate(self._att, x)
                 act = layer["gate_up"].forward_add_rmsnorm(x, None, layer["norm2"], shape.eps, silu_mul=True)
                 layer["down"].forward_accumulate(act, x)
@@ -218,7 +218,7 @@ class QuantLlama:
             for li, layer in enumerate(self.layers):
                 native.add_rmsnorm(x, None, layer["norm1"], self._hdn, shape.eps)
                 qkv = layer["qkv"](self._hdn)
-                native.rope_decode_attention(qkv, pos, self.cos, self.sin, self.k_cache[li], self.v_cache[li], self._att)
+                native.rope_decode_attention(qkv, pos, self.cos, self.sin, self.k_cache[li], self.v_cache[li], self._att, shape.layers)
                 layer["o"].forward_accumulate(self._att, x)
                 native.add_rmsnorm(x, None, layer["norm2"], self._hdn, shape.eps)
                 layer["down"].forward_accumulate(layer["gate_up"].forward_silu_mul(self._hdn), x)
@@ -227,7 +227,7 @@ class QuantLlama:
         for li, layer in enumerate(self.layers):
             native.add_rmsnorm(x, delta, layer["norm1"], self._hdn, shape.eps)
             qkv = self.linear(layer["qkv"], self._hdn)
-            native.rope_decode_attention(qkv, pos, self.cos, self.sin, self.k_cache[li], self.v_cache[li], self._att)
+            native.rope_decode_attention(qkv, pos, self.cos, self.sin, self.k_cache[li], self.v_cache[li], self._att, shape.layers)
             delta = self.linear(layer["o"], self._att)
             native.add_rmsnorm(x, delta, layer["norm2"], self._hdn, shape.eps)
             # SiLU(gate) * up: in the gate+up projection's final sum for few rows, else one launch behind it
