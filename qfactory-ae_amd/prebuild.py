@@ -354,7 +354,7 @@ def wide_cases():
         # fewer steps per iteration and groups than the table's form
         (70, 100, 1152, 8, 64, False, (1, 3, 2, 1, 1, 2)), (49, 72, 1408, 8, 64, True, (1, 2, 2, 1, 1, 2)),
         (39, 40, 896, 8, 32, False, (1, 2, 1, 1, 1, 2)), (34, 36, 1152, 8, 64, False, (1, 1, 1, 1, 1, 4)),
-        (66, 130, 1280, 4, 128, False, (1, 4, 2, 1, 1, 1))]] + [_case(256, 12288, 1024)]
+        (66, 130, 1280, 4, 128, False, (1, 4, 2, 1, 1, 1))]] + [_case(256, 12288, 1024), _case(32, 33281, 4608)]
 
 
 def search_cases():

@@ -866,11 +866,16 @@ GEMM_WIDE_COST_8BIT = {(1, 7, 1, 1, 2, 1): 0.528}
 # 2240 x 1792, seven windows, 12.5 -> 13.4.
 GEMM_WIDE_PAIR_WINDOWS = 6
 GEMM_WIDE_MIN_M = 17           # the 32-row bucket: 9280 x 4608 at 2 bits 13.9 -> 11.6 us, 8192 x 28672 49.8 -> 46.3, 8192 x 8192 level
-# ... but not in more than one and up to two and a half rounds of 32 x 64 blocks there: its blocks fill a CU's LDS, so a second round
-# starts when the first has ended, where the other kernel's smaller blocks share CUs.  Other kernel against this one, 24 rows:
-# 19008 x 14592 at 4 bits 54.9 against 65.4 us, 24576 x 4352 21.4 / 24.4, 23552 x 11776 at 8 bits 80.4 / 89.0; of random problems
-# at 17 - 32 rows 26 of 28 in that range took longer here (up to 21 %), four of five past 2.5 rounds 9 - 10 % less.
-GEMM_WIDE_NOT_AT_32 = (NUM_CUS, 2.5 * NUM_CUS)
+# ... but not in more than one and up to two rounds of 32 x 64 blocks there: its blocks fill a CU's LDS, so a second round
+# starts when the first has ended, where the other kernel's smaller blocks share CUs.  That kernel against this one, 17 / 24 / 32 rows on
+# 17 ... 32 thousand columns: 4 bits 4 - 15 % less time on seven shapes of seven (24576 x 8192 32.8 / 33.0 / 33.4 against 37.5 / 38.2 /
+# 38.8 us); 8 bits from 9 % less (21808 x 20992) to 10 % more (24192 x 7936), 2 bits from 3 % less to 13 % more.
+# Past two rounds this one takes less time at every width, as 32 x 224 at 2 and 4 bits (one round up to 57344 columns; 36864 x 4608
+# 32.2 / 33.2 / 34.1 against 29.9 / 29.6 / 29.8, 34816 x 14336 94.4 / 98.1 / 104.0 against 84.6 / 84.1 / 84.7), as 32 x 64 at 8 bits (38400 x
+# 8192 94.8 / 98.9 / 103.2 against 84.7 / 87.1 / 90.0): 33 shapes at 4 bits 0 - 21 %, ten at 2 bits 15 - 19 %, 25 at 8 bits 7 - 22 %.
+# Rows shorter than 4608 (4352 alone at 4 bits, 4 - 13 %) keep a line of two and a half rounds.
+GEMM_WIDE_NOT_AT_32 = (NUM_CUS, 2 * NUM_CUS)
+GEMM_WIDE_NOT_AT_32_SHORT = (4608, 2.5 * NUM_CUS)
 
 
 def gemm_wide_lds_bytes(cfg, nbits):
@@ -961,7 +966,10 @@ def _gemm_wide_tiling(M, N, K, nbits, group_size):
         cost = (0.6 * whole + 0.4 * exact) * per_step
         if best is None or cost < best[0]:
             best = (cost, cfg)
-    if best is None or (M <= 32 and GEMM_WIDE_NOT_AT_32[0] < -(-N // 64) <= GEMM_WIDE_NOT_AT_32[1]):
+    few, many = GEMM_WIDE_NOT_AT_32
+    if K < GEMM_WIDE_NOT_AT_32_SHORT[0]:
+        many = GEMM_WIDE_NOT_AT_32_SHORT[1]
+    if best is None or (M <= 32 and few < -(-N // 64) <= many):
         return None
     return best[1]
 

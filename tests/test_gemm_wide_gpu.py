@@ -55,6 +55,22 @@ def test_tilings_at_their_edges(oracle, case):
         assert torch.equal(first[:rows], store[:rows]) and store[rows:].isnan().all()
 
 
+def test_the_widest_layers_of_17_to_32_rows(oracle):
+    """More columns than two rounds of 32 x 64 blocks, the last of 149 tiles 129 columns wide: the layer's own launch, against the
+    oracle at the ends of the first and the last tiles."""
+    from qfactory import QLinear
+    from qfactory.core import tiling
+    N, K = 33281, 4608
+    assert tiling.gemm_wide_tiling(32, N, K, 4, 128)["WN"] == 7
+    A, weight, scale, zero = make_problem(7, 32, N, K, 4, 128)
+    layer = QLinear.init(32, K, N, 4, weight.cuda(), 128, scale.cuda(), zero.cuda(), compile_flags=NO_SEARCH)
+    rows = [*range(230), *range(N - 360, N)]
+    want = reference_output(oracle, A, layer.w, layer.s, layer.z, 4, 128, rows=rows)
+    whole = layer(A.cuda())
+    assert_close(oracle, whole.cpu().numpy()[:, rows], want, "32 rows")
+    assert torch.equal(layer(A[:17].cuda()), whole[:17])
+
+
 def test_every_tiling_of_a_search(oracle):
     """All candidates of a search on a ragged problem (windows of K that do not deal evenly over the groups among them)
     against the oracle: a search may pick any."""

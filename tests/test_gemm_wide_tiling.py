@@ -43,6 +43,18 @@ def test_where_the_rule_takes_over():
         assert "qf::GemmWideCfg<" in q.emit()
 
 
+@pytest.mark.parametrize("K", [4608, 5120, 8192, 14336])
+@pytest.mark.parametrize("nbits", [2, 4, 8])
+def test_at_32_rows_only_two_rounds_of_blocks_stay_on_the_other_kernel(nbits, K):
+    """More than two rounds of 32 x 64 blocks are one round of 32 x 224 at 2 and 4 bits: nothing there waits for a first round to end."""
+    from qfactory.core import tiling
+    for N in (16385, 24576, 32768):
+        assert tiling.gemm_wide_tiling(32, N, K, nbits, 128) is None
+    for N in (16384, 32769, 33280, 36864, 40960):
+        t = tiling.gemm_wide_tiling(32, N, K, nbits, 128)
+        assert t is not None and 32 * t["NT"] * t["WN"] == (64 if nbits == 8 or N == 16384 else 224), (N, t)
+
+
 def _qfunc(M, N, K, nbits, gs):
     import torch
     from qfactory.core.qfunc import QMatmulQFunc
