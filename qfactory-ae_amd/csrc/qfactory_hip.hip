@@ -26,9 +26,9 @@ int launched(const char* fn) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Weight repack, bound by memory: four bytes are read per field.  A block takes 128 columns n and 32 main-plane words
-// of K (32 threads x 4 columns side by side, 16 units of K): a thread reads 16 bytes of every k of its unit -- 512
-// contiguous bytes per k and 32 threads -- builds four columns' words in registers, and the words change their orientation
+// Weight repack, bound by memory: four bytes are read per field.  A block takes 128 columns n (64 of a small layer)
+// and 32 main-plane words of K (32 threads x 4 columns side by side, 16 units of K): a thread reads 16 bytes of every k of its
+// unit -- 512 contiguous bytes per k and 32 threads -- builds four columns' words in registers, and the words change their orientation
 // through LDS, so that a row of the output is written 128 bytes at a time.  (A 4-byte word per thread straight to its row left
 // 32-byte pieces: 22016 x 4096 at 4 bits 102 us = 4.0 TB/s.  Through LDS by columns of a block, 22016 x 4096 / 4096 x 4096 / 8192 x
 // 28672 at 4 bits: 32 columns 81 / 16.7 / 210 us, 64 73 / 15.1 / 190, 128 with 256 threads 71 / 14.1 / 183, 128 with 512 70.6 / 13.8 /
@@ -55,16 +55,15 @@ __device__ __forceinline__ void report(uint32_t* bad) {
     __hip_atomic_store(bad, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-constexpr int kPackThreads = 512;
-
-template <int NBITS>
+template <int NBITS_, int THREADS_>
 struct PackCfg {
+    static constexpr int NBITS = NBITS_, THREADS = THREADS_;
     static constexpr int B = NBITS == 3 ? 2 : NBITS;           // field width of the main plane
     static constexpr int P = 32 / B;                           // elements per main-plane word
     static constexpr int UNIT = NBITS == 3 ? 32 : (P < 8 ? 8 : P);      // elements of K per thread and pass
     static constexpr int UW = UNIT / P;                        // main-plane words per unit
     static constexpr int WORDS = 32;                           // main-plane words of a block
-    static constexpr int COLS = kPackThreads / 4;              // its columns: sixteen units of K side by side
+    static constexpr int COLS = THREADS / 4;              // its columns: sixteen units of K side by side
     static constexpr int PASSES = WORDS / UW / 16;
     static constexpr int KB = WORDS * P;                       // elements of K of a block
     static constexpr int HI = NBITS == 3 ? WORDS / 2 : 0;      // 1-bit-plane words of a block
@@ -72,10 +71,10 @@ struct PackCfg {
 };
 
 // VEC: N a multiple of four and 16-byte aligned rows, four columns per load; otherwise single words
-template <int NBITS, bool VEC>
+template <class C, bool VEC>
 __device__ __forceinline__ void pack_weight_tile(int64_t bx, int64_t by, const int32_t* __restrict__ weight, uint32_t* __restrict__ out,
                                                  int64_t K, int64_t N, uint32_t* __restrict__ bad) {
-    using C = PackCfg<NBITS>;
+    constexpr int NBITS = C::NBITS;
     __shared__ uint32_t tile[C::COLS][C::PITCH];
     const int tx = threadIdx.x % (C::COLS / 4), ty = threadIdx.x / (C::COLS / 4);
     const int64_t n0 = bx * C::COLS, n = n0 + 4 * tx;
@@ -119,24 +118,25 @@ __device__ __forceinline__ void pack_weight_tile(int64_t bx, int64_t by, const i
     __syncthreads();
     const int64_t row_words = K * NBITS / 32;
     const int64_t w0 = by * C::WORDS;
-    for (int i = threadIdx.x; i < C::COLS * C::WORDS; i += kPackThreads) {
+    for (int i = threadIdx.x; i < C::COLS * C::WORDS; i += C::THREADS) {
         const int r = i / C::WORDS, w = i % C::WORDS;
         if (n0 + r < N && w0 + w < K / C::P) out[(n0 + r) * row_words + w0 + w] = tile[r][w];
     }
     if constexpr (NBITS == 3) {                                 // the 1-bit plane behind the row's 2-bit plane
         const int64_t h0 = by * C::HI;
-        for (int i = threadIdx.x; i < C::COLS * C::HI; i += kPackThreads) {
+        for (int i = threadIdx.x; i < C::COLS * C::HI; i += C::THREADS) {
             const int r = i / C::HI, w = i % C::HI;
             if (n0 + r < N && h0 + w < K / 32) out[(n0 + r) * row_words + K / 16 + h0 + w] = tile[r][C::WORDS + w];
         }
     }
 }
 
+template <int THREADS>
 __device__ __forceinline__ void pack_zero_tile(int64_t block, const int32_t* __restrict__ zero, uint8_t* __restrict__ out,
                                                int64_t G, int64_t N, int nbits, int fb, uint32_t* __restrict__ bad) {
     const int p8 = 8 / fb;
     const int64_t row_bytes = G / p8;
-    const int64_t idx = block * kPackThreads + threadIdx.x;      // over N * row_bytes, n fastest
+    const int64_t idx = block * THREADS + threadIdx.x;      // over N * row_bytes, n fastest
     if (idx >= N * row_bytes) return;
     const int64_t n = idx % N, byte = idx / N;
     const int32_t maxv = (1 << nbits) - 1;
@@ -152,15 +152,16 @@ __device__ __forceinline__ void pack_zero_tile(int64_t block, const int32_t* __r
     if (bad != nullptr && (seen & ~(uint32_t)maxv) != 0) report(bad);
 }
 
+template <int THREADS>
 __device__ __forceinline__ void transpose_u16_tile(int64_t bx, int64_t by, const uint16_t* __restrict__ in, uint16_t* __restrict__ out,
                                                    int64_t G, int64_t N) {
     __shared__ uint16_t tile[32][33];
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;           // 32 x 16
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;           // 32 x THREADS / 32
     const int64_t n0 = bx * 32, g0 = by * 32;
-    for (int r = ty; r < 32; r += kPackThreads / 32)
+    for (int r = ty; r < 32; r += THREADS / 32)
         if (g0 + r < G && n0 + tx < N) tile[r][tx] = in[(g0 + r) * N + n0 + tx];
     __syncthreads();
-    for (int r = ty; r < 32; r += kPackThreads / 32)
+    for (int r = ty; r < 32; r += THREADS / 32)
         if (n0 + r < N && g0 + tx < G) out[(n0 + r) * G + g0 + tx] = tile[tx][r];
 }
 
@@ -177,36 +178,51 @@ struct PackJob {
     unsigned scale_blocks, zero_blocks;
 };
 
-template <int NBITS, bool VEC>
-__global__ __launch_bounds__(kPackThreads) void pack_layer_kernel(PackJob j) {
+template <class C, bool VEC>
+__global__ __launch_bounds__(C::THREADS) void pack_layer_kernel(PackJob j) {
     unsigned b = blockIdx.x;
     if (b < j.scale_blocks) {
         const unsigned columns = (unsigned)((j.N + 31) / 32);
-        transpose_u16_tile(b % columns, b / columns, j.scale, j.s_out, j.G, j.N);
+        transpose_u16_tile<C::THREADS>(b % columns, b / columns, j.scale, j.s_out, j.G, j.N);
         return;
     }
     b -= j.scale_blocks;
     if (b < j.zero_blocks) {
-        pack_zero_tile(b, j.zero, j.z_out, j.G, j.N, j.nbits, j.fb, j.bad);
+        pack_zero_tile<C::THREADS>(b, j.zero, j.z_out, j.G, j.N, j.nbits, j.fb, j.bad);
         return;
     }
     b -= j.zero_blocks;
-    const unsigned columns = (unsigned)((j.N + PackCfg<NBITS>::COLS - 1) / PackCfg<NBITS>::COLS);
-    pack_weight_tile<NBITS, VEC>(b % columns, b / columns, j.weight, j.w_out, j.K, j.N, j.bad);
+    const unsigned columns = (unsigned)((j.N + C::COLS - 1) / C::COLS);
+    pack_weight_tile<C, VEC>(b % columns, b / columns, j.weight, j.w_out, j.K, j.N, j.bad);
 }
 
-template <int NBITS>
-int launch_layer(const char* fn, PackJob j, hipStream_t stream) {
-    const int64_t weight_blocks = j.weight ? (j.N + PackCfg<NBITS>::COLS - 1) / PackCfg<NBITS>::COLS * ((j.K + PackCfg<NBITS>::KB - 1) / PackCfg<NBITS>::KB) : 0;
+template <class C>
+int64_t weight_blocks(const PackJob& j) {
+    return j.weight ? (j.N + C::COLS - 1) / C::COLS * ((j.K + C::KB - 1) / C::KB) : 0;
+}
+
+template <class C>
+int launch_blocks(const char* fn, PackJob j, hipStream_t stream) {
     const int64_t scale_blocks = j.scale ? (j.N + 31) / 32 * ((j.G + 31) / 32) : 0;
-    const int64_t zero_blocks = j.zero ? (j.N * (j.G / (8 / j.fb)) + kPackThreads - 1) / kPackThreads : 0;
-    if (weight_blocks + scale_blocks + zero_blocks > 0x7fffffff) return fail(fn, "too many blocks");
+    const int64_t zero_blocks = j.zero ? (j.N * (j.G / (8 / j.fb)) + C::THREADS - 1) / C::THREADS : 0;
+    const int64_t blocks = weight_blocks<C>(j) + scale_blocks + zero_blocks;
+    if (blocks > 0x7fffffff) return fail(fn, "too many blocks");
     j.scale_blocks = (unsigned)scale_blocks;
     j.zero_blocks = (unsigned)zero_blocks;
     const bool vec = j.N % 4 == 0 && (uintptr_t)j.weight % 16 == 0;
-    hipLaunchKernelGGL((vec ? pack_layer_kernel<NBITS, true> : pack_layer_kernel<NBITS, false>),
-                       dim3((unsigned)(weight_blocks + scale_blocks + zero_blocks)), dim3(kPackThreads), 0, stream, j);
+    hipLaunchKernelGGL((vec ? pack_layer_kernel<C, true> : pack_layer_kernel<C, false>), dim3((unsigned)blocks), dim3(C::THREADS), 0, stream, j);
     return launched(fn);
+}
+
+// Blocks of 128 columns for layers of more than 128 of them, of 64 for smaller ones, which leave CUs without work either way and
+// take as long as a block does.  64 / 128 columns, cold weights, scales and zero-points with them: 1024 x 1024 at 2 / 3 / 4 / 8 bits 5.9 / 6.3 /
+// 4.7 / 4.0 against 7.9 / 8.1 / 5.3 / 4.4 us, 4096 x 2048 (128 blocks but at 8 bits) 8.9 / 9.5 / 8.9 / 9.8 against 9.9 / 10.7 / 9.1 / 9.8; 4096 x 1100 at
+// 4 bits (144 blocks) 8.2 against 7.6, 4096 x 3072 at 2 / 3 / 4 / 8 bits (192 blocks at 2 and 3) 13.0 / 13.5 / 12.0 / 15.0 against 11.9 / 12.7 /
+// 13.1 / 14.2.
+template <int NBITS>
+int launch_layer(const char* fn, const PackJob& j, hipStream_t stream) {
+    return weight_blocks<PackCfg<NBITS, 512>>(j) <= 128 ? launch_blocks<PackCfg<NBITS, 256>>(fn, j, stream)
+                                                        : launch_blocks<PackCfg<NBITS, 512>>(fn, j, stream);
 }
 
 int launch_layer(const char* fn, const PackJob& j, hipStream_t stream) {

@@ -110,6 +110,14 @@ def test_weight_packer_at_the_edges_of_a_block(oracle, nbits, K, N, offset):
     test_weight_packer_at_tile_edges(oracle, nbits, K, N, offset)
 
 
+@pytest.mark.parametrize("nbits,k_block", [(2, 512), (3, 512), (4, 256), (8, 128)])
+@pytest.mark.parametrize("N,offset", [(132, 0), (129, 0), (252, 1), (256, 0)])
+def test_weight_packer_at_the_edges_of_wide_blocks(oracle, nbits, k_block, N, offset):
+    """Two by 64 blocks of 128 columns are still packed by 64 columns, two by 65 (the last block of K a part of one) by 128."""
+    for K in (64 * k_block, 64 * k_block + 32):
+        test_weight_packer_at_tile_edges(oracle, nbits, K, N, offset)
+
+
 @pytest.mark.parametrize("nbits", [2, 3, 4, 8])
 @pytest.mark.parametrize("value", ["top", "negative", "lowest", "highest"])
 def test_values_out_of_range_are_refused(nbits, value):

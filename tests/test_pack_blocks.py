@@ -1,0 +1,30 @@
+"""Which blocks a layer is packed by: 64 columns and 256 threads up to 128 blocks of 128 columns, 512 threads beyond.  The launch goes to
+a stand-in that prints it."""
+import os
+import subprocess
+import sys
+
+HIP_CALLS = r"""
+#include <stddef.h>
+#include <stdio.h>
+typedef struct { unsigned x, y, z; } dim3_;
+int __hipPushCallConfiguration(dim3_ g, dim3_ b, size_t lds, void* s) { (void)lds; (void)s; printf("%u %u\n", g.x, b.x); fflush(stdout); return 1; }
+int hipGetLastError(void) { return 0; }
+"""
+
+# (nbits, K, N) -> blocks, threads
+CASES = [((4, 1024, 1024), (16 * 4, 256)), ((2, 4096, 64), (8, 256)), ((2, 4096, 2048), (32 * 8, 256)), ((3, 4096, 2049), (17 * 8, 512)),
+         ((4, 4096, 1024), (16 * 16, 256)), ((4, 4128, 1024), (8 * 17, 512)), ((8, 4096, 1024), (8 * 32, 512)), ((4, 4096, 22016), (172 * 16, 512))]
+
+
+def test_small_layers_are_packed_by_narrow_blocks(tmp_path):
+    from qfactory import native
+    native.build()
+    (tmp_path / "calls.c").write_text(HIP_CALLS)
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "calls.c"), "-o", str(tmp_path / "calls.so")], check=True)
+    probe = ("import ctypes; from ctypes import c_int64 as I, c_void_p as P; lib = ctypes.CDLL(%r)\n"
+             "for nbits, K, N in %r:\n assert lib.qf_pack_weight(P(16), P(16), I(K), I(N), nbits, None) == 0\n")
+    out = subprocess.run([sys.executable, "-c", probe % (native.LIBRARY, [case for case, _ in CASES])],
+                         env=dict(os.environ, LD_PRELOAD=str(tmp_path / "calls.so")), check=True, capture_output=True, text=True,
+                         timeout=120).stdout.splitlines()
+    assert out == [f"{blocks} {threads}" for _, (blocks, threads) in CASES]
