@@ -30,7 +30,7 @@ int qf_prefill_attention(const uint16_t* q, const uint16_t* k_cache, const uint1
 
 /*
  * qf_decode_attention and qf_rope_decode_attention with the number of launches of this shape, each on caches of its own, that lie between
- * one launch on these caches and the next: the layers of the model (0: not known, taken as 8).  Where the rows that they read together
+ * one launch on these caches and the next: the layers of the model (0: not known).  Where the rows that they read together
  * are more than the 256 MB of the Infinity Cache, they are loaded past it.  The results are the same.
  */
 int qf_decode_attention_layers(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, const int64_t* pos,

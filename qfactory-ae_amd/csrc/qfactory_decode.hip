@@ -155,31 +155,24 @@ __global__ __launch_bounds__(kThreads) void rope_kv_store_kernel(const f16* __re
 }
 
 // ---------------------------------------------------------------------------------------------
-// Attention of one query per (sequence, head) over cache positions 0 .. pos, one block of 16 or 4 waves per
-// (head, sequence).  LPK = hd/8 lanes share a key or value row (16 bytes each), so a block covers
-// 1024/LPK or 256/LPK positions per pass.  One pass over the cache: every group of LPK lanes walks its share of
-// the positions with a running maximum (key and value row requested together), the groups of a wave are merged
-// by lane shuffles, the waves through LDS.
+// Attention of one query per (sequence, head) over cache positions 0 .. pos, one block of 8 waves per (head, sequence).
+// LPK = hd/8 lanes share a key or value row (16 bytes each), so a block covers 512/LPK positions per stage.  One pass over
+// the cache: every group of LPK lanes takes its share of the positions (key and value row requested together), the groups
+// of a wave are merged by lane shuffles, the waves through LDS.
 //
 // FUSED: q, k, v of the new position come straight from the QKV projection (row b = [3][H][hd]); q and k are
 // rotated here (pairs (2i, 2i+1), angles of table row pos, rounded to fp16 as a separate rotation kernel would
 // store them), k and v are appended to the cache, and the new position is served from LDS rather than
 // re-read from memory the block has just written.
 // ---------------------------------------------------------------------------------------------
-// 8 waves per block and up to the first 8 positions of every group requested up front, at every batch size.  Measured with
-// 8 of them always, 32 heads of 128 at 130 / 191 / 250 cache positions, cold caches: 5.4 / 5.6 / 6.0 us at batch 1, 10.4 / 12.4 /
-// 14.9 at batch 16, 28.9 / 37.1 / 47.3 at batch 64 (there the kernel reads 200 MB of cache per launch and is HBM-bound).
-// Against that: 16 waves walking the cache two positions at a time 5.6 / 6.2 / 6.8 and 11.5 / 14.2 / 16.7 at batch 1 and 16;
-// 4 waves per block and one pass with a running maximum (the variant that served 1024 pairs and more) 8.7 / 10.8 /
-// 13.7 at batch 4, 11.8 / 14.9 / 18.0 at batch 16, 30.8 / 41.9 / 52.8 at batch 64, and 5 - 7 % behind at 500 and 900
-// positions too.  Every wave repeats the rotation of q and the merge steps, so more waves cost vector issue; a launch
-// costs 4.0 us before it touches the cache (the position, then the new token's q / k / v, then the stores: three
-// dependent round trips behind a 1.7 us launch).
+// 8 waves per block at every batch size.  At 191 positions of 32 heads of 128, cold caches, 16 waves that walked the cache two positions
+// at a time took 11 % longer at batch 1 and 15 % at 16, 4 waves with a running maximum 20 % at batch 16 and 13 % at 64 (both against
+// eight stages for every sequence).  Every wave repeats the rotation of q and the merge steps, so more waves cost vector issue.
 constexpr int kAttnThreads = 512;
 constexpr int64_t kCacheBytes = 256 << 20;      // the Infinity Cache
 constexpr int64_t kMostLayers = 1 << 20;
 constexpr int kUsualLayers = 8;                 // where the caller does not say how many
-constexpr int kAttnPrefetch = 8;          // positions per group requested up front at most (256 at 128-wide heads)
+constexpr int kAttnPrefetch = 8;                // stages requested up front at most (256 positions at 128-wide heads)
 
 __device__ __forceinline__ f16x8 rotate8(const f16x8 x, const float* __restrict__ c, const float* __restrict__ s) {
 #pragma clang fp contract(off)                                // same roundings as rope_kv_store_kernel
@@ -235,8 +228,11 @@ template <int V> struct Tag { static constexpr int value = V; };
 // rotated -- so that the cache rows and the new token's q / k / v travel together instead of one after the other.  The kernel
 // takes as many as the sequence has (its position is known on the device only, so all forms are in the one kernel): stages
 // past the end cost requests, registers and arithmetic, and only the last stage has to look for the end of the sequence.
-// 32 heads of 128, cold caches, against eight stages for every sequence: 190 positions at batch 1 / 16 / 64 4.85 / 11.8 / 36.0
-// -> 4.24 / 11.3 / 35.7 us, 60 positions at batch 96 26.6 -> 19.4.
+// 32 heads of 128, cold caches, against eight stages for every sequence, 30 / 60 / 190 / 250 positions: batch 1 4.6 / 4.7 / 4.9 / 5.0 ->
+// 3.3 / 3.5 / 4.4 / 4.9 us, batch 16 6.7 / 7.7 / 11.5 / 13.8 -> 4.6 / 5.9 / 11.2 / 13.6, batch 64 18.2 / 21.9 / 36.3 / 46.7 -> 12.7 / 17.7 / 35.6 /
+// 46.7, and with rows read once (read_once_from) 12.6 / 16.3 / 32.1 (6.3 TB/s) / 42.2.  The two-launch form (76 vector registers
+// where it had 61 - 64, so three blocks per CU instead of four) 3.7 / 4.0 / 4.4 / 4.5 -> 2.9 / 3.3 / 4.2 / 4.4, batch 64 13.8 / 19.0 / 36.1 / 46.5
+// -> 10.7 / 16.2 / 36.7 / 46.4.
 template <int LPK, bool FUSED, int THREADS, int MOST>
 __global__ __launch_bounds__(THREADS) void decode_attention_kernel(const f16* __restrict__ q_or_qkv, f16* __restrict__ k_cache,
                                                                         f16* __restrict__ v_cache, const int64_t* __restrict__ pos_ptr,
@@ -499,11 +495,13 @@ __global__ __launch_bounds__(kPickThreads) void greedy_next_kernel(const f16* __
 // 190 MB of rows in 2, 4, 8 or 32 layers 236 / 239 (12 sequences, 4 layers), 150 / 167 (4 at 1500 positions, 2 layers), 402 / 472 (one
 // at 1500, 8 layers), 1062 / 1068 (one at 190, 32 layers); 191 ... 256 MB within 1 % (16 at 800 in one layer 101 / 104); 286 and more 1520 / 1501 (3
 // sequences, 32 layers), 1607 / 1562 (8), 480 / 465 (16, 8 layers), 884 / 854 (64).  Above 32 sequences the projections' weights go through that
-// cache too, and one or two layers lose 3 - 7 % below the line (64 sequences in one layer 140 / 131).
+// cache too, which a model of a layer or two would have room for otherwise: fewer than eight layers count as eight there (two layers, 33 ... 64
+// sequences, 60 ... 240 MB of rows 1 - 5 % less read once, 33 at 120 positions 187 / 180; one layer, 64 at 190 140 / 131, 40 at 100 level).
 int read_once_from(int64_t batch, int64_t heads, int64_t head_dim, int64_t layers) {
     const int64_t position = batch * heads * head_dim * 4;
     if (position >= kCacheBytes) return 1;
-    const int64_t step = position * (layers ? layers : kUsualLayers);
+    const bool usual = layers == 0 || (batch > 32 && layers < kUsualLayers);
+    const int64_t step = position * (usual ? kUsualLayers : layers);
     return (int)((kCacheBytes + step - 1) / step);
 }
 

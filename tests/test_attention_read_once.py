@@ -24,7 +24,8 @@ int hipGetLastError(void) { return 0; }
 
 # (batch, heads, head_dim, layers) -> shortest sequence whose rows are loaded past the cache
 CASES = [((16, 32, 128, 8), 128), ((16, 32, 128, 0), 128), ((1, 32, 128, 32), 512), ((4, 32, 128, 32), 128), ((8, 32, 128, 32), 64),
-         ((4, 32, 128, 2), 2048), ((64, 32, 128, 2), 128), ((64, 32, 128, 1), 256), ((64, 32, 64, 1), 512), ((64, 32, 256, 1), 128),
+         ((4, 32, 128, 2), 2048), ((32, 32, 128, 2), 256), ((32, 32, 128, 1), 512), ((32, 32, 64, 1), 1024), ((32, 32, 256, 1), 256),
+         ((64, 32, 128, 2), 32), ((64, 32, 128, 1), 32), ((33, 32, 128, 1), 63), ((64, 32, 128, 16), 16),
          ((5, 32, 32, 1), 13108), ((2, 3, 128, 1 << 20), 1), ((65535, 64, 256, 1), 1), ((1, 1, 32, 1), 2097152)]
 
 
