@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the quantized-linear hot path on one MI355X.
 
-Workload (BASELINE.json configs[1] at M = 1): the four W4A16 g128 asymmetric quantized linears of a
+Workload: at M = 1 the four W4A16 g128 asymmetric quantized linears of a
 Llama-2-7B decoder layer -- fused QKV (12288x4096), O-proj (4096x4096), gate+up (22016x4096) and
 down (4096x11008) -- applied to one fp16 activation row.  One *step* is one pass over those four
 linears for one layer.  Consecutive steps use different layers' weights (NL resident copies, more
@@ -17,10 +17,10 @@ ceilings measured in the same run (`roofline.empirical`: a pure streaming read o
 large dense fp16 GEMM of the vendor library), `cpu_baseline` = the torch CPU port of the reference's test path on
 the same four shapes on this machine's host cores (dequant + matmul, and matmul alone), and one short row per
 shape of the further sections.  The full report -- every section below with every field -- goes to stderr and to
-the side file `bench_report.json` (`write_report`).  Further sections, none of them part of `value`: `small_m` (configs[1] at
-M = 4 / 16, configs[2]: the bit-width sweep at N = K = 8192, the Llama-3-70B shapes at M = 1 and 16),
-`gemm_m256` and `gemm_m32_m64_m128`, `gemm_prefill_m8192` (the Llama-2-7B layers at configs[4]'s
-prefill row count) and `decode` (configs[4]: the Llama-2-7B-shaped decode loop at batch 1 / 16 / 64).
+the side file `bench_report.json` (`write_report`).  Further sections, none of them part of `value`: `small_m` (the same layers at
+M = 4 / 16, the bit-width sweep at N = K = 8192, the Llama-3-70B shapes at M = 1 and 16),
+`gemm_m256` and `gemm_m32_m64_m128` (the Llama-3-70B shapes), `gemm_prefill_m8192` (the Llama-2-7B layers at the row count
+of the decode loop's prefill) and `decode` (the Llama-2-7B-shaped decode loop at batch 1 / 16 / 64).
 
 Other modes (each prints its own JSON and exits): `--counter-pass` and `--counter-pass-matrix` (a few eager
 launches of the GEMV kernels / of the matrix-core kernels beside a copy of known size, for `rocprofv3 --pmc`),
@@ -321,7 +321,7 @@ def dense_fp16_time_us(M, N, K, total_bytes=COLD_BYTES, reps=None):
 
 
 def gemm_report(M=256, shapes=None, reps=None):
-    """BASELINE.json configs[3]: W4A16 g128 GEMM on Llama-3-70B-style shapes, per shape microseconds, TFLOP/s,
+    """W4A16 g128 GEMM on Llama-3-70B-style shapes, per shape microseconds, TFLOP/s,
     the fraction of the dense fp16 MFMA peak and of the HBM peak (M <= 64 is HBM-bound by arithmetic intensity).
     With ``shapes`` / ``reps``: the same report on other layers (the prefill section: launches of a millisecond
     need no 64 per graph to reach the sustained clock)."""
@@ -420,7 +420,7 @@ def _timed_problem(M, N, K, nbits, sym, copies=None):
 
 
 def small_m_report():
-    """BASELINE.json configs[1] at M in {4, 16}, configs[2] (N = K = 8192, M in {1, 16}, 2/3/4/8-bit,
+    """The Llama-2-7B layers at M in {4, 16}, N = K = 8192 (M in {1, 16}, 2/3/4/8-bit,
     symmetric and asymmetric) and the Llama-3-70B shapes at M = 1: per shape microseconds and the fraction
     of the 8 TB/s HBM roofline."""
     import torch
@@ -586,7 +586,7 @@ def shape_sets_report():
 
 
 def decode_report(batches=(1, 16, 64), prompt_len=128, new_tokens=128):
-    """the Llama-2-7B-shaped greedy decode loop (32 layers, every linear a W4A16 g128
+    """The Llama-2-7B-shaped greedy decode loop (32 layers, every linear a W4A16 g128
     QLinear, random weights and prompt ids): tokens/s and the share of a decode step spent in the quantized
     linears, per batch size (qfactory-ae_amd/decode_llama.py)."""
     import torch
@@ -887,7 +887,7 @@ def main():
         result["gemm_m256"] = {"peak_TFLOP/s": MFMA_F16_PEAK_TFLOPS, "dense_fp16_TFLOP/s_measured": round(dense_tflops, 1),
                                "shapes": gemm_report(256)}
         result["gemm_m32_m64_m128"] = [rec for m_rows in (32, 64, 128) for rec in gemm_report(m_rows)]
-        # configs[4]'s prefill: 64 sequences x 128 prompt tokens through the Llama-2-7B layers
+        # the decode loop's prefill: 64 sequences x 128 prompt tokens through the Llama-2-7B layers
         result["gemm_prefill_m8192"] = gemm_report(8192, shapes=SHAPES, reps=16)
     if not args.no_small_m:
         result["small_m"] = small_m_report()

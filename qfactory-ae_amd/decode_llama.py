@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Single-GPU greedy decode loop of a Llama-2-7B-shaped model whose linears are W4A16 g128 QLinear.
 
-BASELINE.json configs[4]: 32 layers, hidden 4096, 32 heads, SwiGLU MLP 11008, vocab 32000, RMSNorm,
+32 layers, hidden 4096, 32 heads, SwiGLU MLP 11008, vocab 32000, RMSNorm,
 RoPE; random-initialised weights; batch in {1, 16, 64}; 128 random prompt ids, 128 greedy output
 tokens.  It stands in for the reference's end-to-end runs through vLLM (reproduce/fig11,
 third_party/vllm-qfactory.patch), which need vLLM and model downloads.
@@ -84,7 +84,7 @@ class QuantLlama:
                 "gate_up": _random_qlinear(batch, h, 2 * shape.mlp, shape, gen),
                 "down": _random_qlinear(batch, shape.mlp, h, shape, gen),
             })
-        # the output projection is a quantized linear like the others (configs[4]: every linear), 32000 x 4096
+        # the output projection is a quantized linear like the others, 32000 x 4096
         self.lm_head = _random_qlinear(batch, h, shape.vocab, shape, gen)
         self.k_cache = torch.zeros(shape.layers, batch, shape.heads, shape.max_len, hd, dtype=torch.float16, device="cuda")
         self.v_cache = torch.zeros_like(self.k_cache)

@@ -834,9 +834,10 @@ def gemm_candidates(M, N, K, nbits, group_size):
 # Tilings of the pipelined kernel (qf::GemmWideCfg, include/qf_gemm_wide.hip.h): (WM, WN, MT, NT, KI, WK) -> us per round
 # of blocks and 64 elements of K.  The figures are medians of a sweep of eighteen tilings over 22016 x 4096, 4096 x 11008 and
 # 10240 x 8192 at 32 ... 2048 rows (W4 g128, cold weights): with the round model of gemm_wide_tiling they pick the fastest of the
-# sweep on 23 of its 27 cells (up to 3 % off on the others).
-# At 8 bits (ten shapes at 24 ... 1024 rows, the forms of _gemm_wide_tiling) the same figures pick within 7 % of the fastest on 97 of
-# 104 cells, 8 - 16 % off on six, and 63 % off on one (2432 x 20480 at 96 rows, where two rounds of 32 x 32 tiles share CUs).
+# sweep on 23 of its 27 cells (up to 3 % off on the others), and on nine other shapes from 3584 x 5888 to 57344 x 8192 at 24 ... 1024
+# rows on 92 of 99 (up to 7 % off).  At 8 bits (ten shapes at 24 ... 1024 rows, every tiling in up to five forms) the same figures are
+# within 3 % of the fastest on 79 of 110 cells, 7 % on 94, 10 % on 104, and up to 15 % off on the others (2432 x 20480 at 512 rows 139 us as
+# 64 x 128, 121 as 64 x 96).
 GEMM_WIDE_COST = {
     (1, 4, 8, 2, 1, 1): 1.520,     # 256 x 256
     (2, 2, 4, 3, 1, 1): 1.258,     # 256 x 192
@@ -856,8 +857,8 @@ GEMM_WIDE_COST = {
     (1, 2, 1, 1, 2, 4): 0.149,     # 32 x 64
     (1, 1, 1, 1, 2, 4): 0.103,     # 32 x 32
 }
-# Where those figures do not hold.  8 bits, 32 x 224: 30 rows on 43648 x 9984 103 us as 32 x 64, 114 as 32 x 224 (2 and 4 bits, 23 ... 28
-# rows on 39360 ... 41984 columns: 7 - 19 % less as 32 x 224).
+# Where those figures do not hold.  8 bits, 32 x 224: 1 - 14 % behind 32 x 64 on ten shapes of 33280 ... 40960 columns at 17 ... 32 rows (38400 x
+# 8192 at 24 87.1 us as 32 x 64, 94.5 as 32 x 224), 3 - 5 % ahead on 57344, where it fills the machine.
 GEMM_WIDE_COST_8BIT = {(1, 7, 1, 1, 2, 1): 0.528}
 # Two groups of two waves of two weight tiles: from six windows of K on, not at 8 bits.  Of random problems at 17 - 2500 rows those with
 # fewer windows took 1 - 9 % longer than as four waves of one weight tile (462 rows on 6528 x 1024 10.5 -> 11.5 us), at 8 bits

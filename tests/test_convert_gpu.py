@@ -106,7 +106,7 @@ def test_weight_packer_at_tile_edges(oracle, nbits, K, N, offset):
 @pytest.mark.parametrize("nbits", [2, 3, 4, 8])
 @pytest.mark.parametrize("K,N,offset", [(32, 128, 0), (1056, 132, 0), (544, 124, 0), (512, 129, 0), (96, 260, 1), (4128, 127, 0)])
 def test_weight_packer_at_the_edges_of_a_block(oracle, nbits, K, N, offset):
-    """One block of 128 columns, a little more and a little less, by fours and by single words."""
+    """128 columns, a little more and a little less, by fours and by single words."""
     test_weight_packer_at_tile_edges(oracle, nbits, K, N, offset)
 
 
