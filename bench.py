@@ -441,11 +441,11 @@ def small_m_report():
 
     for M in (4, 16):
         for name, N, K in SHAPES:
-            one("configs[1]", M, N, K, NBITS, False)
+            one("llama2-7b", M, N, K, NBITS, False)
     for M in (1, 16):
         for nbits in (2, 3, 4, 8):
             for sym in (False, True):
-                one("configs[2]", M, 8192, 8192, nbits, sym)
+                one("bit widths", M, 8192, 8192, nbits, sym)
     # the 28672-wide end of the "4096 - 28672-wide LLM shapes" the GEMV target names: Llama-3-70B at M = 1
     for name, N, K in GEMM_SHAPES:
         one("70b-gemv", 1, N, K, NBITS, False)
@@ -738,8 +738,8 @@ def main():
                     help="skip the eager layer(x) timing (its launches would mix into a kernel trace's averages)")
     ap.add_argument("--small-m", action="store_true", help="accepted for compatibility: the small-M report is on by default")
     ap.add_argument("--no-small-m", action="store_true",
-                    help="skip configs[1] at M = 4, 16, the configs[2] bit-width sweep and the 70B shapes at M = 1")
-    ap.add_argument("--no-decode", action="store_true", help="skip the configs[4] decode loop")
+                    help="skip the Llama-2-7B layers at M = 4, 16, the bit-width sweep at N = K = 8192 and the 70B shapes at M = 1, 16")
+    ap.add_argument("--no-decode", action="store_true", help="skip the decode loop")
     ap.add_argument("--no-graph", action="store_true", help="enqueue the timed steps eagerly from Python")
     ap.add_argument("--launch-floor", action="store_true",
                     help="only measure the launch floor (a kernel that does nothing, several grids) and the streaming-read "
@@ -863,7 +863,7 @@ def main():
         "value": round(value, 1), "unit": "GB/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
         "ms_per_step": round(ms_per_step, 5), "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": "f16", "data": "synthetic",
-        "config": {"workload": "configs[1] at M=1: W4A16 g128 asymmetric GEMV over Llama-2-7B shapes "
+        "config": {"workload": "M=1: W4A16 g128 asymmetric GEMV over Llama-2-7B shapes "
                                "(12288x4096, 4096x4096, 22016x4096, 4096x11008), one step = the four linears of one layer",
                    "bits": NBITS, "group_size": GS, "M": M, "weight_copies": args.layers,
                    "bytes_per_step": int(step_bytes), "timed_with": "eager" if args.no_graph else "one HIP graph of all steps"},

@@ -13,7 +13,7 @@ def _canned_full():
     gemm = [{"name": n, "N": N, "K": K, "M": 256, "us": 230.41, "TFLOP/s": 1043.8, "mfma_frac": 0.4148, "GB/s": 1204.9,
              "hbm_frac": 0.1506, "dense_fp16_us": 260.12, "speedup_over_dense_fp16": 1.129, "kernel": kernel}
             for n, N, K in bench.GEMM_SHAPES]
-    small = [{"config": "configs[2]", "M": M, "N": 8192, "K": 8192, "bits": b, "sym": sym, "us": 14.583, "GB/s": 2426.8,
+    small = [{"config": "bit widths", "M": M, "N": 8192, "K": 8192, "bits": b, "sym": sym, "us": 14.583, "GB/s": 2426.8,
               "hbm_frac": 0.3034, "TFLOP/s": 147.27, "kernel": kernel}
              for M in (1, 4, 16) for b in (2, 3, 4, 8) for sym in (False, True)] * 2
     decode = [{"batch": b, "value": 15732.3456, "decode_step_us": 4068.123, "quantized_linear_share": 0.56789,

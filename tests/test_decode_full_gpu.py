@@ -82,7 +82,7 @@ def test_full_size_decode_step_matches_the_torch_evaluation(llama, batch):
 
 
 def test_full_size_prompt_of_128_tokens_then_decode_at_batch_1(llama):
-    """configs[4] as written, at batch 1: 128 prompt tokens through ``prefill`` (the GEMM kernels at 128 rows, one
+    """The decode loop at full size, at batch 1: 128 prompt tokens through ``prefill`` (the GEMM kernels at 128 rows, one
     launch for RoPE and the cache rows), then greedy tokens through the fused decode step, which then attends to
     129 and more cache positions -- against the PyTorch evaluation fed the same tokens."""
     prompt_len, steps = 128, 3
