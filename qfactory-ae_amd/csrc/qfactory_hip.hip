@@ -26,7 +26,7 @@ int launched(const char* fn) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Weight repack, bound by memory: four bytes are read per field.  A block takes 128 columns n (64 of a small layer)
+// Weight repack, bound by memory: four bytes are read per field.  A block takes 128 columns n (64 by the rule of launch_layer)
 // and 32 main-plane words of K (32 threads x 4 columns side by side, 16 units of K): a thread reads 16 bytes of every k of its
 // unit -- 512 contiguous bytes per k and 32 threads -- builds four columns' words in registers, and the words change their orientation
 // through LDS, so that a row of the output is written 128 bytes at a time.  (A 4-byte word per thread straight to its row left
@@ -214,15 +214,18 @@ int launch_blocks(const char* fn, PackJob j, hipStream_t stream) {
     return launched(fn);
 }
 
-// Blocks of 128 columns for layers of more than 128 of them, of 64 for smaller ones, which leave CUs without work either way and
-// take as long as a block does.  64 / 128 columns, cold weights, scales and zero-points with them: 1024 x 1024 at 2 / 3 / 4 / 8 bits 5.9 / 6.3 /
-// 4.7 / 4.0 against 7.9 / 8.1 / 5.3 / 4.4 us, 4096 x 2048 (128 blocks but at 8 bits) 8.9 / 9.5 / 8.9 / 9.8 against 9.9 / 10.7 / 9.1 / 9.8; 4096 x 1100 at
-// 4 bits (144 blocks) 8.2 against 7.6, 4096 x 3072 at 2 / 3 / 4 / 8 bits (192 blocks at 2 and 3) 13.0 / 13.5 / 12.0 / 15.0 against 11.9 / 12.7 /
-// 13.1 / 14.2.
+// Blocks of 128 columns, but of 64 where there would be few of 128 and where the second on a CU would have it to itself.
+// Up to 128 blocks leave CUs without work either way and take as long as a block does: 64 / 128 columns, cold weights, scales and
+// zero-points with them, 1024 x 1024 at 2 / 3 / 4 / 8 bits 5.9 / 6.3 / 4.7 / 4.0 against 7.9 / 8.1 / 5.3 / 4.4 us.  144 ... 224 blocks take
+// 0 - 10 % less by 128 columns at 2 and 3 bits (4096 x 3072 at 2 12.0 against 10.8), within 3 % at 4 and 8.  More than 256 and up to 384, one and a
+// half per CU, 0 - 13 % more: 4096 x 5120 at 2 / 3 bits 18.0 / 19.1 against 19.2 / 20.2, 8192 x 1280 at 4 10.3 / 11.6, 4096 x 1152 at 8 6.3 / 6.9; so do
+// 256 of them at 4 and 8 bits, whose scales and zero-points are more blocks in front (4096 x 1024 at 8 5.9 / 6.6), at 2 and 3 they take
+// 4 - 8 % less.  Beyond, 128 columns take 4 % less in the mean (4096 x 4096 at 4 15.6 / 14.1; 87 points up to 1536 blocks, 0.87 - 1.08 x).
 template <int NBITS>
 int launch_layer(const char* fn, const PackJob& j, hipStream_t stream) {
-    return weight_blocks<PackCfg<NBITS, 512>>(j) <= 128 ? launch_blocks<PackCfg<NBITS, 256>>(fn, j, stream)
-                                                        : launch_blocks<PackCfg<NBITS, 512>>(fn, j, stream);
+    const int64_t wide = weight_blocks<PackCfg<NBITS, 512>>(j);
+    const bool narrow = wide <= 128 || (wide >= (NBITS >= 4 ? 256 : 257) && wide <= 384);
+    return narrow ? launch_blocks<PackCfg<NBITS, 256>>(fn, j, stream) : launch_blocks<PackCfg<NBITS, 512>>(fn, j, stream);
 }
 
 int launch_layer(const char* fn, const PackJob& j, hipStream_t stream) {

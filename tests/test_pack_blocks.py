@@ -1,5 +1,5 @@
-"""Which blocks a layer is packed by: 64 columns and 256 threads up to 128 blocks of 128 columns, 512 threads beyond.  The launch goes to
-a stand-in that prints it."""
+"""Which blocks a layer is packed by: 64 columns and 256 threads where blocks of 128 columns would be at most 128, or more than one and up
+to one and a half per CU; else 128 columns and 512 threads.  The launch goes to a stand-in that prints it."""
 import os
 import subprocess
 import sys
@@ -14,7 +14,10 @@ int hipGetLastError(void) { return 0; }
 
 # (nbits, K, N) -> blocks, threads
 CASES = [((4, 1024, 1024), (16 * 4, 256)), ((2, 4096, 64), (8, 256)), ((2, 4096, 2048), (32 * 8, 256)), ((3, 4096, 2049), (17 * 8, 512)),
-         ((4, 4096, 1024), (16 * 16, 256)), ((4, 4128, 1024), (8 * 17, 512)), ((8, 4096, 1024), (8 * 32, 512)), ((4, 4096, 22016), (172 * 16, 512))]
+         ((4, 4096, 1024), (16 * 16, 256)), ((4, 4128, 1024), (8 * 17, 512)), ((8, 4096, 896), (7 * 32, 512)), ((4, 4096, 22016), (172 * 16, 512)),
+         ((8, 4096, 1024), (16 * 32, 256)), ((4, 4096, 2048), (32 * 16, 256)), ((2, 4096, 4096), (32 * 8, 512)), ((3, 4096, 4096), (32 * 8, 512)),
+         ((2, 4096, 4097), (65 * 8, 256)), ((3, 4096, 4224), (66 * 8, 256)), ((4, 4096, 3072), (48 * 16, 256)), ((8, 4096, 1536), (24 * 32, 256)),
+         ((4, 4096, 3073), (25 * 16, 512)), ((8, 4128, 1536), (12 * 33, 512)), ((2, 4096, 6145), (49 * 8, 512))]
 
 
 def test_small_layers_are_packed_by_narrow_blocks(tmp_path):
