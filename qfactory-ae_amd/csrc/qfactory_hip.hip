@@ -202,14 +202,13 @@ int64_t weight_blocks(const PackJob& j) {
 }
 
 template <class C>
-int launch_blocks(const char* fn, PackJob j, hipStream_t stream) {
+int launch_blocks(const char* fn, PackJob j, bool vec, hipStream_t stream) {
     const int64_t scale_blocks = j.scale ? (j.N + 31) / 32 * ((j.G + 31) / 32) : 0;
     const int64_t zero_blocks = j.zero ? (j.N * (j.G / (8 / j.fb)) + C::THREADS - 1) / C::THREADS : 0;
     const int64_t blocks = weight_blocks<C>(j) + scale_blocks + zero_blocks;
     if (blocks > 0x7fffffff) return fail(fn, "too many blocks");
     j.scale_blocks = (unsigned)scale_blocks;
     j.zero_blocks = (unsigned)zero_blocks;
-    const bool vec = j.N % 4 == 0 && (uintptr_t)j.weight % 16 == 0;
     hipLaunchKernelGGL((vec ? pack_layer_kernel<C, true> : pack_layer_kernel<C, false>), dim3((unsigned)blocks), dim3(C::THREADS), 0, stream, j);
     return launched(fn);
 }
@@ -221,11 +220,15 @@ int launch_blocks(const char* fn, PackJob j, hipStream_t stream) {
 // half per CU, 0 - 13 % more: 4096 x 5120 at 2 / 3 bits 18.0 / 19.1 against 19.2 / 20.2, 8192 x 1280 at 4 10.3 / 11.6, 4096 x 1152 at 8 6.3 / 6.9; so do
 // 256 of them at 4 and 8 bits, whose scales and zero-points are more blocks in front (4096 x 1024 at 8 5.9 / 6.6), at 2 and 3 they take
 // 4 - 8 % less.  Beyond, 128 columns take 4 % less in the mean (4096 x 4096 at 4 15.6 / 14.1; 87 points up to 1536 blocks, 0.87 - 1.08 x).
+// Columns loaded one by one are packed by 64 beyond 256 blocks at all: 4096 x 5117 at 2 / 3 / 4 bits 27.7 / 28.7 / 25.0 against 34.7 / 37.3 / 28.2,
+// 4096 x 8189 at 2 37.1 against 49.0, 4096 x 3069 at 8 17.1 against 20.1 (60 points 0.97 - 1.37 x, twenty of them within 2 %); 144 ... 256
+// blocks are level by either, but 256 at 3 bits 23.1 by 128 columns, 28.1 by 64.
 template <int NBITS>
 int launch_layer(const char* fn, const PackJob& j, hipStream_t stream) {
     const int64_t wide = weight_blocks<PackCfg<NBITS, 512>>(j);
-    const bool narrow = wide <= 128 || (wide >= (NBITS >= 4 ? 256 : 257) && wide <= 384);
-    return narrow ? launch_blocks<PackCfg<NBITS, 256>>(fn, j, stream) : launch_blocks<PackCfg<NBITS, 512>>(fn, j, stream);
+    const bool vec = j.N % 4 == 0 && (uintptr_t)j.weight % 16 == 0;
+    const bool narrow = wide <= 128 || (wide >= (NBITS >= 4 ? 256 : 257) && (wide <= 384 || !vec));
+    return narrow ? launch_blocks<PackCfg<NBITS, 256>>(fn, j, vec, stream) : launch_blocks<PackCfg<NBITS, 512>>(fn, j, vec, stream);
 }
 
 int launch_layer(const char* fn, const PackJob& j, hipStream_t stream) {
